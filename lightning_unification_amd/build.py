@@ -127,7 +127,7 @@ def build_bindings(verbose=False):
 def build_oracle(verbose=False):
     odir = os.path.join(ROOT, "oracle")
     _run(["make", "-B", "-s", "-C", odir, "-j8"], verbose)
-    if os.path.isdir(REFERENCE):
+    if os.path.isdir(os.path.join(REFERENCE, "pennylane_lightning", "core", "src")):
         _run(["make", "-B", "-s", "-C", odir, "-j8", "ref", f"REF={REFERENCE}"], verbose)
 
 
