@@ -45,11 +45,13 @@ def _run(cmd, verbose):
 TILE_FLAGS = ["-mllvm", "-structurizecfg-skip-uniform-regions=true"]
 
 # (source, object, extra flags): the tile-pass kernel once per
-# (precision, tile size) so that its variants compile in parallel
+# (precision, tile size) so that its variants compile in parallel, the
+# backward sweep's once per precision
 ENGINE_UNITS = [("pl_amd.hip", "pl_amd.o", []), ("batch.hip", "batch.o", []), ("mlp.hip", "mlp.o", [])] + [
     ("tiled.hip", f"tiled_{'c128' if d else 'c64'}_{kb}.o",
      [f"-DPL_TILE_DOUBLE={d}", f"-DPL_TILE_KB={kb}", *TILE_FLAGS])
-    for d in (1, 0) for kb in ((3, 4, 5) if d else (3, 4, 5, 6))]
+    for d in (1, 0) for kb in ((3, 4, 5) if d else (3, 4, 5, 6))] + [
+    ("sweep.hip", f"sweep_{'c128' if d else 'c64'}.o", [f"-DPL_SWEEP_DOUBLE={d}", *TILE_FLAGS]) for d in (1, 0)]
 
 
 def _deps(path, seen=None):

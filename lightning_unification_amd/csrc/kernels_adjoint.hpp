@@ -1,338 +1,474 @@
-// Fused adjoint-Jacobian step (one operation of the backward sweep of
-// AdjointJacobianLQubit.hpp:282-329).
+// The backward sweep of the adjoint Jacobian (AdjointJacobianLQubit.hpp:282-329)
+// and of the vector-Jacobian product (VectorJacobianProduct.hpp:77-155) in tile
+// passes.
 //
-// Reference order per op i:  mu <- lambda;  lambda <- U_i^dag lambda;
-// mu <- G_i mu;  J[t][k] = -2 s Im<H_k|mu>;  H_k <- U_i^dag H_k.
-// Here, per amplitude group of op i (U_i and G_i lowered on one geometry):
-// load lambda's group, form mu = G lambda in registers, store U^dag lambda;
-// then for each H_k: load its group, accumulate Im(conj(H_k) . mu), store
-// U^dag H_k.  mu never touches HBM and every state is read and written once
-// per op: (2 + 2K) state passes against the reference's (6 + 4K).
+// Per operation, in reverse, the sweep needs <H_k|G lambda> of a trainable
+// operation's generator G, then undoes the operation on lambda and every H_k.
+// A launch per operation moves (1 + K) states for a few FMAs an amplitude:
+// 60 us a step with 10 observables at 20 qubits, all of it cache and HBM
+// traffic.  Here a workgroup of NW wavefronts holds a tile of lambda and of KH
+// of the H_k (all combinations of the pass's bits) in registers and runs every
+// step of the pass on it, so a pass moves each state once however many steps
+// it has.  A thread's 2^RB amplitudes differ in the window bits; a step mixes
+// one window bit, with compile-time register indexes, and a change of window
+// goes through LDS, one state at a time through one buffer.  A step per trip
+// through LDS instead (amplitudes kept there) was bound by LDS latency and
+// address arithmetic: 5 us a step for six resident wavefronts.
+// 20 qubits, 600 parameters, 20 observables: 8 passes of 0.67 ms, 5.4 ms for
+// the Jacobian against 84 ms; bound by FP64 issue (about 2.5 ms of multiply-adds
+// at full rate, window changes, wavefront reductions) and by the states'
+// traffic (0.16 ms a pass).
+//
+// Steps (sweep.hpp) hold runs of operations with one geometry.  A run of 2x2
+// operations is one step: every <H|G_j lambda_j> inside it is a linear form of
+// the transition matrix M_ab = sum conj(h_a) lambda_b at the run's start, whose
+// needed parts are accumulated, in FP64, while the run's product matrix is
+// applied.
 #pragma once
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include "kernels_reduce.hpp"
+#include "sweep_launch.hpp"
 
 namespace plamd {
 
-template <class T, int M> struct AdjOp {
-    Geom geo;
-    uint64_t off[M];
-    dcx<T> ud[M * M];
-    dcx<T> g[M * M];
-    int ud_diag;
-};
+// Sums of a and b over lanes l and l ^ 32: a's in the lower half, b's in the upper.
+__device__ __forceinline__ double sweep_fold32(double a, double b) {
+    const auto ua = static_cast<unsigned long long>(__double_as_longlong(a));
+    const auto ub = static_cast<unsigned long long>(__double_as_longlong(b));
+    const auto lo = __builtin_amdgcn_permlane32_swap(static_cast<unsigned>(ua), static_cast<unsigned>(ub), false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(static_cast<unsigned>(ua >> 32), static_cast<unsigned>(ub >> 32),
+                                                     false, false);
+    const double x = __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi[0]) << 32) | lo[0]));
+    const double y = __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi[1]) << 32) | lo[1]));
+    return x + y;
+}
+// Sums of a and b over lanes l and l ^ 16: a's in even rows of 16 lanes, b's in odd ones.
+__device__ __forceinline__ double sweep_fold16(double a, double b) {
+    const auto ua = static_cast<unsigned long long>(__double_as_longlong(a));
+    const auto ub = static_cast<unsigned long long>(__double_as_longlong(b));
+    const auto lo = __builtin_amdgcn_permlane16_swap(static_cast<unsigned>(ua), static_cast<unsigned>(ub), false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(static_cast<unsigned>(ua >> 32), static_cast<unsigned>(ub >> 32),
+                                                     false, false);
+    const double x = __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi[0]) << 32) | lo[0]));
+    const double y = __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi[1]) << 32) | lo[1]));
+    return x + y;
+}
+template <int CTRL> __device__ __forceinline__ double sweep_dpp(double v) {
+    const auto u = static_cast<unsigned long long>(__double_as_longlong(v));
+    const unsigned lo = static_cast<unsigned>(__builtin_amdgcn_mov_dpp(static_cast<int>(static_cast<unsigned>(u)), CTRL, 0xf, 0xf, true));
+    const unsigned hi = static_cast<unsigned>(__builtin_amdgcn_mov_dpp(static_cast<int>(static_cast<unsigned>(u >> 32)), CTRL, 0xf, 0xf, true));
+    return __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi) << 32) | lo));
+}
+// Totals of four values over the wavefront: row r of 16 lanes (lane / 16 = r)
+// ends with the total of v[sweep_row(r)].
+__device__ __forceinline__ double sweep_sum4(double v0, double v1, double v2, double v3) {
+    // rows 0..3 after the folds: v0, v2, v1, v3
+    double s = sweep_fold16(sweep_fold32(v0, v1), sweep_fold32(v2, v3));
+    s += sweep_dpp<0x128>(s); // rotations within a row by 8, 4, 2, 1
+    s += sweep_dpp<0x124>(s);
+    s += sweep_dpp<0x122>(s);
+    s += sweep_dpp<0x121>(s);
+    return s;
+}
+__device__ __forceinline__ int sweep_row(int r) { return ((r & 1) << 1) | (r >> 1); }
 
-constexpr int kAdjMaxObs = 16; // observables per launch
-// bytes of states one adjoint sweep keeps in flight when the states do not
-// all fit on die: MI355X has 256 MB of Infinity Cache in front of HBM
-constexpr size_t kAdjCacheBytes = size_t{192} << 20;
-constexpr int kAdjChunk = 4;    // observables whose loads are in flight together
-
-template <class T, int M>
-__device__ __forceinline__ void matvec(const dcx<T> *m, int diag, const v2<T> *x, v2<T> *y) {
-    if (diag) {
-#pragma unroll
-        for (int r = 0; r < M; r++) {
-            y[r] = cmul(m[r * M + r], x[r]);
-        }
-    } else {
-#pragma unroll
-        for (int r = 0; r < M; r++) {
-            v2<T> acc = cmul(m[r * M], x[0]);
-#pragma unroll
-            for (int c = 1; c < M; c++) {
-                cfma(acc, m[r * M + c], x[c]);
-            }
-            y[r] = acc;
-        }
-    }
+// Local index -> place in the LDS buffer, linear in its bits.  With a window
+// bit among the lowest, neighbouring lanes hold every other amplitude of 128
+// bytes; flipping the bits inside 128 bytes where the next bit is set spreads
+// them over all banks again.
+__device__ __forceinline__ uint32_t sweep_place(uint32_t e) {
+    constexpr int b = 4; // 16 doubles
+    return e ^ (((e >> b) & 1U) * ((1U << b) - 1));
 }
 
-// Block totals of the per-thread accumulators acc[0 .. nobs): each wave sums
-// with shuffles into an LDS table, one barrier, then thread k adds the waves'
-// entries in order (nobs is uniform across the block).
-__device__ __forceinline__ void adj_block_totals(const double *acc, int nobs, double *__restrict__ out) {
-    __shared__ double wpart[kBlock / 64][kAdjMaxObs];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+// thread bits spread over the local bits outside the window
+template <int RB> __device__ __forceinline__ uint32_t sweep_thread_part(uint32_t t, uint32_t win) {
 #pragma unroll
-    for (int k = 0; k < kAdjMaxObs; k++) {
-        if (k < nobs) {
-            const double s = wave_sum(acc[k]);
-            if (lane == 0) {
-                wpart[wave][k] = s;
+    for (int j = 0; j < RB; j++) {
+        const uint32_t m = (1U << ((win >> (4 * j)) & 15U)) - 1;
+        t = ((t & ~m) << 1) | (t & m);
+    }
+    return t;
+}
+template <int RB> __device__ __forceinline__ uint32_t sweep_reg_part(int r, uint32_t win) {
+    uint32_t e = 0;
+#pragma unroll
+    for (int j = 0; j < RB; j++) {
+        e |= ((r >> j) & 1) ? 1U << ((win >> (4 * j)) & 15U) : 0U;
+    }
+    return e;
+}
+
+__device__ __forceinline__ double sweep_fma(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
+// Updates of the register tile.  The last multiply-add of every amplitude
+// writes the amplitude's own register, in the lanes of `m` only; the lane
+// condition is an execution mask inside the block, so a step has no divergent
+// branch.  Left to the compiler (branches on the condition, results in
+// registers of their own), every step's results were copied back where the
+// steps' branches join: 241 registers and two wavefronts a SIMD for KH = 2 in
+// complex128, a third of the instructions moves.  All 64 lanes are active
+// around every block.
+__device__ __forceinline__ void sweep_into(uint64_t m, double2 &a, double u, double tx, double ty) {
+    asm("s_mov_b64 exec, %2\n\t"
+        "v_fma_f64 %0, %3, %0, %4\n\t"
+        "v_fma_f64 %1, %3, %1, %5\n\t"
+        "s_mov_b64 exec, -1"
+        : "+v"(a.x), "+v"(a.y)
+        : "s"(m), "v"(u), "v"(tx), "v"(ty));
+}
+__device__ __forceinline__ void sweep_into2(uint64_t m, double2 &a, double2 &b, double ua, double ub, double t0,
+                                            double t1, double t2, double t3) {
+    asm("s_mov_b64 exec, %4\n\t"
+        "v_fma_f64 %0, %5, %0, %7\n\t"
+        "v_fma_f64 %1, %5, %1, %8\n\t"
+        "v_fma_f64 %2, %6, %2, %9\n\t"
+        "v_fma_f64 %3, %6, %3, %10\n\t"
+        "s_mov_b64 exec, -1"
+        : "+v"(a.x), "+v"(a.y), "+v"(b.x), "+v"(b.y)
+        : "s"(m), "s"(ua), "s"(ub), "v"(t0), "v"(t1), "v"(t2), "v"(t3));
+}
+// a <-> b in the lanes of m
+__device__ __forceinline__ void sweep_exchange(uint64_t m, double2 &a, double2 &b) {
+    double t;
+    asm("s_mov_b64 exec, %5\n\t"
+        "v_mov_b64 %4, %0\n\t"
+        "v_mov_b64 %0, %2\n\t"
+        "v_mov_b64 %2, %4\n\t"
+        "v_mov_b64 %4, %1\n\t"
+        "v_mov_b64 %1, %3\n\t"
+        "v_mov_b64 %3, %4\n\t"
+        "s_mov_b64 exec, -1"
+        : "+v"(a.x), "+v"(a.y), "+v"(b.x), "+v"(b.y), "=&v"(t)
+        : "s"(m));
+}
+
+// (a, b) <- u (a, b) in the lanes of m, 16 multiply-adds
+__device__ __forceinline__ void sweep_apply2(uint64_t m, const dcx<double> *u, double2 &a, double2 &b) {
+    const double t0 = sweep_fma(-u[0].i, a.y, sweep_fma(u[1].r, b.x, -u[1].i * b.y));
+    const double t1 = sweep_fma(u[0].i, a.x, sweep_fma(u[1].r, b.y, u[1].i * b.x));
+    const double t2 = sweep_fma(-u[3].i, b.y, sweep_fma(u[2].r, a.x, -u[2].i * a.y));
+    const double t3 = sweep_fma(u[3].i, b.x, sweep_fma(u[2].r, a.y, u[2].i * a.x));
+    sweep_into2(m, a, b, u[0].r, u[3].r, t0, t1, t2, t3);
+}
+
+// Workgroups are numbered (tile walker w, observable group grp), groups of one
+// walker on one XCD where the grid allows it, since they read the same lambda
+// tiles.  Group grp takes KH observables.  The group numbered `writer` writes
+// lambda to lam_out (which may be lam_in when no other group reads it).
+// partial[(((slot0 + slot) * NC + c) * K + k) * W + w], W walkers.
+template <class T, int NW, int KH, bool FULL>
+__global__ __launch_bounds__(64 * NW, 4) void k_sweep(const SweepArgs<T> A, const SweepStep *__restrict__ prog) {
+    constexpr int NC = FULL ? kSweepFull : kSweepReal;
+    constexpr int RB = kSweepRegBits, R = 1 << RB;
+    static_assert(RB == 3, "the steps' switches name three register bits");
+    constexpr int TB = 6 + (NW == 4 ? 2 : NW == 2 ? 1 : 0); // thread bits
+    constexpr int S = 1 + KH;                               // states: lambda, then the H_k
+    constexpr uint32_t HOME = [] { // window at a tile's load and store: the highest local bits
+        uint32_t v = 0;
+        for (int j = 0; j < RB; j++) {
+            v |= static_cast<uint32_t>(TB + j) << (4 * j);
+        }
+        return v;
+    }();
+    extern __shared__ unsigned char smem_raw[];
+    // real parts, then imaginary parts: a 16-byte element would tie the two
+    // registers of an amplitude into one tuple, which the in-place updates
+    // would have to copy out of and back into
+    double *tile = reinterpret_cast<double *>(smem_raw);
+    constexpr uint32_t IM = 1U << (TB + RB);
+    double *sums = reinterpret_cast<double *>(tile + 2 * IM); // [wave][slot][KH][NC]
+    const uint32_t tid = threadIdx.x;
+    const int lane = tid & 63, wave = tid >> 6;
+    int w, grp;
+    if (A.W & 7) {
+        grp = static_cast<int>(blockIdx.x) % A.ngrp;
+        w = static_cast<int>(blockIdx.x) / A.ngrp;
+    } else {
+        const int xcd = blockIdx.x & 7, y = blockIdx.x >> 3;
+        grp = y % A.ngrp;
+        w = (y / A.ngrp) * 8 + xcd;
+    }
+    grp += A.grp0;
+    const int k0 = grp * KH, nk = A.K - k0 < KH ? A.K - k0 : KH;
+    v2<T> *h[KH];
+#pragma unroll
+    for (int kk = 0; kk < KH; kk++) {
+        h[kk] = A.hs[k0 + (kk < nk ? kk : 0)];
+    }
+    // the program into the caches at once: a step's scalar loads would each
+    // meet memory otherwise, one after another
+    for (uint32_t o = tid * 64; o < A.nsteps * sizeof(SweepStep); o += 64 * NW * 64) {
+        asm volatile("" ::"v"(*reinterpret_cast<const int *>(reinterpret_cast<const char *>(prog) + o)));
+    }
+    const int nsum = A.nslots * KH * NC;
+    double *mine = sums + wave * nsum;
+    for (int i = lane; i < nsum; i += 64) {
+        mine[i] = 0;
+    }
+    const SweepGeom &geo = A.geo;
+    auto spread = [&](uint32_t e) { // local index -> bits of the state index
+        uint64_t g = e & ((1U << geo.low) - 1);
+        for (int b = geo.low; b < geo.bits; b++) {
+            g |= static_cast<uint64_t>((e >> b) & 1U) << geo.hb[b - geo.low];
+        }
+        return g;
+    };
+    const uint32_t size = 1U << geo.bits; // a state smaller than the tile leaves the rest zero
+    const uint64_t thread_at = spread(tid);
+    double2 x[S][R];
+    for (uint64_t q = w; q < A.ntiles; q += A.W) {
+        uint64_t base = q << geo.low;
+        for (int b = 0; b < geo.bits - geo.low; b++) {
+            const int p = geo.hb[b];
+            base = ((base >> p) << (p + 1)) | (base & ((uint64_t{1} << p) - 1));
+        }
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const uint32_t e = (static_cast<uint32_t>(r) << TB) | tid;
+            const uint64_t a = base | thread_at | spread(static_cast<uint32_t>(r) << TB);
+#pragma unroll
+            for (int i = 0; i < S; i++) {
+                x[i][r] = double2{0, 0};
+                if (e < size && (i == 0 || i - 1 < nk)) {
+                    const v2<T> v = (i == 0 ? A.lam_in : h[i ? i - 1 : 0])[a];
+                    x[i][r] = double2{v.x, v.y};
+                }
+            }
+        }
+        uint32_t win = HOME;
+        auto window = [&](uint32_t to) {
+            const uint32_t tf = sweep_place(sweep_thread_part<RB>(tid, win));
+            const uint32_t tt = sweep_place(sweep_thread_part<RB>(tid, to));
+#pragma unroll
+            for (int i = 0; i < S; i++) {
+                __syncthreads();
+#pragma unroll
+                for (int r = 0; r < R; r++) {
+                    const uint32_t p = tf ^ sweep_place(sweep_reg_part<RB>(r, win));
+                    tile[p] = x[i][r].x;
+                    tile[p + IM] = x[i][r].y;
+                }
+                __syncthreads();
+#pragma unroll
+                for (int r = 0; r < R; r++) {
+                    const uint32_t p = tt ^ sweep_place(sweep_reg_part<RB>(r, to));
+                    x[i][r].x = tile[p];
+                    x[i][r].y = tile[p + IM];
+                }
+            }
+            win = to;
+        };
+        for (int s = 0; s < A.nsteps; s++) {
+            const SweepStep &st = prog[s];
+            const int kind = st.kind;
+            if (kind == kSweepWindow) {
+                window(st.rp);
+                continue;
+            }
+            if ((base & st.omask) != st.oval) {
+                continue;
+            }
+            const int slot = st.slot;
+            const bool on = (tid & st.lm) == st.lv;
+            const uint64_t lanes = __ballot(on);
+            const uint32_t rm = st.rm, rv = st.rv;
+            const uint32_t rp = st.rp;
+            const uint32_t tpar = (__popc(tid & st.lp) + __popcll(base & st.op)) & 1U; // kSweepDiag
+            // the sums first, reading only, then the update: together, the
+            // old and the new amplitudes would be live at once
+            if (slot >= 0) {
+                double acc[KH][NC];
+#pragma unroll
+                for (int kk = 0; kk < KH; kk++) {
+#pragma unroll
+                    for (int c = 0; c < NC; c++) {
+                        acc[kk][c] = 0;
+                    }
+                }
+                auto pairs = [&](auto jt) {
+                    constexpr int J = decltype(jt)::value;
+#pragma unroll
+                    for (int p = 0; p < R / 2; p++) {
+                        const int i0 = ((p >> J) << (J + 1)) | (p & ((1 << J) - 1)), i1 = i0 | (1 << J);
+                        if ((static_cast<uint32_t>(i0) & rm) != rv) {
+                            continue;
+                        }
+                        const double ax = x[0][i0].x, ay = x[0][i0].y, bx = x[0][i1].x, by = x[0][i1].y;
+#pragma unroll
+                        for (int kk = 0; kk < KH; kk++) {
+                            const double cx = x[1 + kk][i0].x, cy = x[1 + kk][i0].y, dx = x[1 + kk][i1].x,
+                                         dy = x[1 + kk][i1].y;
+                            double *t = acc[kk];
+                            t[0] = sweep_fma(cx, ay, sweep_fma(-cy, ax, t[0]));
+                            t[1] = sweep_fma(dx, by, sweep_fma(-dy, bx, t[1]));
+                            t[2] = sweep_fma(cx, by, sweep_fma(-cy, bx, sweep_fma(dx, ay, sweep_fma(-dy, ax, t[2]))));
+                            t[3] = sweep_fma(cx, bx, sweep_fma(cy, by, sweep_fma(-dx, ax, sweep_fma(-dy, ay, t[3]))));
+                            if constexpr (FULL) {
+                                t[4] = sweep_fma(cx, ax, sweep_fma(cy, ay, t[4]));
+                                t[5] = sweep_fma(dx, bx, sweep_fma(dy, by, t[5]));
+                                t[6] = sweep_fma(cx, bx, sweep_fma(cy, by, sweep_fma(dx, ax, sweep_fma(dy, ay, t[6]))));
+                                t[7] = sweep_fma(cx, by, sweep_fma(-cy, bx, sweep_fma(-dx, ay, sweep_fma(dy, ax, t[7]))));
+                            }
+                        }
+                    }
+                };
+                if (kind == kSweepDiag) { // even register parity plus, and less, odd
+#pragma unroll
+                    for (int r = 0; r < R; r++) {
+                        if ((static_cast<uint32_t>(r) & rm) != rv) {
+                            continue;
+                        }
+                        const bool odd = __popc(static_cast<uint32_t>(r) & rp) & 1U; // uniform
+                        const double ax = x[0][r].x, ay = x[0][r].y;
+#pragma unroll
+                        for (int kk = 0; kk < KH; kk++) {
+                            const double cx = x[1 + kk][r].x, cy = x[1 + kk][r].y;
+                            const double im = sweep_fma(cx, ay, -cy * ax);
+                            acc[kk][0] += im;
+                            acc[kk][1] += odd ? -im : im;
+                            if constexpr (FULL) {
+                                const double re = sweep_fma(cx, ax, cy * ay);
+                                acc[kk][4] += re;
+                                acc[kk][5] += odd ? -re : re;
+                            }
+                        }
+                    }
+#pragma unroll
+                    for (int kk = 0; kk < KH; kk++) {
+#pragma unroll
+                        for (int c = 0; c < NC; c += 4) {
+                            const double both = acc[kk][c], less = tpar ? -acc[kk][c + 1] : acc[kk][c + 1];
+                            acc[kk][c] = 0.5 * (both + less);
+                            acc[kk][c + 1] = 0.5 * (both - less);
+                        }
+                    }
+                } else {
+                    switch (st.j) {
+                    case 0: pairs(std::integral_constant<int, 0>{}); break;
+                    case 1: pairs(std::integral_constant<int, 1>{}); break;
+                    default: pairs(std::integral_constant<int, 2>{}); break;
+                    }
+                }
+#pragma unroll
+                for (int kk = 0; kk < KH; kk++) {
+#pragma unroll
+                    for (int c = 0; c < NC; c += 4) {
+                        const double t = sweep_sum4(on ? acc[kk][c] : 0.0, on ? acc[kk][c + 1] : 0.0,
+                                                    on ? acc[kk][c + 2] : 0.0, on ? acc[kk][c + 3] : 0.0);
+                        if ((lane & 15) == 0) {
+                            mine[(slot * KH + kk) * NC + c + sweep_row(lane >> 4)] += t;
+                        }
+                    }
+                }
+            }
+            if (kind == kSweepDense) {
+                dcx<double> u[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    u[i] = st.u[i];
+                }
+                auto dense = [&](auto jt) {
+                    constexpr int J = decltype(jt)::value;
+#pragma unroll
+                    for (int p = 0; p < R / 2; p++) {
+                        const int i0 = ((p >> J) << (J + 1)) | (p & ((1 << J) - 1)), i1 = i0 | (1 << J);
+                        if ((static_cast<uint32_t>(i0) & rm) == rv) {
+#pragma unroll
+                            for (int i = 0; i < S; i++) {
+                                sweep_apply2(lanes, u, x[i][i0], x[i][i1]);
+                            }
+                        }
+                    }
+                };
+                switch (st.j) {
+                case 0: dense(std::integral_constant<int, 0>{}); break;
+                case 1: dense(std::integral_constant<int, 1>{}); break;
+                default: dense(std::integral_constant<int, 2>{}); break;
+                }
+            } else if (kind == kSweepFlip) {
+                auto flip = [&](auto jt) {
+                    constexpr int J = decltype(jt)::value;
+#pragma unroll
+                    for (int p = 0; p < R / 2; p++) {
+                        const int i0 = ((p >> J) << (J + 1)) | (p & ((1 << J) - 1)), i1 = i0 | (1 << J);
+                        if ((static_cast<uint32_t>(i0) & rm) == rv) {
+#pragma unroll
+                            for (int i = 0; i < S; i++) {
+                                sweep_exchange(lanes, x[i][i0], x[i][i1]);
+                            }
+                        }
+                    }
+                };
+                switch (st.j) {
+                case 0: flip(std::integral_constant<int, 0>{}); break;
+                case 1: flip(std::integral_constant<int, 1>{}); break;
+                default: flip(std::integral_constant<int, 2>{}); break;
+                }
+            } else { // kSweepDiag
+                const dcx<double> u0 = st.u[0], u1 = st.u[1];
+                // this lane's phase at even and at odd parity of the register index
+                const dcx<double> ue{tpar ? u1.r : u0.r, tpar ? u1.i : u0.i}, uo{tpar ? u0.r : u1.r, tpar ? u0.i : u1.i};
+#pragma unroll
+                for (int r = 0; r < R; r++) {
+                    if ((static_cast<uint32_t>(r) & rm) == rv) {
+                        const bool odd = __popc(static_cast<uint32_t>(r) & rp) & 1U; // uniform
+                        const dcx<double> u{odd ? uo.r : ue.r, odd ? uo.i : ue.i};
+#pragma unroll
+                        for (int i = 0; i < S; i++) {
+                            sweep_into(lanes, x[i][r], u.r, -u.i * x[i][r].y, u.i * x[i][r].x);
+                        }
+                    }
+                }
+            }
+        }
+        if (win != HOME) {
+            window(HOME);
+        }
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const uint32_t e = (static_cast<uint32_t>(r) << TB) | tid;
+            const uint64_t a = base | thread_at | spread(static_cast<uint32_t>(r) << TB);
+            if (e < size) {
+                if (grp == A.writer) {
+                    A.lam_out[a] = v2<T>{static_cast<T>(x[0][r].x), static_cast<T>(x[0][r].y)};
+                }
+#pragma unroll
+                for (int kk = 0; kk < KH; kk++) {
+                    if (kk < nk) {
+                        h[kk][a] = v2<T>{static_cast<T>(x[1 + kk][r].x), static_cast<T>(x[1 + kk][r].y)};
+                    }
+                }
             }
         }
     }
     __syncthreads();
-    if (threadIdx.x < nobs) {
-        double t = 0;
-        for (int w = 0; w < kBlock / 64; w++) {
-            t += wpart[w][threadIdx.x];
+    for (int i = tid; i < nsum; i += 64 * NW) {
+        const int c = i % NC, kk = (i / NC) % KH, slot = i / (NC * KH);
+        double t = sums[i];
+        for (int v = 1; v < NW; v++) {
+            t += sums[v * nsum + i];
         }
-        out[threadIdx.x] = t;
+        if (kk < nk) {
+            A.partial[((static_cast<uint64_t>(A.slot0 + slot) * NC + c) * A.K + k0 + kk) * A.W + w] = t;
+        }
     }
 }
 
-// states[0] = lambda, states[1 .. nobs] = H_k of this launch.
-// TRAIN: accumulate Im<H_k|G lambda>; partial[block * nobs + k].
-// update_lambda: write U^dag lambda (only the last launch of an op does).
-template <class T, int M, bool TRAIN>
-__global__ __launch_bounds__(kBlock) void k_adjoint_step(v2<T> *const *__restrict__ states,
-                                                         int nobs, uint64_t nwork,
-                                                         const AdjOp<T, M> op,
-                                                         int update_lambda,
-                                                         double *__restrict__ partial) {
-    double acc[kAdjMaxObs];
-#pragma unroll
-    for (int k = 0; k < kAdjMaxObs; k++) {
-        acc[k] = 0;
-    }
-    v2<T> *lam = states[0];
-    const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kBlock;
-    for (uint64_t g = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x; g < nwork; g += stride) {
-        const uint64_t base = expand(g, op.geo);
-        v2<T> x[M], y[M], mu[M];
-        if (TRAIN || update_lambda) {
-#pragma unroll
-            for (int j = 0; j < M; j++) {
-                x[j] = lam[base | op.off[j]];
-            }
-        }
-        if (TRAIN) {
-            matvec<T, M>(op.g, 0, x, mu);
-        }
-        if (update_lambda) {
-            matvec<T, M>(op.ud, op.ud_diag, x, y);
-#pragma unroll
-            for (int j = 0; j < M; j++) {
-                lam[base | op.off[j]] = y[j];
-            }
-        }
-        // observables in chunks: a chunk's loads are all issued before its
-        // stores (the H_k may alias as far as the compiler knows)
-#pragma unroll
-        for (int k0 = 0; k0 < kAdjMaxObs; k0 += kAdjChunk) {
-            v2<T> hx[kAdjChunk][M];
-#pragma unroll
-            for (int c = 0; c < kAdjChunk; c++) {
-                if (k0 + c < nobs) {
-                    const v2<T> *h = states[1 + k0 + c];
-#pragma unroll
-                    for (int j = 0; j < M; j++) {
-                        hx[c][j] = h[base | op.off[j]];
-                    }
-                }
-            }
-#pragma unroll
-            for (int c = 0; c < kAdjChunk; c++) {
-                if (k0 + c < nobs) {
-                    if (TRAIN) {
-                        double s = 0;
-#pragma unroll
-                        for (int j = 0; j < M; j++) {
-                            // Im(conj(h) * mu)
-                            s += double(hx[c][j].x) * double(mu[j].y) - double(hx[c][j].y) * double(mu[j].x);
-                        }
-                        acc[k0 + c] += s;
-                    }
-                    matvec<T, M>(op.ud, op.ud_diag, hx[c], y);
-                    v2<T> *h = states[1 + k0 + c];
-#pragma unroll
-                    for (int j = 0; j < M; j++) {
-                        h[base | op.off[j]] = y[j];
-                    }
-                }
-            }
-        }
-    }
-    if (TRAIN) {
-        adj_block_totals(acc, nobs, partial + static_cast<uint64_t>(blockIdx.x) * nobs);
-    }
-}
-
-// Same step for parity-phase ops (MultiRZ): per amplitude, U^dag and G are
-// phases selected by the parity of i & mask.
-template <class T, bool TRAIN>
-__global__ __launch_bounds__(kBlock) void k_adjoint_parity(v2<T> *const *__restrict__ states,
-                                                           int nobs, uint64_t len, uint64_t mask,
-                                                           dcx<T> u0, dcx<T> u1, dcx<T> g0,
-                                                           dcx<T> g1, int update_lambda,
-                                                           double *__restrict__ partial) {
-    double acc[kAdjMaxObs];
-#pragma unroll
-    for (int k = 0; k < kAdjMaxObs; k++) {
-        acc[k] = 0;
-    }
-    v2<T> *lam = states[0];
-    const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kBlock;
-    for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x; i < len; i += stride) {
-        const bool odd = __popcll(i & mask) & 1;
-        const dcx<T> u = odd ? u1 : u0;
-        v2<T> x;
-        if (TRAIN || update_lambda) {
-            x = lam[i];
-        }
-        v2<T> mu;
-        if (TRAIN) {
-            mu = cmul(odd ? g1 : g0, x);
-        }
-        if (update_lambda) {
-            lam[i] = cmul(u, x);
-        }
-#pragma unroll
-        for (int k0 = 0; k0 < kAdjMaxObs; k0 += kAdjChunk) {
-            v2<T> hv[kAdjChunk];
-#pragma unroll
-            for (int c = 0; c < kAdjChunk; c++) {
-                if (k0 + c < nobs) {
-                    hv[c] = states[1 + k0 + c][i];
-                }
-            }
-#pragma unroll
-            for (int c = 0; c < kAdjChunk; c++) {
-                if (k0 + c < nobs) {
-                    if (TRAIN) {
-                        acc[k0 + c] += double(hv[c].x) * double(mu.y) - double(hv[c].y) * double(mu.x);
-                    }
-                    states[1 + k0 + c][i] = cmul(u, hv[c]);
-                }
-            }
-        }
-    }
-    if (TRAIN) {
-        adj_block_totals(acc, nobs, partial + static_cast<uint64_t>(blockIdx.x) * nobs);
-    }
-}
-
-// Trainable steps whose partial sums wait in their own slots of the partial
-// buffer, reduced together by one launch (k_adjoint_final_many).
-constexpr int kAdjFinalSlots = 64;
-struct AdjFinal {
-    double factor; // the generator's scale times -2 (sign of the inverse)
-    int nblocks;   // blocks of the step's launch, each wrote nobs partials
-    int nobs;      // observables of the launch
-    int dst;       // jacobian offset of its first observable
-};
-struct AdjFinals {
-    AdjFinal t[kAdjFinalSlots];
-};
-
-// For slot s = blockIdx.y and observable k = blockIdx.x:
-// jac[dst + k] = factor * sum_b partial_s[b * nobs + k], 256 threads each
-// summing a strided share of the blocks, then a fixed-order block sum.
-__global__ __launch_bounds__(kBlock) void k_adjoint_final_many(const double *__restrict__ partial,
-                                                               size_t slot_stride, const AdjFinals tab,
-                                                               double *__restrict__ jac) {
-    const AdjFinal t = tab.t[blockIdx.y];
-    const int k = blockIdx.x;
-    if (k >= t.nobs) {
-        return; // the whole block
-    }
-    const double *p = partial + static_cast<size_t>(blockIdx.y) * slot_stride;
+// out[v] = sum of partial[v * W .. + W), one wavefront per value, fixed order
+static __global__ __launch_bounds__(64) void k_sweep_sums(const double *__restrict__ partial, int W,
+                                                          double *__restrict__ out) {
+    const double *p = partial + static_cast<uint64_t>(blockIdx.x) * W;
     double s = 0;
-    for (int b = threadIdx.x; b < t.nblocks; b += kBlock) {
-        s += p[static_cast<size_t>(b) * t.nobs + k];
+    for (int i = threadIdx.x; i < W; i += 64) {
+        s += p[i];
     }
-    const double2 r = block_sum2(double2{s, 0});
+    s = wave_sum(s);
     if (threadIdx.x == 0) {
-        jac[t.dst + k] = t.factor * r.x;
-    }
-}
-
-// Fused step of the vector-Jacobian product's backward sweep
-// (VectorJacobianProduct.hpp:77-155): per amplitude group of the op, load
-// lambda's and mu's groups; if the op is trainable, accumulate the complex
-// <mu|G lambda> (= <G mu|lambda>, G Hermitian and zero outside the op's
-// geometry); store U^dag lambda and U^dag mu.  One launch per op, each state
-// read and written once; partial[blockIdx.x] = the block's sum.
-template <class T, int M, bool TRAIN>
-__global__ __launch_bounds__(kBlock) void k_vjp_step(v2<T> *__restrict__ lam, v2<T> *__restrict__ mu,
-                                                     uint64_t nwork, const AdjOp<T, M> op,
-                                                     double2 *__restrict__ partial) {
-    double2 acc{0, 0};
-    const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kBlock;
-    for (uint64_t g = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x; g < nwork; g += stride) {
-        const uint64_t base = expand(g, op.geo);
-        v2<T> x[M], h[M], y[M];
-#pragma unroll
-        for (int j = 0; j < M; j++) {
-            x[j] = lam[base | op.off[j]];
-            h[j] = mu[base | op.off[j]];
-        }
-        if (TRAIN) {
-            v2<T> gx[M];
-            matvec<T, M>(op.g, 0, x, gx);
-#pragma unroll
-            for (int j = 0; j < M; j++) {
-                // conj(h) * gx
-                acc.x += double(h[j].x) * double(gx[j].x) + double(h[j].y) * double(gx[j].y);
-                acc.y += double(h[j].x) * double(gx[j].y) - double(h[j].y) * double(gx[j].x);
-            }
-        }
-        matvec<T, M>(op.ud, op.ud_diag, x, y);
-#pragma unroll
-        for (int j = 0; j < M; j++) {
-            lam[base | op.off[j]] = y[j];
-        }
-        matvec<T, M>(op.ud, op.ud_diag, h, y);
-#pragma unroll
-        for (int j = 0; j < M; j++) {
-            mu[base | op.off[j]] = y[j];
-        }
-    }
-    if (TRAIN) {
-        const double2 r = block_sum2(acc);
-        if (threadIdx.x == 0) {
-            partial[blockIdx.x] = r;
-        }
-    }
-}
-
-// The same for parity-phase ops (MultiRZ): U^dag and G are phases selected
-// by the parity of i & mask.
-template <class T, bool TRAIN>
-__global__ __launch_bounds__(kBlock) void k_vjp_parity(v2<T> *__restrict__ lam, v2<T> *__restrict__ mu,
-                                                       uint64_t len, uint64_t mask, dcx<T> u0, dcx<T> u1,
-                                                       dcx<T> g0, dcx<T> g1, double2 *__restrict__ partial) {
-    double2 acc{0, 0};
-    const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kBlock;
-    for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x; i < len; i += stride) {
-        const bool odd = __popcll(i & mask) & 1;
-        const v2<T> x = lam[i], h = mu[i];
-        if (TRAIN) {
-            const v2<T> gx = cmul(odd ? g1 : g0, x);
-            acc.x += double(h.x) * double(gx.x) + double(h.y) * double(gx.y);
-            acc.y += double(h.x) * double(gx.y) - double(h.y) * double(gx.x);
-        }
-        const dcx<T> u = odd ? u1 : u0;
-        lam[i] = cmul(u, x);
-        mu[i] = cmul(u, h);
-    }
-    if (TRAIN) {
-        const double2 r = block_sum2(acc);
-        if (threadIdx.x == 0) {
-            partial[blockIdx.x] = r;
-        }
-    }
-}
-
-// out[rows[b]] = sum over i < nblocks of partial[rows[b] * nblocks + i], in
-// a fixed order: one block per row
-__global__ __launch_bounds__(kBlock) void k_vjp_final(const double2 *__restrict__ partial, int nblocks,
-                                                      const int *__restrict__ rows, double2 *__restrict__ out) {
-    const int t = rows[blockIdx.x];
-    double2 s{0, 0};
-    for (int b = threadIdx.x; b < nblocks; b += kBlock) {
-        const double2 p = partial[static_cast<size_t>(t) * nblocks + b];
-        s.x += p.x;
-        s.y += p.y;
-    }
-    const double2 r = block_sum2(s);
-    if (threadIdx.x == 0) {
-        out[t] = r;
+        out[blockIdx.x] = s;
     }
 }
 

@@ -21,6 +21,7 @@
 #include <cstdint>
 #include <stdexcept>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 namespace plamd {
@@ -403,6 +404,34 @@ GroupOp<P> lower_gate(int n, int id, const int *wires, int nw, bool inv, const P
     }
     default:
         throw OutOfRange("unknown gate id");
+    }
+}
+
+// A gate lowered in double and rounded to P once: its matrix is the nearest to
+// the exact one, where lowering in P would round the angle first (an angle
+// near 2 pi loses 2e-7 in float, more than every later rounding).
+template <class P>
+GroupOp<P> lower_gate_as(int n, int id, const int *wires, int nw, bool inv, const double *prm, int np) {
+    GroupOp<double> d = lower_gate<double>(n, id, wires, nw, inv, prm, np);
+    if constexpr (std::is_same_v<P, double>) {
+        return d;
+    } else {
+        GroupOp<P> g;
+        g.kind = static_cast<typename GroupOp<P>::Kind>(d.kind);
+        g.M = d.M;
+        g.nb = d.nb;
+        std::copy(d.pos, d.pos + kMaxPos, g.pos);
+        g.fixed = d.fixed;
+        g.off = std::move(d.off);
+        for (const auto &z : d.mat) {
+            g.mat.emplace_back(static_cast<P>(z.real()), static_cast<P>(z.imag()));
+        }
+        g.diag = d.diag;
+        g.parity_mask = d.parity_mask;
+        for (int j = 0; j < 2; j++) {
+            g.parity_phase[j] = {static_cast<P>(d.parity_phase[j].real()), static_cast<P>(d.parity_phase[j].imag())};
+        }
+        return g;
     }
 }
 

@@ -8,7 +8,7 @@
 // HIP stream.  There is no CPU compute path: if the device work cannot be
 // enqueued the call fails with PL_ERR_DEVICE.
 #include "engine_common.hpp"
-#include "kernels_adjoint.hpp"
+#include "sweep.hpp"
 #include "kernels_reduce.hpp"
 #include "kernels_sample.hpp"
 #include "kernels_mfma.hpp"
@@ -357,17 +357,8 @@ template <class T> struct Engine {
         }
     }
 
-    std::vector<T> params_t(const double *p, int np) const {
-        std::vector<T> v(np);
-        for (int i = 0; i < np; i++) {
-            v[i] = static_cast<T>(p[i]);
-        }
-        return v;
-    }
-
     void gate(V *sv, int id, const int *w, int nw, bool inv, const double *p, int np) {
-        const auto pt = params_t(p, np);
-        apply(lower_gate<T>(n(), id, w, nw, inv, pt.data(), np), sv);
+        apply(lower_gate_as<T>(n(), id, w, nw, inv, p, np), sv);
     }
 
     void matrix(V *sv, const double *m, const int *w, int nw, bool inv) {
@@ -708,16 +699,6 @@ template <class T> struct Engine {
         HIP_OK(hipMemcpyAsync(&r, part + kReduceBlocks, sizeof(r), hipMemcpyDeviceToHost, h->stream));
         HIP_OK(hipStreamSynchronize(h->stream));
         return {r.x, r.y};
-    }
-
-    // <a|b> left in device memory at *slot, ordered on the engine's stream with
-    // no wait; part holds kReduceBlocks partials and must not overlap slot.
-    void dot_to(const V *a, const V *b, double2 *part, double2 *slot) {
-        const unsigned grid = std::min<unsigned>(grid_for(len(), 1, 4), kReduceBlocks);
-        hipLaunchKernelGGL((k_dot<T>), dim3(grid), dim3(kBlock), 0, h->stream, a, b, len(), part);
-        HIP_OK(hipGetLastError());
-        hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(kBlock), 0, h->stream, part, (int)grid, slot);
-        HIP_OK(hipGetLastError());
     }
 
     // sum_t c_t <psi|P_t|psi> over Pauli words, grouped by x-mask
@@ -1389,31 +1370,232 @@ template <class F> int dispatch(pl_sv_t h, F &&f) {
 }
 
 // ---------------------------------------------------------------------------
-// adjoint sweep (AdjointJacobianLQubit.hpp:212-336)
+// Backward sweep of the adjoint Jacobian and the VJP (kernels_adjoint.hpp,
+// sweep.hpp): lam = the final state, hs = the K states swept with it (all
+// scratch, overwritten).  emit(t, k, z, scale): a part z of <h_k|G lambda> at
+// trainable parameter t = 0 .. ntp - 1 (its imaginary part only unless FULL),
+// the parts to be added up; scale = the generator's, negated for an inverted
+// operation; parameters that no operation carries are not reported.
 // ---------------------------------------------------------------------------
-template <class T>
-void adjoint_sweep(Engine<T> &E, int nops, const int *ids, const int *nwires, const int *wires,
-                   const uint8_t *inverse, const int *nparams, const double *params,
-                   const int *prog, const double *coeffs, const double *mats, int ntp,
-                   const int *tp, double *jac_out) {
+struct SweepTape {
+    int nops;
+    const int *ids, *nwires, *wires;
+    const uint8_t *inverse;
+    const int *nparams;
+    const double *params;
+};
+
+template <class T> constexpr int kSweepLow = std::is_same_v<T, double> ? 3 : 4; // one 128-byte line
+// States up to this size keep a second lambda, so that every observable group
+// of a pass can run at once; larger ones fill the device group by group.
+constexpr size_t kSweepTwoLambdas = size_t{64} << 20;
+constexpr size_t kSweepPartBytes = size_t{64} << 20; // partial sums held before they are added up
+
+template <class T, bool FULL, class Emit>
+void backward_sweep(Engine<T> &E, const SweepTape &t, v2<T> *lam, const std::vector<v2<T> *> &hs, int ntp,
+                    const int *tp, Emit &&emit) {
     using V = v2<T>;
+    constexpr int NC = FULL ? kSweepFull : kSweepReal;
     pl_sv *h = E.h;
-    struct Op {
-        int id;
-        std::vector<int> w;
-        bool inv;
-        std::vector<double> p;
+    const int K = static_cast<int>(hs.size());
+    std::vector<int> woff(t.nops + 1, 0), poff(t.nops + 1, 0);
+    size_t num_par_ops = 0;
+    for (int i = 0; i < t.nops; i++) {
+        woff[i + 1] = woff[i] + t.nwires[i];
+        poff[i + 1] = poff[i] + t.nparams[i];
+        num_par_ops += t.nparams[i] > 0 ? 1 : 0;
+    }
+    SweepSteps builder;
+    std::vector<SweepOp> parts;
+    long long cur_param = static_cast<long long>(num_par_ops) - 1;
+    int tp_pos = ntp - 1;
+    for (int i = t.nops - 1; i >= 0; i--) {
+        if (t.nparams[i] > 1) {
+            throw InvalidArg("The operation is not supported using the adjoint differentiation method");
+        }
+        if (t.ids[i] == -1) {
+            continue;
+        }
+        if (tp_pos < 0) {
+            break;
+        }
+        const int *w = t.wires + woff[i];
+        const GroupOp<double> ud = lower_gate<double>(E.n(), t.ids[i], w, t.nwires[i], t.inverse[i] == 0,
+                                                      t.params + poff[i], t.nparams[i]);
+        bool train = false;
+        SweepTrain tr{};
+        GroupOp<double> g;
+        if (t.nparams[i] > 0) {
+            if (cur_param == tp[tp_pos]) {
+                train = true;
+                double s = 0;
+                g = lower_generator<double>(E.n(), t.ids[i], w, t.nwires[i], true, &s);
+                tr.row = tp_pos--;
+                tr.scale = s * (t.inverse[i] ? -1.0 : 1.0);
+            }
+            cur_param--;
+        }
+        if (ud.kind == GroupOp<double>::Noop) {
+            continue;
+        }
+        if (sweep_expand_op(ud, train ? &g : nullptr, tr, parts)) {
+            for (const SweepOp &op : parts) {
+                builder.add(op);
+            }
+            continue;
+        }
+        SweepOp op;
+        op.big = true;
+        op.tape = i;
+        for (int j = 0; j < t.nwires[i]; j++) {
+            op.extra |= uint64_t{1} << (E.n() - 1 - w[j]);
+        }
+        if (train) {
+            op.train.push_back(tr);
+        }
+        builder.add(op);
+    }
+    builder.finish();
+    const auto &steps = builder.steps;
+    if (steps.empty()) {
+        return;
+    }
+
+    // the widest tile the state fills: four wavefronts, or fewer for a small one
+    constexpr int RB = kSweepRegBits;
+    const int waves = E.n() >= 8 + RB ? 4 : E.n() == 7 + RB ? 2 : 1;
+    const int tb = 6 + (waves == 4 ? 2 : waves == 2 ? 1 : 0);
+    const int bits = std::min(E.n(), tb + RB), low = std::min(E.n(), kSweepLow<T>);
+    const uint64_t ntiles = E.len() >> bits;
+    // observables per workgroup: two share their lambda where that still
+    // leaves a workgroup for every place on the device (16 wavefronts a CU)
+    const uint64_t places = uint64_t(device_cus()) * 16 / waves;
+    const int KH = !FULL && K > 1 && ntiles * ((K + 1) / 2) >= places ? 2 : 1;
+    const int ngrp = (K + KH - 1) / KH;
+    const bool two = ngrp > 1 && h->state_bytes() <= kSweepTwoLambdas;
+    const int per_launch = two ? ngrp : 1; // groups per launch
+    // tile walkers per group: several workgroups a place, so that the last
+    // round is a small part of the pass
+    uint64_t walkers = std::min<uint64_t>(ntiles, std::max<uint64_t>(1, 6 * places / per_launch));
+    if (walkers >= 8) {
+        walkers &= ~uint64_t{7}; // one XCD's walkers are every eighth
+    }
+    const int W = static_cast<int>(walkers);
+
+    ScratchScope sc(h);
+    V *other = two ? static_cast<V *>(sc.get()) : lam;
+    V *mu = nullptr;
+    auto **dhs = static_cast<V **>(buf(h, kBufSweepStates, K * sizeof(V *)));
+    HIP_OK(hipMemcpyAsync(dhs, hs.data(), K * sizeof(V *), hipMemcpyHostToDevice, h->stream));
+    auto *dprog = static_cast<SweepStep *>(buf(h, kBufSweepProg, 2 * steps.size() * sizeof(SweepStep)));
+    std::vector<SweepStep> prog;
+    prog.reserve(2 * steps.size()); // steps and windows; never moves: copies may still read it
+    struct Drain { // nor does it end before them when a call below fails
+        hipStream_t s;
+        ~Drain() { (void)hipStreamSynchronize(s); }
+    } drain{h->stream};
+    // slots in flight: partial sums of `cap` slots before a reduction
+    size_t nslots_all = 0;
+    for (const auto &s : steps) {
+        nslots_all += !s.big && !s.train.empty() ? 1 : 0;
+    }
+    const size_t slot_bytes = size_t(NC) * K * W * sizeof(double);
+    const size_t cap = std::min<size_t>(std::max<size_t>(nslots_all, 1),
+                                        std::max<size_t>(kSweepSlots, kSweepPartBytes / slot_bytes));
+    auto *part = static_cast<double *>(buf(h, kBufSweepPart, cap * slot_bytes));
+    auto *dsums = static_cast<double *>(buf(h, kBufSweepSums, std::max<size_t>(nslots_all, 1) * NC * K * sizeof(double)));
+    std::vector<int> slot_step; // step of every slot so far
+    size_t reduced = 0;         // slots already added up
+    auto reduce = [&] {
+        const size_t m = slot_step.size() - reduced;
+        if (m > 0) {
+            HIP_OK(launch_sweep_sums(part, W, static_cast<unsigned>(m * NC * K), dsums + reduced * NC * K, h->stream));
+            reduced = slot_step.size();
+        }
     };
-    std::vector<Op> ops(nops);
-    for (int i = 0, wo = 0, po = 0; i < nops; i++) {
-        ops[i].id = ids[i];
-        ops[i].w.assign(wires + wo, wires + wo + nwires[i]);
-        wo += nwires[i];
-        ops[i].inv = inverse[i] != 0;
-        ops[i].p.assign(params + po, params + po + nparams[i]);
-        po += nparams[i];
-        if (ops[i].id != -1) {
-            gate_name(ops[i].id);
+
+    SweepScheduler sched(E.n(), bits, low, steps);
+    SweepPass ps;
+    while (sched.next(ps)) {
+        if (ps.big) {
+            // lambda and every h op by op: dots with mu = G lambda first
+            const SweepOp &op = steps[ps.ops[0]];
+            const int i = op.tape;
+            const int *w = t.wires + woff[i];
+            const GroupOp<T> ud = lower_gate_as<T>(E.n(), t.ids[i], w, t.nwires[i], t.inverse[i] == 0,
+                                                   t.params + poff[i], t.nparams[i]);
+            for (const auto &tr : op.train) {
+                if (!mu) {
+                    mu = static_cast<V *>(sc.get());
+                }
+                E.copy(mu, lam);
+                T s = 0;
+                E.apply(lower_generator<T>(E.n(), t.ids[i], w, t.nwires[i], false, &s), mu);
+                for (int k = 0; k < K; k++) {
+                    emit(tr.row, k, E.dot(hs[k], mu), tr.scale);
+                }
+            }
+            E.apply(ud, lam);
+            for (V *s : hs) {
+                E.apply(ud, s);
+            }
+            continue;
+        }
+        const size_t p0 = prog.size();
+        size_t mine = 0;
+        for (int i : ps.ops) {
+            mine += steps[i].train.empty() ? 0 : 1;
+        }
+        if (slot_step.size() - reduced + mine > cap) {
+            reduce();
+        }
+        const size_t slot0 = slot_step.size() - reduced;
+        for (int i : ps.ops) {
+            if (!steps[i].train.empty()) {
+                slot_step.push_back(i);
+            }
+        }
+        sweep_program(steps, ps, low, tb, prog);
+        const int ns = static_cast<int>(prog.size() - p0);
+        HIP_OK(hipMemcpyAsync(dprog + p0, prog.data() + p0, ns * sizeof(SweepStep), hipMemcpyHostToDevice,
+                              h->stream));
+        SweepArgs<T> a{lam, other, dhs, K, 0, 0, ngrp - 1, W, ntiles, {}, dprog + p0, ns, static_cast<int>(mine),
+                       static_cast<int>(slot0), part};
+        a.geo.bits = bits;
+        a.geo.low = low;
+        std::copy(ps.hb.begin(), ps.hb.end(), a.geo.hb);
+        for (int g0 = 0; g0 < ngrp; g0 += per_launch) {
+            a.grp0 = g0;
+            a.ngrp = std::min(per_launch, ngrp - g0);
+            HIP_OK(launch_sweep<T>(waves, KH, FULL, a, h->stream));
+        }
+        std::swap(lam, other);
+    }
+    reduce();
+    std::vector<double> sums(slot_step.size() * NC * K);
+    if (!sums.empty()) {
+        HIP_OK(hipMemcpyAsync(sums.data(), dsums, sums.size() * sizeof(double), hipMemcpyDeviceToHost, h->stream));
+    }
+    HIP_OK(hipStreamSynchronize(h->stream)); // also ends every copy from prog and hs
+    for (size_t sl = 0; sl < slot_step.size(); sl++) {
+        const SweepOp &op = steps[slot_step[sl]];
+        for (int k = 0; k < K; k++) {
+            auto c = [&](int i) { return sums[(sl * NC + i) * K + k]; };
+            for (const auto &tr : op.train) {
+                emit(tr.row, k, sweep_value(tr, FULL, c), tr.scale);
+            }
+        }
+    }
+}
+
+// AdjointJacobian::adjointJacobian (AdjointJacobianLQubit.hpp:212-336)
+template <class T>
+void adjoint_sweep(Engine<T> &E, const SweepTape &t, const int *prog, const double *coeffs, const double *mats,
+                   int ntp, const int *tp, double *jac_out) {
+    using V = v2<T>;
+    for (int i = 0; i < t.nops; i++) {
+        if (t.ids[i] != -1) {
+            gate_name(t.ids[i]);
         }
     }
     ObsReader rd{prog, coeffs, mats};
@@ -1425,254 +1607,30 @@ void adjoint_sweep(Engine<T> &E, int nops, const int *ids, const int *nwires, co
     if (ntp == 0) {
         return; // JacobianData::hasTrainableParams() false: nothing to do
     }
-    for (int t = 1; t < ntp; t++) {
-        if (tp[t] <= tp[t - 1]) {
+    for (int i = 1; i < ntp; i++) {
+        if (tp[i] <= tp[i - 1]) {
             throw InvalidArg("trainable parameter indices must be sorted ascending");
         }
     }
     if (K == 0) {
         return;
     }
-    ScratchScope sc(h);
+    ScratchScope sc(E.h);
     V *lam = static_cast<V *>(sc.get());
     E.copy(lam, E.psi());
-    std::vector<V *> states{lam};
+    std::vector<V *> hs;
     for (int k = 0; k < K; k++) {
         V *hk = static_cast<V *>(sc.get());
         E.obs_into(hk, lam, obs[k]);
-        states.push_back(hk);
+        hs.push_back(hk);
     }
-    // Observables per sweep: when lambda and every H_k exceed the on-die
-    // cache but fit in it in groups, the sweep runs once per group with a
-    // fresh lambda, so each group's states stay cache-resident across ops.
-    const size_t sbytes = E.len() * sizeof(V);
-    int per_sweep = K;
-    if (sbytes * (K + 1) > kAdjCacheBytes && sbytes * 2 <= kAdjCacheBytes) {
-        const int fit = std::max<int>(1, static_cast<int>(kAdjCacheBytes / sbytes) - 1);
-        const int nsweep = (K + fit - 1) / fit;
-        per_sweep = (K + nsweep - 1) / nsweep;
-    }
-    // device tables: state pointers, jacobian, partials
-    V **dstates = nullptr;
-    double *djac = nullptr, *dpart = nullptr;
-    const unsigned grid = std::min<unsigned>(grid_for(E.len(), 1, 8), kReduceBlocks);
-    // one pointer table per chunk of at most kAdjMaxObs observables of a
-    // sweep: lambda, then the chunk's H_k (built once, so no launch waits on
-    // a staging copy); chunks are numbered sweep by sweep
-    std::vector<V *> tables;
-    for (int s0 = 0; s0 < K; s0 += per_sweep) {
-        const int ns = std::min(per_sweep, K - s0);
-        for (int k0 = 0; k0 < ns; k0 += kAdjMaxObs) {
-            const size_t at = tables.size();
-            tables.resize(at + kAdjMaxObs + 1, nullptr);
-            tables[at] = lam;
-            for (int k = k0; k < std::min(ns, k0 + kAdjMaxObs); k++) {
-                tables[at + 1 + (k - k0)] = states[1 + s0 + k];
-            }
-        }
-    }
-    HIP_OK(hipMalloc(&dstates, tables.size() * sizeof(V *)));
-    HIP_OK(hipMalloc(&djac, size_t(ntp) * K * sizeof(double)));
-    // each trainable step's partial sums in a slot of their own; the slots'
-    // final sums run kAdjFinalSlots at a time (one launch, not one per step)
-    const size_t slot_stride = size_t(grid) * kAdjMaxObs;
-    HIP_OK(hipMalloc(&dpart, kAdjFinalSlots * slot_stride * sizeof(double)));
-    struct Free {
-        void *a, *b, *c;
-        ~Free() {
-            (void)hipFree(a);
-            (void)hipFree(b);
-            (void)hipFree(c);
-        }
-    } fr{dstates, djac, dpart};
-    HIP_OK(hipMemcpyAsync(dstates, tables.data(), tables.size() * sizeof(V *),
-                          hipMemcpyHostToDevice, E.h->stream));
-    HIP_OK(hipMemsetAsync(djac, 0, size_t(ntp) * K * sizeof(double), E.h->stream));
-
-    size_t num_par_ops = 0;
-    for (auto &o : ops) {
-        num_par_ops += o.p.empty() ? 0 : 1;
-    }
-    AdjFinals pending{};
-    int npending = 0;
-    auto flush_finals = [&] {
-        if (npending > 0) {
-            hipLaunchKernelGGL(k_adjoint_final_many, dim3(kAdjMaxObs, npending), dim3(kBlock), 0, E.h->stream,
-                               dpart, slot_stride, pending, djac);
-            HIP_OK(hipGetLastError());
-            npending = 0;
-        }
-    };
-    // the slot for the next trainable step's partials (all slots in use: their
-    // sums first)
-    auto slot = [&] {
-        if (npending == kAdjFinalSlots) {
-            flush_finals();
-        }
-        return dpart + static_cast<size_t>(npending) * slot_stride;
-    };
-    auto finish = [&](unsigned nblocks, int nk, double factor, int dst) {
-        pending.t[npending++] = AdjFinal{factor, static_cast<int>(nblocks), nk, dst};
-    };
-    ScratchScope sc2(h);
-    V *mu = nullptr;
-    size_t chunk_base = 0; // first pointer table of the current sweep
-    for (int s0 = 0; s0 < K; s0 += per_sweep) {
-    const int ns = std::min(per_sweep, K - s0);
-    if (s0 > 0) {
-        E.copy(lam, E.psi()); // the next group starts again from psi
-    }
-    int t_num = ntp - 1;
-    long long cur_param = static_cast<long long>(num_par_ops) - 1;
-    int tp_pos = ntp - 1;
-    for (int i = nops - 1; i >= 0; i--) {
-        const Op &op = ops[i];
-        if (op.p.size() > 1) {
-            throw InvalidArg("The operation is not supported using the adjoint differentiation method");
-        }
-        if (op.id == -1) {
-            continue;
-        }
-        if (tp_pos < 0) {
-            break;
-        }
-        const auto pt = E.params_t(op.p.data(), static_cast<int>(op.p.size()));
-        const GroupOp<T> ud = lower_gate<T>(E.n(), op.id, op.w.data(), static_cast<int>(op.w.size()),
-                                            !op.inv, pt.data(), static_cast<int>(pt.size()));
-        bool train = false;
-        GroupOp<T> g;
-        double factor = 0;
-        int row = 0;
-        if (!op.p.empty()) {
-            if (cur_param == tp[tp_pos]) {
-                train = true;
-                T s = 0;
-                g = lower_generator<T>(E.n(), op.id, op.w.data(), static_cast<int>(op.w.size()),
-                                       true, &s);
-                factor = -2.0 * static_cast<double>(s) * (op.inv ? -1.0 : 1.0);
-                row = t_num * K + s0;
-                t_num--;
-                tp_pos--;
-            }
-            cur_param--;
-        }
-        const bool fusable =
-            ud.kind == GroupOp<T>::Noop ||
-            (ud.kind == GroupOp<T>::Parity && (!train || g.same_geometry(ud))) ||
-            (ud.kind == GroupOp<T>::Group && ud.M <= 4 && (!train || g.same_geometry(ud)));
-        if (!fusable) {
-            // unfused: mu = lambda; lambda <- U^dag lambda; mu <- G mu; dots; H_k <- U^dag H_k
-            if (train) {
-                if (!mu) {
-                    mu = static_cast<V *>(sc2.get());
-                }
-                E.copy(mu, lam);
-            }
-            E.apply(ud, lam);
-            if (train) {
-                T s = 0;
-                E.apply(lower_generator<T>(E.n(), op.id, op.w.data(), static_cast<int>(op.w.size()),
-                                           false, &s),
-                        mu);
-                std::vector<double> row_vals(ns);
-                for (int k = 0; k < ns; k++) {
-                    row_vals[k] = factor * E.dot(states[1 + s0 + k], mu).imag();
-                }
-                HIP_OK(hipMemcpyAsync(djac + row, row_vals.data(), ns * sizeof(double),
-                                      hipMemcpyHostToDevice, E.h->stream));
-                HIP_OK(hipStreamSynchronize(E.h->stream));
-            }
-            for (int k = 0; k < ns; k++) {
-                E.apply(ud, states[1 + s0 + k]);
-            }
-            continue;
-        }
-        if (ud.kind == GroupOp<T>::Noop) {
-            // Identity: U^dag = I, no generator
-            continue;
-        }
-        // fused launches, kAdjMaxObs observables each; lambda updated by the last
-        for (int k0 = 0; k0 < ns; k0 += kAdjMaxObs) {
-            const int nk = std::min(kAdjMaxObs, ns - k0);
-            const int upd = (k0 + nk == ns) ? 1 : 0;
-            // states for this launch: lambda followed by H_(s0+k0) .. H_(s0+k0+nk-1)
-            V *const *st = dstates + (chunk_base + size_t(k0 / kAdjMaxObs)) * (kAdjMaxObs + 1);
-            if (ud.kind == GroupOp<T>::Parity) {
-                const dcx<T> u0{ud.parity_phase[0].real(), ud.parity_phase[0].imag()};
-                const dcx<T> u1{ud.parity_phase[1].real(), ud.parity_phase[1].imag()};
-                dcx<T> g0{1, 0}, g1{1, 0};
-                if (train) {
-                    g0 = {g.parity_phase[0].real(), g.parity_phase[0].imag()};
-                    g1 = {g.parity_phase[1].real(), g.parity_phase[1].imag()};
-                    hipLaunchKernelGGL((k_adjoint_parity<T, true>), dim3(grid), dim3(kBlock), 0,
-                                       E.h->stream, st, nk, E.len(), ud.parity_mask, u0, u1, g0,
-                                       g1, upd, slot());
-                } else {
-                    hipLaunchKernelGGL((k_adjoint_parity<T, false>), dim3(grid), dim3(kBlock), 0,
-                                       E.h->stream, st, nk, E.len(), ud.parity_mask, u0, u1, g0,
-                                       g1, upd, dpart);
-                }
-            } else {
-                auto go = [&](auto mtag) {
-                    constexpr int M = decltype(mtag)::value;
-                    AdjOp<T, M> a{};
-                    a.geo.fixed = ud.fixed;
-                    a.geo.nb = ud.nb;
-                    for (int q = 0; q < ud.nb; q++) {
-                        a.geo.pos[q] = ud.pos[q];
-                    }
-                    for (int j = 0; j < M; j++) {
-                        a.off[j] = ud.off[j];
-                    }
-                    for (int j = 0; j < M * M; j++) {
-                        a.ud[j] = {ud.mat[j].real(), ud.mat[j].imag()};
-                        a.g[j] = train ? dcx<T>{g.mat[j].real(), g.mat[j].imag()} : dcx<T>{0, 0};
-                    }
-                    a.ud_diag = ud.diag ? 1 : 0;
-                    const uint64_t nwork = E.len() >> ud.nb;
-                    // a trainable step ends with one cross-lane reduction per observable
-                    // in every wavefront: two work items per thread amortise it
-                    const unsigned gr = std::min<unsigned>(grid_for(nwork, train ? 2 : 1, 8), kReduceBlocks);
-                    if (train) {
-                        hipLaunchKernelGGL((k_adjoint_step<T, M, true>), dim3(gr), dim3(kBlock), 0,
-                                           E.h->stream, st, nk, nwork, a, upd, slot());
-                    } else {
-                        hipLaunchKernelGGL((k_adjoint_step<T, M, false>), dim3(gr), dim3(kBlock), 0,
-                                           E.h->stream, st, nk, nwork, a, upd, dpart);
-                    }
-                    return gr;
-                };
-                unsigned gr = 0;
-                switch (ud.M) {
-                case 1: gr = go(std::integral_constant<int, 1>{}); break;
-                case 2: gr = go(std::integral_constant<int, 2>{}); break;
-                default: gr = go(std::integral_constant<int, 4>{}); break;
-                }
-                HIP_OK(hipGetLastError());
-                if (train) {
-                    finish(gr, nk, factor, row + k0);
-                }
-                continue;
-            }
-            HIP_OK(hipGetLastError());
-            if (train) {
-                finish(grid, nk, factor, row + k0);
-            }
-        }
-    }
-    chunk_base += static_cast<size_t>((ns + kAdjMaxObs - 1) / kAdjMaxObs);
-    }
-    flush_finals();
-    std::vector<double> J(size_t(ntp) * K);
-    HIP_OK(hipMemcpyAsync(J.data(), djac, J.size() * sizeof(double), hipMemcpyDeviceToHost,
-                          E.h->stream));
-    HIP_OK(hipStreamSynchronize(E.h->stream));
-    // parameter-major -> observable-major (AdjointJacobianLQubit.hpp:331-334)
-    for (int k = 0; k < K; k++) {
-        for (int t = 0; t < ntp; t++) {
-            jac_out[size_t(k) * ntp + t] = J[size_t(t) * K + k];
-        }
-    }
+    // observable-major (AdjointJacobianLQubit.hpp:331-334); written once the
+    // whole sweep has succeeded
+    std::vector<double> J(size_t(ntp) * K, 0.0);
+    backward_sweep<T, false>(E, t, lam, hs, ntp, tp, [&](int row, int k, std::complex<double> z, double scale) {
+        J[size_t(k) * ntp + row] -= 2.0 * scale * z.imag();
+    });
+    std::copy(J.begin(), J.end(), jac_out);
 }
 
 } // namespace plamd
@@ -1683,30 +1641,19 @@ using namespace plamd;
 // extern "C"
 // ===========================================================================
 // VectorJacobianProduct::operator() (VectorJacobianProduct.hpp:77-155):
-// lambda = psi, mu = dy; for operations in reverse (state preparations
-// skipped, stopping once every trainable parameter is done): for a trainable
-// one, w_t = i s <G mu | lambda> with s the generator scale times -1 for an
-// inverted operation; then lambda <- U^dag lambda and mu <- U^dag mu.  Ops of
-// at most 4 members (and parity phases) whose generator shares their
-// geometry take one fused launch each (k_vjp_step); the rest go op by op.
+// lambda = psi, mu = dy; w_t = i s <G mu | lambda> with s the generator scale
+// times -1 for an inverted operation (G is Hermitian).
 template <class T>
-void vjp_sweep(Engine<T> &E, int nops, const int *ids, const int *nwires, const int *wires,
-               const uint8_t *inverse, const int *nparams, const double *params, const double *dy,
-               int ntp, const int *tp, double *out) {
+void vjp_sweep(Engine<T> &E, const SweepTape &t, const double *dy, int ntp, const int *tp, double *out) {
     using V = v2<T>;
     pl_sv *h = E.h;
-    std::vector<int> woff(nops + 1, 0), poff(nops + 1, 0);
-    size_t num_par_ops = 0;
-    for (int i = 0; i < nops; i++) {
-        woff[i + 1] = woff[i] + nwires[i];
-        poff[i + 1] = poff[i] + nparams[i];
-        num_par_ops += nparams[i] > 0 ? 1 : 0;
-        if (ids[i] != -1) {
-            gate_name(ids[i]);
+    for (int i = 0; i < t.nops; i++) {
+        if (t.ids[i] != -1) {
+            gate_name(t.ids[i]);
         }
     }
-    for (int t = 1; t < ntp; t++) {
-        if (tp[t] <= tp[t - 1]) {
+    for (int i = 1; i < ntp; i++) {
+        if (tp[i] <= tp[i - 1]) {
             throw InvalidArg("trainable parameter indices must be sorted ascending");
         }
     }
@@ -1716,140 +1663,30 @@ void vjp_sweep(Engine<T> &E, int nops, const int *ids, const int *nwires, const 
     ScratchScope sc(h);
     V *lam = static_cast<V *>(sc.get());
     V *mu = static_cast<V *>(sc.get());
-    V *mud = static_cast<V *>(sc.get());
     E.copy(lam, E.psi());
-    {
-        std::vector<V> host(E.len());
+    std::vector<V> host;
+    if constexpr (std::is_same_v<T, double>) {
+        upload_host(h, mu, dy, E.len() * sizeof(V)); // the same layout
+    } else {
+        host.resize(E.len());
         for (uint64_t i = 0; i < E.len(); i++) {
             host[i].x = static_cast<T>(dy[2 * i]);
             host[i].y = static_cast<T>(dy[2 * i + 1]);
         }
         upload_host(h, mu, host.data(), E.len() * sizeof(V));
-        HIP_OK(hipStreamSynchronize(h->stream));
     }
-    long long cur_param = static_cast<long long>(num_par_ops) - 1;
-    int tp_pos = ntp - 1;
-    // <G mu|lambda> of trainable parameter t stays on the device in dots[t]
-    // until the sweep ends: one read-back instead of a wait per parameter
-    auto *part = reinterpret_cast<double2 *>(reduce_buf(h, (kReduceBlocks + size_t(ntp)) * sizeof(double2)));
-    double2 *dots = part + kReduceBlocks;
-    std::vector<double> scale(ntp, 0.0);
+    std::vector<double> w(2 * size_t(ntp), 0.0);
     std::vector<char> reached(ntp, 0);
-    // fused steps (k_vjp_step / k_vjp_parity): one launch per op; a trainable
-    // op's block partials go to its row of vpart, all rows reduced at the end
-    const unsigned grid = std::min<unsigned>(grid_for(E.len(), 1, 8), kReduceBlocks);
-    auto *vpart = static_cast<double2 *>(buf(h, kBufVjp, size_t(ntp) * grid * sizeof(double2)));
-    std::vector<int> fused_rows;
-    for (int i = nops - 1; i >= 0; i--) {
-        if (nparams[i] > 1) {
-            throw InvalidArg("The operation is not supported using the adjoint differentiation method");
-        }
-        if (ids[i] == -1) {
-            continue;
-        }
-        if (tp_pos < 0) {
-            break;
-        }
-        const int *w = wires + woff[i];
-        const auto pt = E.params_t(params + poff[i], nparams[i]);
-        const GroupOp<T> ud = lower_gate<T>(E.n(), ids[i], w, nwires[i], inverse[i] == 0, pt.data(),
-                                            nparams[i]);
-        bool train = false;
-        int row = -1;
-        GroupOp<T> g;
-        if (nparams[i] > 0) {
-            if (cur_param == tp[tp_pos]) {
-                train = true;
-                row = tp_pos;
-                T s = 0;
-                g = lower_generator<T>(E.n(), ids[i], w, nwires[i], true, &s);
-                scale[tp_pos] = static_cast<double>(s) * (inverse[i] ? -1.0 : 1.0);
-                reached[tp_pos] = 1;
-                tp_pos--;
-            }
-            cur_param--;
-        }
-        const bool fusable = (ud.kind == GroupOp<T>::Noop && !train) ||
-                             (ud.kind == GroupOp<T>::Parity && (!train || g.same_geometry(ud))) ||
-                             (ud.kind == GroupOp<T>::Group && ud.M <= 4 && (!train || g.same_geometry(ud)));
-        if (!fusable) {
-            if (train) {
-                E.copy(mud, mu);
-                T s = 0;
-                E.apply(lower_generator<T>(E.n(), ids[i], w, nwires[i], false, &s), mud);
-                E.dot_to(mud, lam, part, dots + row);
-            }
-            E.apply(ud, lam);
-            E.apply(ud, mu);
-            continue;
-        }
-        if (ud.kind == GroupOp<T>::Noop) {
-            continue;
-        }
-        double2 *pp = train ? vpart + size_t(row) * grid : nullptr;
-        if (ud.kind == GroupOp<T>::Parity) {
-            const dcx<T> u0{ud.parity_phase[0].real(), ud.parity_phase[0].imag()};
-            const dcx<T> u1{ud.parity_phase[1].real(), ud.parity_phase[1].imag()};
-            dcx<T> g0{1, 0}, g1{1, 0};
-            if (train) {
-                g0 = {g.parity_phase[0].real(), g.parity_phase[0].imag()};
-                g1 = {g.parity_phase[1].real(), g.parity_phase[1].imag()};
-                hipLaunchKernelGGL((k_vjp_parity<T, true>), dim3(grid), dim3(kBlock), 0, h->stream, lam, mu,
-                                   E.len(), ud.parity_mask, u0, u1, g0, g1, pp);
-            } else {
-                hipLaunchKernelGGL((k_vjp_parity<T, false>), dim3(grid), dim3(kBlock), 0, h->stream, lam, mu,
-                                   E.len(), ud.parity_mask, u0, u1, g0, g1, pp);
-            }
-        } else {
-            auto go = [&](auto mtag) {
-                constexpr int M = decltype(mtag)::value;
-                AdjOp<T, M> a{};
-                a.geo.fixed = ud.fixed;
-                a.geo.nb = ud.nb;
-                for (int q = 0; q < ud.nb; q++) {
-                    a.geo.pos[q] = ud.pos[q];
-                }
-                for (int j = 0; j < M; j++) {
-                    a.off[j] = ud.off[j];
-                }
-                for (int j = 0; j < M * M; j++) {
-                    a.ud[j] = {ud.mat[j].real(), ud.mat[j].imag()};
-                    a.g[j] = train ? dcx<T>{g.mat[j].real(), g.mat[j].imag()} : dcx<T>{0, 0};
-                }
-                a.ud_diag = ud.diag ? 1 : 0;
-                const uint64_t nwork = E.len() >> ud.nb;
-                if (train) {
-                    hipLaunchKernelGGL((k_vjp_step<T, M, true>), dim3(grid), dim3(kBlock), 0, h->stream, lam, mu,
-                                       nwork, a, pp);
-                } else {
-                    hipLaunchKernelGGL((k_vjp_step<T, M, false>), dim3(grid), dim3(kBlock), 0, h->stream, lam, mu,
-                                       nwork, a, pp);
-                }
-            };
-            switch (ud.M) {
-            case 1: go(std::integral_constant<int, 1>{}); break;
-            case 2: go(std::integral_constant<int, 2>{}); break;
-            default: go(std::integral_constant<int, 4>{}); break;
-            }
-        }
-        HIP_OK(hipGetLastError());
-        if (train) {
-            fused_rows.push_back(row);
-        }
-    }
-    if (!fused_rows.empty()) {
-        const auto *drows = static_cast<const int *>(stage(h, fused_rows.data(), fused_rows.size() * sizeof(int)));
-        hipLaunchKernelGGL(k_vjp_final, dim3(static_cast<unsigned>(fused_rows.size())), dim3(kBlock), 0, h->stream,
-                           vpart, static_cast<int>(grid), drows, dots);
-        HIP_OK(hipGetLastError());
-    }
-    std::vector<double2> z(ntp);
-    HIP_OK(hipMemcpyAsync(z.data(), dots, ntp * sizeof(double2), hipMemcpyDeviceToHost, h->stream));
+    backward_sweep<T, true>(E, t, lam, {mu}, ntp, tp, [&](int row, int, std::complex<double> z, double scale) {
+        w[2 * row] -= scale * z.imag();
+        w[2 * row + 1] += scale * z.real();
+        reached[row] = 1;
+    });
     HIP_OK(hipStreamSynchronize(h->stream));
-    for (int t = 0; t < ntp; t++) {
-        if (reached[t]) {
-            out[2 * t] = -scale[t] * z[t].y;
-            out[2 * t + 1] = scale[t] * z[t].x;
+    for (int i = 0; i < ntp; i++) {
+        if (reached[i]) {
+            out[2 * i] = w[2 * i];
+            out[2 * i + 1] = w[2 * i + 1];
         }
     }
 }
@@ -2384,8 +2221,8 @@ int pl_adjoint_jacobian(pl_sv_t h, int nops, const int *ids, const int *nwires, 
                         const int *prog, const double *coeffs, const double *mats, int ntp,
                         const int *tp, double *jac) {
     return dispatch(h, [&](auto &E) {
-        adjoint_sweep(E, nops, ids, nwires, wires, inverse, nparams, params, prog, coeffs, mats,
-                      ntp, tp, jac);
+        adjoint_sweep(E, SweepTape{nops, ids, nwires, wires, inverse, nparams, params}, prog, coeffs, mats, ntp,
+                      tp, jac);
     });
 }
 
@@ -2396,7 +2233,7 @@ int pl_vjp(pl_sv_t h, int nops, const int *ids, const int *nwires, const int *wi
         if (!dy || (ntp > 0 && (!tp || !vjp)) || nops < 0) {
             throw InvalidArg("null argument");
         }
-        vjp_sweep(E, nops, ids, nwires, wires, inverse, nparams, params, dy, ntp, tp, vjp);
+        vjp_sweep(E, SweepTape{nops, ids, nwires, wires, inverse, nparams, params}, dy, ntp, tp, vjp);
     });
 }
 

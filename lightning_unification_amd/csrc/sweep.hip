@@ -1,0 +1,43 @@
+// The backward sweep's pass kernel, one translation unit per precision
+// (PL_SWEEP_DOUBLE), compiled like the tile passes with uniform regions left
+// unstructured: a step's branches are all on scalars, and structuring them
+// makes the compiler copy the register tile at every join.
+#include "kernels_adjoint.hpp"
+
+namespace plamd {
+
+template <class T> hipError_t launch_sweep(int waves, int kh, bool full, const SweepArgs<T> &a, hipStream_t s) {
+    auto go = [&](auto nw, auto k, auto f) {
+        constexpr int NW = decltype(nw)::value, KH = decltype(k)::value;
+        constexpr bool FULL = decltype(f)::value != 0;
+        constexpr size_t tile = sizeof(double2) << (6 + kSweepRegBits + (NW == 4 ? 2 : NW == 2 ? 1 : 0));
+        const size_t lds = tile + size_t(a.nslots) * NW * KH * (FULL ? kSweepFull : kSweepReal) * sizeof(double);
+        hipLaunchKernelGGL((k_sweep<T, NW, KH, FULL>), dim3(static_cast<unsigned>(a.W * a.ngrp)), dim3(64 * NW), lds,
+                           s, a, a.prog);
+        return hipGetLastError();
+    };
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
+    using I4 = std::integral_constant<int, 4>;
+    using I0 = std::integral_constant<int, 0>;
+    if (full) { // one state is swept with lambda
+        return waves == 4 ? go(I4{}, I1{}, I1{}) : waves == 2 ? go(I2{}, I1{}, I1{}) : go(I1{}, I1{}, I1{});
+    }
+    if (kh == 2) {
+        return waves == 4 ? go(I4{}, I2{}, I0{}) : waves == 2 ? go(I2{}, I2{}, I0{}) : go(I1{}, I2{}, I0{});
+    }
+    return waves == 4 ? go(I4{}, I1{}, I0{}) : waves == 2 ? go(I2{}, I1{}, I0{}) : go(I1{}, I1{}, I0{});
+}
+
+#if PL_SWEEP_DOUBLE
+template hipError_t launch_sweep<double>(int, int, bool, const SweepArgs<double> &, hipStream_t);
+
+hipError_t launch_sweep_sums(const double *partial, int W, unsigned count, double *out, hipStream_t s) {
+    hipLaunchKernelGGL(k_sweep_sums, dim3(count), dim3(64), 0, s, partial, W, out);
+    return hipGetLastError();
+}
+#else
+template hipError_t launch_sweep<float>(int, int, bool, const SweepArgs<float> &, hipStream_t);
+#endif
+
+} // namespace plamd

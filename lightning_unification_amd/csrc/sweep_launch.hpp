@@ -1,0 +1,73 @@
+// Data of the backward sweep's passes and the launch of one
+// (kernels_adjoint.hpp; the kernel is compiled in its own translation units,
+// sweep.hip).
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "kernels_gate.hpp"
+
+namespace plamd {
+
+enum SweepKind : int {
+    kSweepWindow = 0, // other local bits become register bits
+    kSweepDense,      // a 2x2 on register bit j
+    kSweepFlip,       // an X on register bit j (CNOT, Toffoli)
+    kSweepDiag,       // phase u[0] or u[1] by the parity of masked bits
+};
+
+// One step on a tile whose local index is split into register bits (the
+// window) and thread bits (the others, ascending).  It acts where all tested
+// bits have their values: (register index & rm) == rv, (thread & lm) == lv and
+// (bits outside the tile & omask) == oval.  kSweepDiag: the phase is u[parity
+// of register & rp, thread & lp and outside & op].  kSweepWindow: rp holds the
+// new window's positions, four bits each.
+struct SweepStep {
+    int kind;
+    int j;
+    uint32_t rm, rv, lm, lv, rp, lp;
+    int slot; // accumulation slot of the pass, -1: not trainable
+    int pad;
+    uint64_t omask, oval, op;
+    dcx<double> u[4];
+};
+
+// Sums kept per slot and observable, of M_ab = sum conj(h_a) lambda_b over the
+// step's pairs (kSweepDiag: a = b = the parity):
+//   0 Im M00, 1 Im M11, 2 Im(M01 + M10), 3 Re(M01 - M10)
+// and for the complex form also
+//   4 Re M00, 5 Re M11, 6 Re(M01 + M10), 7 Im(M01 - M10).
+constexpr int kSweepReal = 4, kSweepFull = 8;
+constexpr int kSweepSlots = 64;    // trainable steps per pass
+constexpr int kSweepMaxBits = 11;  // widest tile
+
+constexpr int kSweepRegBits = 3;   // register bits of a tile: 8 amplitudes a thread and state
+
+struct SweepGeom {
+    int bits;              // local bits of the state: min(n, the tile's)
+    int low;               // the lowest `low` bit positions are local bits 0 .. low - 1
+    int hb[kSweepMaxBits]; // positions of local bits low .., ascending
+};
+
+// States are held in T and swept in double: a pass of complex64 states rounds
+// each amplitude once, where its steps would round it once each.
+template <class T> struct SweepArgs {
+    const v2<T> *lam_in;
+    v2<T> *lam_out;
+    v2<T> *const *hs;
+    int K, grp0, ngrp, writer, W;
+    uint64_t ntiles;
+    SweepGeom geo;
+    const SweepStep *prog;
+    int nsteps, nslots, slot0;
+    double *partial;
+};
+
+// One launch of args.ngrp observable groups (kh observables each) with `waves`
+// (1, 2 or 4) wavefronts per tile; full: the complex sums too.
+template <class T> hipError_t launch_sweep(int waves, int kh, bool full, const SweepArgs<T> &args, hipStream_t s);
+// out[v] = sum of partial[v W .. (v + 1) W), v < count
+hipError_t launch_sweep_sums(const double *partial, int W, unsigned count, double *out, hipStream_t s);
+
+} // namespace plamd

@@ -273,11 +273,7 @@ GroupOp<T> tile_group(int n, const TapeView &t, int i, int woff, int poff, int l
         }
         lw[a] = k - 1 - m;
     }
-    std::vector<T> prm(t.nparams[i]);
-    for (int a = 0; a < t.nparams[i]; a++) {
-        prm[a] = static_cast<T>(t.params[poff + a]);
-    }
-    return lower_gate<T>(k, t.ids[i], lw.data(), t.nwires[i], t.inverse[i] != 0, prm.data(), t.nparams[i]);
+    return lower_gate_as<T>(k, t.ids[i], lw.data(), t.nwires[i], t.inverse[i] != 0, t.params + poff, t.nparams[i]);
 }
 
 template <class T> TpOp<T> tile_lds_op(const GroupOp<T> &g) {
