@@ -99,6 +99,7 @@ template <class T> struct BatchPlan final : BatchPlanBase {
     uint64_t *dxm = nullptr;
     double *dparams = nullptr, *dgrads = nullptr, *denergy = nullptr;
     double2 *dcs = nullptr; // (cos, sin) of every half angle, refreshed each replay
+    BMat *dmats = nullptr;  // every wire's 2x2 per layer, refreshed each replay
     int *dcirc_lists = nullptr;
     uint64_t *dprefix = nullptr;
     std::vector<LaunchSpec> seq;
@@ -164,6 +165,7 @@ template <class T> struct BatchPlan final : BatchPlanBase {
         HIP_OK(hipMalloc(&dparams, std::max<uint64_t>(npar, 1) * sizeof(double)));
         HIP_OK(hipMalloc(&dgrads, std::max<uint64_t>(npar, 1) * sizeof(double)));
         HIP_OK(hipMalloc(&dcs, std::max<uint64_t>(npar, 1) * sizeof(double2)));
+        HIP_OK(hipMalloc(&dmats, std::max<uint64_t>(npar / npat, 1) * sizeof(BMat)));
         HIP_OK(hipMalloc(&denergy, 2 * std::max(nc, 1) * sizeof(double))); // energies, then <psi|psi>
         if (!terms.empty()) {
             HIP_OK(hipMemcpy(dterms, terms.data(), terms.size() * sizeof(PauliTerm), hipMemcpyHostToDevice));
@@ -186,7 +188,7 @@ template <class T> struct BatchPlan final : BatchPlanBase {
         for (void *p : {static_cast<void *>(arena), static_cast<void *>(dcircs),
                         static_cast<void *>(dterms), static_cast<void *>(dxm),
                         static_cast<void *>(dparams), static_cast<void *>(dgrads), static_cast<void *>(dcs),
-                        static_cast<void *>(denergy), static_cast<void *>(dcirc_lists),
+                        static_cast<void *>(dmats), static_cast<void *>(denergy), static_cast<void *>(dcirc_lists),
                         static_cast<void *>(dprefix)}) {
             if (p) {
                 (void)hipFree(p);
@@ -269,7 +271,7 @@ template <class T> struct BatchPlan final : BatchPlanBase {
                 }
             }
             prefixes.push_back(tot);
-            if (tot * kBlock > 0xFFFFFFFFull) { // work-items per launch dimension
+            if (tot * std::max(kBlock, 64 << std::max(0, w - 9)) > 0xFFFFFFFFull) { // work-items per launch dimension
                 throw InvalidArg("batch too large for tile width " + std::to_string(w) +
                                  ": one launch would exceed 2^32 work-items");
             }
@@ -331,14 +333,32 @@ template <class T> struct BatchPlan final : BatchPlanBase {
         capture();
     }
 
+    // One rotation stage: 2^(W - 9) wavefronts a workgroup (one below 9 bits),
+    // three register bits a thread.
+    template <bool ADJ> void stage(const LaunchSpec &ls, int lb, int hb, int gl, int gh) {
+        auto go = [&](auto nw) {
+            constexpr int NW = decltype(nw)::value;
+            const size_t lds = sizeof(double2) * 8 * 64 * NW;
+            hipLaunchKernelGGL((k_batch_stage<T, NW, ADJ>), dim3(static_cast<unsigned>(ls.blocks)), dim3(64 * NW), lds,
+                               stream, arena, dcircs, ls.L, W, ls.stage, ls.layer, lb, hb, gl, gh, npat, pat, dmats,
+                               dcs, dgrads);
+        };
+        switch (W) {
+        case 13: go(std::integral_constant<int, 16>{}); break;
+        case 12: go(std::integral_constant<int, 8>{}); break;
+        case 11: go(std::integral_constant<int, 4>{}); break;
+        case 10: go(std::integral_constant<int, 2>{}); break;
+        default: go(std::integral_constant<int, 1>{}); break;
+        }
+    }
+
     void enqueue() {
-        const size_t tile_bytes = (size_t{1} << W) * sizeof(V);
         hipLaunchKernelGGL(k_zero, dim3((npar + kBlock - 1) / kBlock + 1), dim3(kBlock), 0, stream,
                            dgrads, npar);
         hipLaunchKernelGGL(k_zero, dim3((2 * nc + kBlock - 1) / kBlock + 1), dim3(kBlock), 0, stream,
                            denergy, static_cast<uint64_t>(2 * nc));
-        hipLaunchKernelGGL(k_batch_trig, dim3((npar + kBlock - 1) / kBlock + 1), dim3(kBlock), 0, stream,
-                           dparams, npar, dcs);
+        hipLaunchKernelGGL(k_batch_mats, dim3((npar / npat + kBlock - 1) / kBlock + 1), dim3(kBlock), 0, stream,
+                           dparams, npar / npat, npat, pat, dcs, dmats);
         for (const auto &ls : seq) {
             const dim3 grid(static_cast<unsigned>(ls.blocks));
             const int cur = entangler ? (ls.layer & 1) : 0;
@@ -350,8 +370,7 @@ template <class T> struct BatchPlan final : BatchPlanBase {
             case LaunchSpec::Rot: {
                 // stage 0 of layer l >= 1 gathers through layer l-1's entangler
                 const int gsrc = (entangler && ls.layer > 0 && ls.stage == 0) ? nxt : -1;
-                hipLaunchKernelGGL((k_batch_rot<T>), grid, dim3(kBlock), tile_bytes, stream, arena,
-                                   dcircs, ls.L, W, ls.stage, ls.layer, cur, gsrc, npat, pat, dcs);
+                stage<false>(ls, cur, -1, gsrc, -1);
                 break;
             }
             case LaunchSpec::Ring:
@@ -366,9 +385,7 @@ template <class T> struct BatchPlan final : BatchPlanBase {
             case LaunchSpec::RotAdj:
                 // lambda and H of layer l+1's side (buffers nxt) are gathered
                 // through the inverse entangler at each circuit's first stage
-                hipLaunchKernelGGL((k_batch_rot_adj<T>), grid, dim3(kBlock), 2 * tile_bytes, stream,
-                                   arena, dcircs, ls.L, W, ls.stage, ls.layer, cur, 2 + cur,
-                                   entangler ? nxt : -1, entangler ? 2 + nxt : -1, npat, pat, dcs, dgrads);
+                stage<true>(ls, cur, 2 + cur, entangler ? nxt : -1, entangler ? 2 + nxt : -1);
                 break;
             }
             const hipError_t err = hipGetLastError();

@@ -30,130 +30,10 @@
 #include <stdint.h>
 
 #include "kernels_reduce.hpp"
+#include "reg_tile.hpp"
 #include "sweep_launch.hpp"
 
 namespace plamd {
-
-// Sums of a and b over lanes l and l ^ 32: a's in the lower half, b's in the upper.
-__device__ __forceinline__ double sweep_fold32(double a, double b) {
-    const auto ua = static_cast<unsigned long long>(__double_as_longlong(a));
-    const auto ub = static_cast<unsigned long long>(__double_as_longlong(b));
-    const auto lo = __builtin_amdgcn_permlane32_swap(static_cast<unsigned>(ua), static_cast<unsigned>(ub), false, false);
-    const auto hi = __builtin_amdgcn_permlane32_swap(static_cast<unsigned>(ua >> 32), static_cast<unsigned>(ub >> 32),
-                                                     false, false);
-    const double x = __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi[0]) << 32) | lo[0]));
-    const double y = __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi[1]) << 32) | lo[1]));
-    return x + y;
-}
-// Sums of a and b over lanes l and l ^ 16: a's in even rows of 16 lanes, b's in odd ones.
-__device__ __forceinline__ double sweep_fold16(double a, double b) {
-    const auto ua = static_cast<unsigned long long>(__double_as_longlong(a));
-    const auto ub = static_cast<unsigned long long>(__double_as_longlong(b));
-    const auto lo = __builtin_amdgcn_permlane16_swap(static_cast<unsigned>(ua), static_cast<unsigned>(ub), false, false);
-    const auto hi = __builtin_amdgcn_permlane16_swap(static_cast<unsigned>(ua >> 32), static_cast<unsigned>(ub >> 32),
-                                                     false, false);
-    const double x = __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi[0]) << 32) | lo[0]));
-    const double y = __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi[1]) << 32) | lo[1]));
-    return x + y;
-}
-template <int CTRL> __device__ __forceinline__ double sweep_dpp(double v) {
-    const auto u = static_cast<unsigned long long>(__double_as_longlong(v));
-    const unsigned lo = static_cast<unsigned>(__builtin_amdgcn_mov_dpp(static_cast<int>(static_cast<unsigned>(u)), CTRL, 0xf, 0xf, true));
-    const unsigned hi = static_cast<unsigned>(__builtin_amdgcn_mov_dpp(static_cast<int>(static_cast<unsigned>(u >> 32)), CTRL, 0xf, 0xf, true));
-    return __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi) << 32) | lo));
-}
-// Totals of four values over the wavefront: row r of 16 lanes (lane / 16 = r)
-// ends with the total of v[sweep_row(r)].
-__device__ __forceinline__ double sweep_sum4(double v0, double v1, double v2, double v3) {
-    // rows 0..3 after the folds: v0, v2, v1, v3
-    double s = sweep_fold16(sweep_fold32(v0, v1), sweep_fold32(v2, v3));
-    s += sweep_dpp<0x128>(s); // rotations within a row by 8, 4, 2, 1
-    s += sweep_dpp<0x124>(s);
-    s += sweep_dpp<0x122>(s);
-    s += sweep_dpp<0x121>(s);
-    return s;
-}
-__device__ __forceinline__ int sweep_row(int r) { return ((r & 1) << 1) | (r >> 1); }
-
-// Local index -> place in the LDS buffer, linear in its bits.  With a window
-// bit among the lowest, neighbouring lanes hold every other amplitude of 128
-// bytes; flipping the bits inside 128 bytes where the next bit is set spreads
-// them over all banks again.
-__device__ __forceinline__ uint32_t sweep_place(uint32_t e) {
-    constexpr int b = 4; // 16 doubles
-    return e ^ (((e >> b) & 1U) * ((1U << b) - 1));
-}
-
-// thread bits spread over the local bits outside the window
-template <int RB> __device__ __forceinline__ uint32_t sweep_thread_part(uint32_t t, uint32_t win) {
-#pragma unroll
-    for (int j = 0; j < RB; j++) {
-        const uint32_t m = (1U << ((win >> (4 * j)) & 15U)) - 1;
-        t = ((t & ~m) << 1) | (t & m);
-    }
-    return t;
-}
-template <int RB> __device__ __forceinline__ uint32_t sweep_reg_part(int r, uint32_t win) {
-    uint32_t e = 0;
-#pragma unroll
-    for (int j = 0; j < RB; j++) {
-        e |= ((r >> j) & 1) ? 1U << ((win >> (4 * j)) & 15U) : 0U;
-    }
-    return e;
-}
-
-__device__ __forceinline__ double sweep_fma(double a, double b, double c) { return __builtin_fma(a, b, c); }
-
-// Updates of the register tile.  The last multiply-add of every amplitude
-// writes the amplitude's own register, in the lanes of `m` only; the lane
-// condition is an execution mask inside the block, so a step has no divergent
-// branch.  Left to the compiler (branches on the condition, results in
-// registers of their own), every step's results were copied back where the
-// steps' branches join: 241 registers and two wavefronts a SIMD for KH = 2 in
-// complex128, a third of the instructions moves.  All 64 lanes are active
-// around every block.
-__device__ __forceinline__ void sweep_into(uint64_t m, double2 &a, double u, double tx, double ty) {
-    asm("s_mov_b64 exec, %2\n\t"
-        "v_fma_f64 %0, %3, %0, %4\n\t"
-        "v_fma_f64 %1, %3, %1, %5\n\t"
-        "s_mov_b64 exec, -1"
-        : "+v"(a.x), "+v"(a.y)
-        : "s"(m), "v"(u), "v"(tx), "v"(ty));
-}
-__device__ __forceinline__ void sweep_into2(uint64_t m, double2 &a, double2 &b, double ua, double ub, double t0,
-                                            double t1, double t2, double t3) {
-    asm("s_mov_b64 exec, %4\n\t"
-        "v_fma_f64 %0, %5, %0, %7\n\t"
-        "v_fma_f64 %1, %5, %1, %8\n\t"
-        "v_fma_f64 %2, %6, %2, %9\n\t"
-        "v_fma_f64 %3, %6, %3, %10\n\t"
-        "s_mov_b64 exec, -1"
-        : "+v"(a.x), "+v"(a.y), "+v"(b.x), "+v"(b.y)
-        : "s"(m), "s"(ua), "s"(ub), "v"(t0), "v"(t1), "v"(t2), "v"(t3));
-}
-// a <-> b in the lanes of m
-__device__ __forceinline__ void sweep_exchange(uint64_t m, double2 &a, double2 &b) {
-    double t;
-    asm("s_mov_b64 exec, %5\n\t"
-        "v_mov_b64 %4, %0\n\t"
-        "v_mov_b64 %0, %2\n\t"
-        "v_mov_b64 %2, %4\n\t"
-        "v_mov_b64 %4, %1\n\t"
-        "v_mov_b64 %1, %3\n\t"
-        "v_mov_b64 %3, %4\n\t"
-        "s_mov_b64 exec, -1"
-        : "+v"(a.x), "+v"(a.y), "+v"(b.x), "+v"(b.y), "=&v"(t)
-        : "s"(m));
-}
-
-// (a, b) <- u (a, b) in the lanes of m, 16 multiply-adds
-__device__ __forceinline__ void sweep_apply2(uint64_t m, const dcx<double> *u, double2 &a, double2 &b) {
-    const double t0 = sweep_fma(-u[0].i, a.y, sweep_fma(u[1].r, b.x, -u[1].i * b.y));
-    const double t1 = sweep_fma(u[0].i, a.x, sweep_fma(u[1].r, b.y, u[1].i * b.x));
-    const double t2 = sweep_fma(-u[3].i, b.y, sweep_fma(u[2].r, a.x, -u[2].i * a.y));
-    const double t3 = sweep_fma(u[3].i, b.x, sweep_fma(u[2].r, a.y, u[2].i * a.x));
-    sweep_into2(m, a, b, u[0].r, u[3].r, t0, t1, t2, t3);
-}
 
 // Workgroups are numbered (tile walker w, observable group grp), groups of one
 // walker on one XCD where the grid allows it, since they read the same lambda
@@ -175,9 +55,6 @@ __global__ __launch_bounds__(64 * NW, 4) void k_sweep(const SweepArgs<T> A, cons
         return v;
     }();
     extern __shared__ unsigned char smem_raw[];
-    // real parts, then imaginary parts: a 16-byte element would tie the two
-    // registers of an amplitude into one tuple, which the in-place updates
-    // would have to copy out of and back into
     double *tile = reinterpret_cast<double *>(smem_raw);
     constexpr uint32_t IM = 1U << (TB + RB);
     double *sums = reinterpret_cast<double *>(tile + 2 * IM); // [wave][slot][KH][NC]
@@ -241,25 +118,7 @@ __global__ __launch_bounds__(64 * NW, 4) void k_sweep(const SweepArgs<T> A, cons
         }
         uint32_t win = HOME;
         auto window = [&](uint32_t to) {
-            const uint32_t tf = sweep_place(sweep_thread_part<RB>(tid, win));
-            const uint32_t tt = sweep_place(sweep_thread_part<RB>(tid, to));
-#pragma unroll
-            for (int i = 0; i < S; i++) {
-                __syncthreads();
-#pragma unroll
-                for (int r = 0; r < R; r++) {
-                    const uint32_t p = tf ^ sweep_place(sweep_reg_part<RB>(r, win));
-                    tile[p] = x[i][r].x;
-                    tile[p + IM] = x[i][r].y;
-                }
-                __syncthreads();
-#pragma unroll
-                for (int r = 0; r < R; r++) {
-                    const uint32_t p = tt ^ sweep_place(sweep_reg_part<RB>(r, to));
-                    x[i][r].x = tile[p];
-                    x[i][r].y = tile[p + IM];
-                }
-            }
+            rt_window<TB, RB>(x, tile, tid, win, to);
             win = to;
         };
         for (int s = 0; s < A.nsteps; s++) {
@@ -303,15 +162,15 @@ __global__ __launch_bounds__(64 * NW, 4) void k_sweep(const SweepArgs<T> A, cons
                             const double cx = x[1 + kk][i0].x, cy = x[1 + kk][i0].y, dx = x[1 + kk][i1].x,
                                          dy = x[1 + kk][i1].y;
                             double *t = acc[kk];
-                            t[0] = sweep_fma(cx, ay, sweep_fma(-cy, ax, t[0]));
-                            t[1] = sweep_fma(dx, by, sweep_fma(-dy, bx, t[1]));
-                            t[2] = sweep_fma(cx, by, sweep_fma(-cy, bx, sweep_fma(dx, ay, sweep_fma(-dy, ax, t[2]))));
-                            t[3] = sweep_fma(cx, bx, sweep_fma(cy, by, sweep_fma(-dx, ax, sweep_fma(-dy, ay, t[3]))));
+                            t[0] = rt_fma(cx, ay, rt_fma(-cy, ax, t[0]));
+                            t[1] = rt_fma(dx, by, rt_fma(-dy, bx, t[1]));
+                            t[2] = rt_fma(cx, by, rt_fma(-cy, bx, rt_fma(dx, ay, rt_fma(-dy, ax, t[2]))));
+                            t[3] = rt_fma(cx, bx, rt_fma(cy, by, rt_fma(-dx, ax, rt_fma(-dy, ay, t[3]))));
                             if constexpr (FULL) {
-                                t[4] = sweep_fma(cx, ax, sweep_fma(cy, ay, t[4]));
-                                t[5] = sweep_fma(dx, bx, sweep_fma(dy, by, t[5]));
-                                t[6] = sweep_fma(cx, bx, sweep_fma(cy, by, sweep_fma(dx, ax, sweep_fma(dy, ay, t[6]))));
-                                t[7] = sweep_fma(cx, by, sweep_fma(-cy, bx, sweep_fma(-dx, ay, sweep_fma(dy, ax, t[7]))));
+                                t[4] = rt_fma(cx, ax, rt_fma(cy, ay, t[4]));
+                                t[5] = rt_fma(dx, bx, rt_fma(dy, by, t[5]));
+                                t[6] = rt_fma(cx, bx, rt_fma(cy, by, rt_fma(dx, ax, rt_fma(dy, ay, t[6]))));
+                                t[7] = rt_fma(cx, by, rt_fma(-cy, bx, rt_fma(-dx, ay, rt_fma(dy, ax, t[7]))));
                             }
                         }
                     }
@@ -327,11 +186,11 @@ __global__ __launch_bounds__(64 * NW, 4) void k_sweep(const SweepArgs<T> A, cons
 #pragma unroll
                         for (int kk = 0; kk < KH; kk++) {
                             const double cx = x[1 + kk][r].x, cy = x[1 + kk][r].y;
-                            const double im = sweep_fma(cx, ay, -cy * ax);
+                            const double im = rt_fma(cx, ay, -cy * ax);
                             acc[kk][0] += im;
                             acc[kk][1] += odd ? -im : im;
                             if constexpr (FULL) {
-                                const double re = sweep_fma(cx, ax, cy * ay);
+                                const double re = rt_fma(cx, ax, cy * ay);
                                 acc[kk][4] += re;
                                 acc[kk][5] += odd ? -re : re;
                             }
@@ -357,10 +216,10 @@ __global__ __launch_bounds__(64 * NW, 4) void k_sweep(const SweepArgs<T> A, cons
                 for (int kk = 0; kk < KH; kk++) {
 #pragma unroll
                     for (int c = 0; c < NC; c += 4) {
-                        const double t = sweep_sum4(on ? acc[kk][c] : 0.0, on ? acc[kk][c + 1] : 0.0,
+                        const double t = rt_sum4(on ? acc[kk][c] : 0.0, on ? acc[kk][c + 1] : 0.0,
                                                     on ? acc[kk][c + 2] : 0.0, on ? acc[kk][c + 3] : 0.0);
                         if ((lane & 15) == 0) {
-                            mine[(slot * KH + kk) * NC + c + sweep_row(lane >> 4)] += t;
+                            mine[(slot * KH + kk) * NC + c + rt_row(lane >> 4)] += t;
                         }
                     }
                 }
@@ -379,7 +238,7 @@ __global__ __launch_bounds__(64 * NW, 4) void k_sweep(const SweepArgs<T> A, cons
                         if ((static_cast<uint32_t>(i0) & rm) == rv) {
 #pragma unroll
                             for (int i = 0; i < S; i++) {
-                                sweep_apply2(lanes, u, x[i][i0], x[i][i1]);
+                                rt_apply2(lanes, u, x[i][i0], x[i][i1]);
                             }
                         }
                     }
@@ -398,7 +257,7 @@ __global__ __launch_bounds__(64 * NW, 4) void k_sweep(const SweepArgs<T> A, cons
                         if ((static_cast<uint32_t>(i0) & rm) == rv) {
 #pragma unroll
                             for (int i = 0; i < S; i++) {
-                                sweep_exchange(lanes, x[i][i0], x[i][i1]);
+                                rt_exchange(lanes, x[i][i0], x[i][i1]);
                             }
                         }
                     }
@@ -419,7 +278,7 @@ __global__ __launch_bounds__(64 * NW, 4) void k_sweep(const SweepArgs<T> A, cons
                         const dcx<double> u{odd ? uo.r : ue.r, odd ? uo.i : ue.i};
 #pragma unroll
                         for (int i = 0; i < S; i++) {
-                            sweep_into(lanes, x[i][r], u.r, -u.i * x[i][r].y, u.i * x[i][r].x);
+                            rt_into(lanes, x[i][r], u.r, -u.i * x[i][r].y, u.i * x[i][r].x);
                         }
                     }
                 }

@@ -9,18 +9,20 @@
 //
 // Every launch covers all circuits that still have work at that step; block
 // b finds its circuit by bisection in a per-launch prefix table.  Rotations
-// run on LDS tiles: a tile holds 2^T amplitudes spanning T bit positions (the
-// 3 lowest bits -- one 128-byte line -- plus up to W-3 target bits), so one
-// HBM pass applies the rotations of up to W wires.  The entangler is one
-// GF(2)-linear gather pass (out[y] = in[src(y)], src bits are parities of y).
-// The adjoint keeps lambda and H_lambda tiles in LDS and accumulates
-// Im<H|G lambda> for every angle of the tile before undoing its rotation.
+// run on register tiles (reg_tile.hpp): a tile holds 2^T amplitudes spanning T
+// bit positions (the 3 lowest bits -- one 128-byte line -- plus up to W-3
+// target bits), so one HBM pass applies the rotations of up to W wires.  The
+// entangler is one GF(2)-linear gather (out[y] = in[src(y)], src bits are
+// parities of y).  The adjoint holds tiles of lambda and H_lambda.
 #pragma once
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "kernels_reduce.hpp"
+#include "reg_tile.hpp"
 
 namespace plamd {
 
@@ -46,16 +48,20 @@ struct BLaunch {
     int count;
 };
 
+// The circuit of block b and the block's place in it: each wavefront narrows
+// the prefix table 64-fold a load (bisection's ten dependent loads took longer
+// than a small tile's rotations).
 __device__ __forceinline__ int find_circ(const BLaunch &L, uint64_t b, uint64_t &local) {
-    int lo = 0, hi = L.count - 1; // largest c with prefix[c] <= b
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (L.prefix[mid] <= b) {
-            lo = mid;
-        } else {
-            hi = mid - 1;
-        }
+    const int lane = threadIdx.x & 63;
+    int lo = 0, n = L.count; // the largest c with prefix[c] <= b lies in [lo, lo + n)
+    while (n > 1) {
+        const int step = (n + 63) / 64, at = lane * step;
+        const uint64_t below = __ballot(at < n && L.prefix[lo + (at < n ? at : 0)] <= b);
+        const int k = __popcll(below) - 1; // prefix[lo] <= b always
+        lo += k * step;
+        n = n - k * step < step ? n - k * step : step;
     }
+    lo = __builtin_amdgcn_readfirstlane(lo);
     local = b - L.prefix[lo];
     return L.circ[lo];
 }
@@ -90,92 +96,50 @@ __device__ __forceinline__ int stage_bits(int n, int W, int s, int *bits, int &a
     return T;
 }
 
-template <class T> struct Rot2 {
-    dcx<T> m[4];
+// The 2x2 of one wire's rotations in one layer.
+struct BMat {
+    dcx<double> u[4];
 };
 
-// exp(-i theta/2 sigma_axis), axis 0 = X, 1 = Y, 2 = Z  (LM.hpp:541-615
-// matrices), from cs = (cos(theta/2), sin(theta/2)); dagger negates sin.
-template <class T> __device__ __forceinline__ Rot2<T> rot_matrix(int axis, double2 cs, bool dagger) {
-    const double c = cs.x, s = dagger ? -cs.y : cs.y;
-    Rot2<T> r;
-    if (axis == 0) {
-        r.m[0] = {T(c), T(0)};
-        r.m[1] = {T(0), T(-s)};
-        r.m[2] = {T(0), T(-s)};
-        r.m[3] = {T(c), T(0)};
-    } else if (axis == 1) {
-        r.m[0] = {T(c), T(0)};
-        r.m[1] = {T(-s), T(0)};
-        r.m[2] = {T(s), T(0)};
-        r.m[3] = {T(c), T(0)};
-    } else {
-        r.m[0] = {T(c), T(-s)};
-        r.m[1] = {T(0), T(0)};
-        r.m[2] = {T(0), T(0)};
-        r.m[3] = {T(c), T(s)};
-    }
-    return r;
-}
-
-// cs[i] = (cos(theta_i / 2), sin(theta_i / 2)) for every angle of the batch,
-// once per replay, so the rotation kernels do no transcendental math
-__global__ __launch_bounds__(kBlock) void k_batch_trig(const double *__restrict__ params, uint64_t n,
-                                                      double2 *__restrict__ cs) {
+// Per (circuit, layer, wire), once per replay: (cos, sin) of every half angle
+// and the product of the pattern's rotations, U = R_{npat-1} .. R_0 with
+// R = exp(-i theta/2 sigma_axis) (LM.hpp:541-615), so the stages do no
+// transcendental math and one 2x2 product per wire.
+__global__ __launch_bounds__(kBlock) void k_batch_mats(const double *__restrict__ params, uint64_t nwires, int npat,
+                                                      int4 pat, double2 *__restrict__ cs, BMat *__restrict__ mats) {
     const uint64_t i = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x;
-    if (i < n) {
+    if (i >= nwires) {
+        return;
+    }
+    const int axes[4] = {pat.x, pat.y, pat.z, pat.w};
+    BMat m;
+    m.u[0] = m.u[3] = {1, 0};
+    m.u[1] = m.u[2] = {0, 0};
+    for (int a = 0; a < npat; a++) {
         double s, c;
-        sincos(0.5 * params[i], &s, &c);
-        cs[i] = double2{c, s};
-    }
-}
-
-template <class T> __device__ __forceinline__ Rot2<T> mat2_mul(const Rot2<T> &a, const Rot2<T> &b) {
-    Rot2<T> r;
-    for (int i = 0; i < 2; i++) {
-        for (int j = 0; j < 2; j++) {
-            const dcx<T> x = a.m[2 * i], y = b.m[j], u = a.m[2 * i + 1], v = b.m[2 + j];
-            r.m[2 * i + j] = {x.r * y.r - x.i * y.i + u.r * v.r - u.i * v.i,
-                              x.r * y.i + x.i * y.r + u.r * v.i + u.i * v.r};
+        sincos(0.5 * params[i * npat + a], &s, &c);
+        cs[i * npat + a] = double2{c, s};
+        dcx<double> r[4] = {{c, 0}, {0, 0}, {0, 0}, {c, 0}};
+        if (axes[a] == 0) {
+            r[1] = r[2] = {0, -s};
+        } else if (axes[a] == 1) {
+            r[1] = {-s, 0};
+            r[2] = {s, 0};
+        } else {
+            r[0].i = -s;
+            r[3].i = s;
         }
+        BMat p;
+        for (int j = 0; j < 2; j++) {
+            for (int k = 0; k < 2; k++) {
+                const dcx<double> x = r[2 * j], y = m.u[k], u = r[2 * j + 1], v = m.u[2 + k];
+                p.u[2 * j + k] = {x.r * y.r - x.i * y.i + u.r * v.r - u.i * v.i,
+                                  x.r * y.i + x.i * y.r + u.r * v.i + u.i * v.r};
+            }
+        }
+        m = p;
     }
-    return r;
-}
-template <class T>
-__device__ __forceinline__ void apply2(const Rot2<T> &r, v2<T> &a, v2<T> &b) {
-    v2<T> x = cmul(r.m[0], a);
-    cfma(x, r.m[1], b);
-    v2<T> y = cmul(r.m[2], a);
-    cfma(y, r.m[3], b);
-    a = x;
-    b = y;
-}
-
-// (a, b) <- R_axis^(dagger?)(theta) (a, b) using the structure of each Pauli
-// rotation (RX symmetric with imaginary off-diagonal, RY real, RZ diagonal):
-// about half the arithmetic of a general 2x2 complex product.
-template <class T>
-__device__ __forceinline__ void rot_apply(int axis, double2 cs, bool dagger, v2<T> &a, v2<T> &b) {
-    const T c = T(cs.x), s = dagger ? T(-cs.y) : T(cs.y);
-    v2<T> x, y;
-    if (axis == 0) { // [[c, -i s], [-i s, c]]
-        x.x = c * a.x + s * b.y;
-        x.y = c * a.y - s * b.x;
-        y.x = s * a.y + c * b.x;
-        y.y = c * b.y - s * a.x;
-    } else if (axis == 1) { // [[c, -s], [s, c]]
-        x.x = c * a.x - s * b.x;
-        x.y = c * a.y - s * b.y;
-        y.x = s * a.x + c * b.x;
-        y.y = s * a.y + c * b.y;
-    } else { // diag(c - i s, c + i s)
-        x.x = c * a.x + s * a.y;
-        x.y = c * a.y - s * a.x;
-        y.x = c * b.x - s * b.y;
-        y.y = c * b.y + s * b.x;
-    }
-    a = x;
-    b = y;
+    mats[i] = m;
 }
 
 // local tile index e -> global amplitude index.  Every stage's tile is bits
@@ -204,66 +168,6 @@ __device__ __forceinline__ uint64_t gather_src(uint64_t y, const uint32_t *rows,
         x |= static_cast<uint64_t>(__popc(static_cast<uint32_t>(y) & rows[b]) & 1) << b;
     }
     return x;
-}
-
-// Forward rotation stage: for every target wire of the tile, the product of
-// its pattern rotations (one 2x2 per wire) is applied in LDS.  gsrc >= 0: the
-// previous layer's entangler is fused in -- the tile is gathered from buffer
-// gsrc through the entangler's map and written to buffer buf (so the
-// entangler costs no pass of its own).
-template <class T>
-__global__ __launch_bounds__(kBlock) void k_batch_rot(v2<T> *__restrict__ arena,
-                                                      const BCirc *__restrict__ circs,
-                                                      const BLaunch L, int W, int stage, int layer,
-                                                      int buf, int gsrc, int npat, int4 pat,
-                                                      const double2 *__restrict__ cs) {
-    extern __shared__ unsigned char smem_raw[];
-    v2<T> *tile = reinterpret_cast<v2<T> *>(smem_raw);
-    uint64_t q;
-    const BCirc &c = circs[find_circ(L, blockIdx.x, q)];
-    int bits[16];
-    int alo, ahi;
-    const int Tn = stage_bits(c.n, W, stage, bits, alo, ahi);
-    const uint64_t len = uint64_t{1} << c.n;
-    v2<T> *sv = arena + c.off + buf * len;
-    const uint64_t base = tile_base(q, bits, Tn);
-    const uint32_t tsz = 1U << Tn;
-    if (gsrc >= 0) {
-        const v2<T> *src = arena + c.off + gsrc * len;
-        for (uint32_t e = threadIdx.x; e < tsz; e += kBlock) {
-            tile[e] = src[gather_src(tile_index(base, e, bits, Tn), c.fwd_rows, c.n)];
-        }
-    } else {
-        for (uint32_t e = threadIdx.x; e < tsz; e += kBlock) {
-            tile[e] = sv[tile_index(base, e, bits, Tn)];
-        }
-    }
-    __syncthreads();
-    const int axes[4] = {pat.x, pat.y, pat.z, pat.w};
-    for (int k = 0; k < Tn; k++) {
-        const int b = bits[k];
-        if (b < alo || b >= ahi) {
-            continue;
-        }
-        const int w = c.n - 1 - b;
-        const double2 *th = cs + c.par + (static_cast<uint64_t>(layer) * c.n + w) * npat;
-        Rot2<T> m = rot_matrix<T>(axes[0], th[0], false);
-        for (int a = 1; a < npat; a++) {
-            m = mat2_mul(rot_matrix<T>(axes[a], th[a], false), m);
-        }
-        for (uint32_t p = threadIdx.x; p < (tsz >> 1); p += kBlock) {
-            const uint32_t lo = p & ((1U << k) - 1);
-            const uint32_t i0 = ((p >> k) << (k + 1)) | lo, i1 = i0 | (1U << k);
-            v2<T> x = tile[i0], y = tile[i1];
-            apply2(m, x, y);
-            tile[i0] = x;
-            tile[i1] = y;
-        }
-        __syncthreads();
-    }
-    for (uint32_t e = threadIdx.x; e < tsz; e += kBlock) {
-        sv[tile_index(base, e, bits, Tn)] = tile[e];
-    }
 }
 
 // Entangler as a gather: dst[y] = src[src_index(y)] for the buffers given.
@@ -366,128 +270,182 @@ __global__ __launch_bounds__(kBlock) void k_batch_obs(v2<T> *__restrict__ arena,
     }
 }
 
-// Adjoint rotation stage: lambda (buffer lb) and H (buffer hb) tiles in LDS.
-// For each target wire, pattern rotations are undone last-to-first; before
-// undoing rotation a, Im<H|G_a lambda> is accumulated for angle a
-// (scale -1/2 and the -2 of the reference's update cancel: dE/dtheta =
-// Im<H|G lambda>, AdjointJacobianLQubit.hpp:70-75).  Each wave reduces its
-// share with shuffles into a per-wave LDS slot; after the last wire one pass
-// adds the four waves' slots and issues one FP64 atomic per angle.
-// glb >= 0: the layer's entangler is undone in the same pass -- for a
-// circuit whose first adjoint stage of the layer this is (stage ==
-// nstage - 1), lambda and H are gathered from buffers glb and ghb through the
-// inverse map and written to lb and hb.
-template <class T>
-__global__ __launch_bounds__(kBlock) void k_batch_rot_adj(v2<T> *__restrict__ arena,
-                                                          const BCirc *__restrict__ circs,
-                                                          const BLaunch L, int W, int stage,
-                                                          int layer, int lb, int hb, int glb, int ghb,
-                                                          int npat, int4 pat, const double2 *__restrict__ cs,
-                                                          double *__restrict__ grads) {
+// One rotation stage of a layer over every circuit that has it: a tile of
+// lambda (ADJ: and of H lambda) in registers, windows of three target bits
+// from the highest down, each bit's 2x2 applied in registers.
+//
+// ADJ undoes the rotations.  The gradients of a wire's letters are linear
+// forms of M_ab = sum conj(h_a) lambda_b on the states before any of them is
+// undone: with W = U G U^dagger, U the letters after the one whose generator
+// is G, W = x X + y Y + z Z and Im <H|G lambda> = z Im(M00 - M11) +
+// x Im(M01 + M10) - y Re(M01 - M10).  So the three sums are accumulated in
+// FP64 per wire and the wire is undone by one 2x2, whatever the pattern's
+// length (scale -1/2 and the -2 of the reference's update cancel:
+// dE/dtheta = Im <H|G lambda>, AdjointJacobianLQubit.hpp:70-75).
+//
+// gl >= 0: the entangler between this layer and the neighbouring one is fused
+// in: at the layer's first stage in execution order (forward stage 0, adjoint
+// stage nstage - 1) lambda and H are gathered from buffers gl and gh through
+// the entangler's index map (forward) or its inverse and written to lb and hb.
+// The map is linear over GF(2), so a source index is the exclusive or of the
+// tile's, the thread's and the register's parts.
+//
+// A trip through LDS and a barrier per wire, as before, left the stages at 2.6
+// (adjoint) and 3.3 TB/s; windows take a third of the trips.  complex64 states
+// are rotated in double: a stage rounds an amplitude once.
+// BATCH_FIGURES
+template <class T, int NW, bool ADJ>
+__global__ __launch_bounds__(64 * NW, NW == 16 ? 4 : ADJ ? 4 : 6) void k_batch_stage(
+    v2<T> *__restrict__ arena, const BCirc *__restrict__ circs, const BLaunch L, int W, int stage, int layer, int lb,
+    int hb, int gl, int gh, int npat, int4 pat, const BMat *__restrict__ mats, const double2 *__restrict__ cs,
+    double *__restrict__ grads) {
+    constexpr int RB = 3, R = 1 << RB, S = ADJ ? 2 : 1;
+    constexpr int TB = 6 + (NW == 16 ? 4 : NW == 8 ? 3 : NW == 4 ? 2 : NW == 2 ? 1 : 0);
+    auto window_at = [](int p) { return static_cast<uint32_t>(p | (p + 1) << 4 | (p + 2) << 8); };
+    constexpr uint32_t HOME = TB | (TB + 1) << 4 | (TB + 2) << 8;
     extern __shared__ unsigned char smem_raw[];
-    __shared__ double wpart[kBlock / 64][kBatchMaxTile][kBatchMaxPattern];
+    __shared__ double wpart[ADJ ? NW : 1][ADJ ? kBatchMaxTile : 1][4];
+    double *buf = reinterpret_cast<double *>(smem_raw);
     uint64_t q;
     const BCirc &c = circs[find_circ(L, blockIdx.x, q)];
     int bits[16];
     int alo, ahi;
     const int Tn = stage_bits(c.n, W, stage, bits, alo, ahi);
-    const uint32_t tsz = 1U << Tn;
-    v2<T> *tl = reinterpret_cast<v2<T> *>(smem_raw);
-    v2<T> *th_ = tl + tsz;
+    const uint32_t tid = threadIdx.x, size = 1U << Tn;
     const uint64_t len = uint64_t{1} << c.n;
-    v2<T> *lam = arena + c.off + lb * len;
-    v2<T> *hh = arena + c.off + hb * len;
+    v2<T> *st[2] = {arena + c.off + lb * len, arena + c.off + (ADJ ? hb : lb) * len};
     const uint64_t base = tile_base(q, bits, Tn);
-    if (glb >= 0 && stage == c.nstage - 1) { // uniform per workgroup
-        const v2<T> *ls = arena + c.off + glb * len, *hs = arena + c.off + ghb * len;
-        for (uint32_t e = threadIdx.x; e < tsz; e += kBlock) {
-            const uint64_t x = gather_src(tile_index(base, e, bits, Tn), c.adj_rows, c.n);
-            tl[e] = ls[x];
-            th_[e] = hs[x];
-        }
-    } else {
-        for (uint32_t e = threadIdx.x; e < tsz; e += kBlock) {
-            const uint64_t g = tile_index(base, e, bits, Tn);
-            tl[e] = lam[g];
-            th_[e] = hh[g];
+    const uint64_t thread_at = tile_index(0, tid, bits, Tn);
+    auto reg_at = [&](int r) { return tile_index(0, static_cast<uint32_t>(r) << TB, bits, Tn); };
+    double2 x[S][R];
+    const bool gather = gl >= 0 && stage == (ADJ ? c.nstage - 1 : 0);
+    const uint32_t *rows = ADJ ? c.adj_rows : c.fwd_rows;
+    const uint64_t from = gather ? gather_src(base, rows, c.n) ^ gather_src(thread_at, rows, c.n) : base | thread_at;
+    const v2<T> *src[2] = {gather ? arena + c.off + gl * len : st[0], gather && ADJ ? arena + c.off + gh * len : st[1]};
+    uint64_t reg_from[RB];
+#pragma unroll
+    for (int j = 0; j < RB; j++) {
+        reg_from[j] = gather ? gather_src(reg_at(1 << j), rows, c.n) : reg_at(1 << j);
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const uint64_t a = from ^ ((r & 1) ? reg_from[0] : 0) ^ ((r & 2) ? reg_from[1] : 0) ^ ((r & 4) ? reg_from[2] : 0);
+        const bool in = ((static_cast<uint32_t>(r) << TB) | tid) < size;
+#pragma unroll
+        for (int i = 0; i < S; i++) {
+            x[i][r] = double2{0, 0};
+            if (in) {
+                const v2<T> v = src[i][a];
+                x[i][r] = double2{v.x, v.y};
+            }
         }
     }
-    __syncthreads();
-    const int axes[4] = {pat.x, pat.y, pat.z, pat.w};
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int slot = 0; // target wires done so far: slot j is bit alo + j
-    for (int k = 0; k < Tn; k++) {
-        const int b = bits[k];
-        if (b < alo || b >= ahi) {
-            continue;
+    // local positions of the target bits: [ka, kb)
+    const int shift = stage == 0 ? 0 : bits[3] - 3;
+    const int ka = alo - shift, kb = ahi - shift;
+    const BMat *lm = mats + c.par / npat + static_cast<uint64_t>(layer) * c.n;
+    const int lane = tid & 63, wave = tid >> 6;
+    uint32_t win = HOME;
+    for (int top = kb; top > ka;) { // target bits at and above `top` are done
+        const int p = top >= 3 ? top - 3 : 0;
+        if (window_at(p) != win) {
+            rt_window<TB, RB>(x, buf, tid, win, window_at(p));
+            win = window_at(p);
         }
-        const int w = c.n - 1 - b;
-        const uint64_t pidx = c.par + (static_cast<uint64_t>(layer) * c.n + w) * npat;
-        double acc[kBatchMaxPattern] = {0, 0, 0, 0};
-        // letter loops run to the compile-time maximum with a guard, so the
-        // per-letter arrays keep static indices and stay in registers
-        double2 rcs[kBatchMaxPattern];
-#pragma unroll
-        for (int a = 0; a < kBatchMaxPattern; a++) {
-            rcs[a] = a < npat ? cs[pidx + a] : double2{1, 0};
-        }
-        for (uint32_t p = threadIdx.x; p < (tsz >> 1); p += kBlock) {
-            const uint32_t lo = p & ((1U << k) - 1);
-            const uint32_t i0 = ((p >> k) << (k + 1)) | lo, i1 = i0 | (1U << k);
-            v2<T> l0 = tl[i0], l1 = tl[i1], h0 = th_[i0], h1 = th_[i1];
-#pragma unroll
-            for (int a = kBatchMaxPattern - 1; a >= 0; a--) {
-                if (a >= npat) {
-                    continue;
-                }
-                // G lambda for G = X, Y or Z on this wire
-                v2<T> g0, g1;
-                if (axes[a] == 0) {
-                    g0 = l1;
-                    g1 = l0;
-                } else if (axes[a] == 1) {
-                    g0.x = l1.y; g0.y = -l1.x;   // -i * l1
-                    g1.x = -l0.y; g1.y = l0.x;   //  i * l0
-                } else {
-                    g0 = l0;
-                    g1.x = -l1.x; g1.y = -l1.y;
-                }
-                // Im(conj(h) g)
-                acc[a] += double(h0.x) * double(g0.y) - double(h0.y) * double(g0.x) +
-                          double(h1.x) * double(g1.y) - double(h1.y) * double(g1.x);
-                rot_apply<T>(axes[a], rcs[a], true, l0, l1);
-                rot_apply<T>(axes[a], rcs[a], true, h0, h1);
+        auto bit = [&](auto jt) {
+            constexpr int J = decltype(jt)::value;
+            const int k = p + J;
+            if (k < ka || k >= top) {
+                return;
             }
-            tl[i0] = l0;
-            tl[i1] = l1;
-            th_[i0] = h0;
-            th_[i1] = h1;
-        }
+            const int b = k + shift;
+            const BMat &mt = lm[c.n - 1 - b];
+            dcx<double> u[4];
+            if constexpr (ADJ) {
+                u[0] = {mt.u[0].r, -mt.u[0].i};
+                u[1] = {mt.u[2].r, -mt.u[2].i};
+                u[2] = {mt.u[1].r, -mt.u[1].i};
+                u[3] = {mt.u[3].r, -mt.u[3].i};
+                double s0 = 0, s1 = 0, s2 = 0;
 #pragma unroll
-        for (int a = 0; a < kBatchMaxPattern; a++) {
-            if (a < npat) {
-                const double s = wave_sum(acc[a]);
-                if (lane == 0) {
-                    wpart[wave][slot][a] = s;
+                for (int pr = 0; pr < R / 2; pr++) {
+                    const int i0 = ((pr >> J) << (J + 1)) | (pr & ((1 << J) - 1)), i1 = i0 | (1 << J);
+                    const double ax = x[0][i0].x, ay = x[0][i0].y, bx = x[0][i1].x, by = x[0][i1].y;
+                    const double cx = x[S - 1][i0].x, cy = x[S - 1][i0].y, dx = x[S - 1][i1].x, dy = x[S - 1][i1].y;
+                    s0 = rt_fma(cx, ay, rt_fma(-cy, ax, rt_fma(-dx, by, rt_fma(dy, bx, s0))));
+                    s1 = rt_fma(cx, by, rt_fma(-cy, bx, rt_fma(dx, ay, rt_fma(-dy, ax, s1))));
+                    s2 = rt_fma(cx, bx, rt_fma(cy, by, rt_fma(-dx, ax, rt_fma(-dy, ay, s2))));
+                }
+                const double t = rt_sum4(s0, s1, s2, 0.0);
+                if ((lane & 15) == 0) {
+                    wpart[wave][b - alo][rt_row(lane >> 4)] = t;
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    u[j] = mt.u[j];
                 }
             }
+#pragma unroll
+            for (int pr = 0; pr < R / 2; pr++) {
+                const int i0 = ((pr >> J) << (J + 1)) | (pr & ((1 << J) - 1)), i1 = i0 | (1 << J);
+#pragma unroll
+                for (int i = 0; i < S; i++) {
+                    rt_apply2(~uint64_t{0}, u, x[i][i0], x[i][i1]);
+                }
+            }
+        };
+        bit(std::integral_constant<int, 2>{});
+        bit(std::integral_constant<int, 1>{});
+        bit(std::integral_constant<int, 0>{});
+        top = p > ka ? p : ka;
+    }
+    if (win != HOME) {
+        rt_window<TB, RB>(x, buf, tid, win, HOME);
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        if (((static_cast<uint32_t>(r) << TB) | tid) < size) {
+            const uint64_t a = base | thread_at | reg_at(r);
+#pragma unroll
+            for (int i = 0; i < S; i++) {
+                st[i][a] = v2<T>{static_cast<T>(x[i][r].x), static_cast<T>(x[i][r].y)};
+            }
         }
-        slot++;
+    }
+    if constexpr (ADJ) {
         __syncthreads();
-    }
-    for (int t = threadIdx.x; t < slot * npat; t += kBlock) {
-        const int sl = t / npat, a = t - sl * npat;
-        double s = 0;
-        for (int v = 0; v < kBlock / 64; v++) {
-            s += wpart[v][sl][a];
+        const int axes[4] = {pat.x, pat.y, pat.z, pat.w};
+        for (int t = tid; t < (ahi - alo) * npat; t += 64 * NW) {
+            const int sl = t / npat, a = t - sl * npat;
+            double s[3] = {0, 0, 0};
+            for (int v = 0; v < NW; v++) {
+#pragma unroll
+                for (int j = 0; j < 3; j++) {
+                    s[j] += wpart[v][sl][j];
+                }
+            }
+            const uint64_t pidx = c.par + (static_cast<uint64_t>(layer) * c.n + (c.n - 1 - (alo + sl))) * npat;
+            // W: the generator's axis turned by the letters after it
+            double w[3] = {axes[a] == 0 ? 1.0 : 0.0, axes[a] == 1 ? 1.0 : 0.0, axes[a] == 2 ? 1.0 : 0.0};
+            for (int l = a + 1; l < npat; l++) {
+                const double2 h = cs[pidx + l];
+                const double co = h.x * h.x - h.y * h.y, si = 2 * h.x * h.y;
+                // right-handed about axis l: (e1, e2) the two following axes
+                const double x0 = w[0], y0 = w[1], z0 = w[2];
+                if (axes[l] == 0) {
+                    w[1] = y0 * co - z0 * si;
+                    w[2] = y0 * si + z0 * co;
+                } else if (axes[l] == 1) {
+                    w[2] = z0 * co - x0 * si;
+                    w[0] = z0 * si + x0 * co;
+                } else {
+                    w[0] = x0 * co - y0 * si;
+                    w[1] = x0 * si + y0 * co;
+                }
+            }
+            atomicAdd(grads + pidx + a, w[2] * s[0] + (w[0] * s[1] - w[1] * s[2]));
         }
-        const int w = c.n - 1 - (alo + sl);
-        atomicAdd(grads + c.par + (static_cast<uint64_t>(layer) * c.n + w) * npat + a, s);
-    }
-    for (uint32_t e = threadIdx.x; e < tsz; e += kBlock) {
-        const uint64_t g = tile_index(base, e, bits, Tn);
-        lam[g] = tl[e];
-        hh[g] = th_[e];
     }
 }
 

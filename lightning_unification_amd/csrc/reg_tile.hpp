@@ -1,0 +1,185 @@
+// Register tiles: a workgroup holds 2^(TB + RB) amplitudes, 2^RB of them in
+// each of its 2^TB threads.  A thread's amplitudes differ in the RB window
+// bits of the local index (`win`, four bits a position, ascending); its thread
+// index supplies the other bits.  Gates on window bits need no exchange; a
+// change of window goes through an LDS buffer of real parts and imaginary
+// parts (an element of both would tie the two registers of an amplitude into
+// one tuple, which in-place updates would have to copy out of and back into).
+// Used by the backward sweep (kernels_adjoint.hpp) and the batched circuits
+// (kernels_batch.hpp).
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "kernels_gate.hpp"
+
+namespace plamd {
+
+// Sums of a and b over lanes l and l ^ 32: a's in the lower half, b's in the upper.
+__device__ __forceinline__ double rt_fold32(double a, double b) {
+    const auto ua = static_cast<unsigned long long>(__double_as_longlong(a));
+    const auto ub = static_cast<unsigned long long>(__double_as_longlong(b));
+    const auto lo = __builtin_amdgcn_permlane32_swap(static_cast<unsigned>(ua), static_cast<unsigned>(ub), false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(static_cast<unsigned>(ua >> 32), static_cast<unsigned>(ub >> 32),
+                                                     false, false);
+    const double x = __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi[0]) << 32) | lo[0]));
+    const double y = __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi[1]) << 32) | lo[1]));
+    return x + y;
+}
+// Sums of a and b over lanes l and l ^ 16: a's in even rows of 16 lanes, b's in odd ones.
+__device__ __forceinline__ double rt_fold16(double a, double b) {
+    const auto ua = static_cast<unsigned long long>(__double_as_longlong(a));
+    const auto ub = static_cast<unsigned long long>(__double_as_longlong(b));
+    const auto lo = __builtin_amdgcn_permlane16_swap(static_cast<unsigned>(ua), static_cast<unsigned>(ub), false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(static_cast<unsigned>(ua >> 32), static_cast<unsigned>(ub >> 32),
+                                                     false, false);
+    const double x = __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi[0]) << 32) | lo[0]));
+    const double y = __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi[1]) << 32) | lo[1]));
+    return x + y;
+}
+template <int CTRL> __device__ __forceinline__ double rt_dpp(double v) {
+    const auto u = static_cast<unsigned long long>(__double_as_longlong(v));
+    const unsigned lo = static_cast<unsigned>(__builtin_amdgcn_mov_dpp(static_cast<int>(static_cast<unsigned>(u)), CTRL, 0xf, 0xf, true));
+    const unsigned hi = static_cast<unsigned>(__builtin_amdgcn_mov_dpp(static_cast<int>(static_cast<unsigned>(u >> 32)), CTRL, 0xf, 0xf, true));
+    return __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi) << 32) | lo));
+}
+// Totals of four values over the wavefront: row r of 16 lanes (lane / 16 = r)
+// ends with the total of v[rt_row(r)].
+__device__ __forceinline__ double rt_sum4(double v0, double v1, double v2, double v3) {
+    // rows 0..3 after the folds: v0, v2, v1, v3
+    double s = rt_fold16(rt_fold32(v0, v1), rt_fold32(v2, v3));
+    s += rt_dpp<0x128>(s); // rotations within a row by 8, 4, 2, 1
+    s += rt_dpp<0x124>(s);
+    s += rt_dpp<0x122>(s);
+    s += rt_dpp<0x121>(s);
+    return s;
+}
+__device__ __forceinline__ int rt_row(int r) { return ((r & 1) << 1) | (r >> 1); }
+
+// Local index -> place in the LDS buffer, linear in its bits.  With a window
+// bit among the lowest, neighbouring lanes hold every other amplitude of 128
+// bytes; flipping the bits inside 128 bytes where the next bit is set spreads
+// them over all banks again.
+__device__ __forceinline__ uint32_t rt_place(uint32_t e) {
+    constexpr int b = 4; // 16 doubles
+    return e ^ (((e >> b) & 1U) * ((1U << b) - 1));
+}
+
+// thread bits spread over the local bits outside the window
+template <int RB> __device__ __forceinline__ uint32_t rt_thread_part(uint32_t t, uint32_t win) {
+#pragma unroll
+    for (int j = 0; j < RB; j++) {
+        const uint32_t m = (1U << ((win >> (4 * j)) & 15U)) - 1;
+        t = ((t & ~m) << 1) | (t & m);
+    }
+    return t;
+}
+__device__ __forceinline__ double rt_fma(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
+// Updates of the register tile.  The last multiply-add of every amplitude
+// writes the amplitude's own register, in the lanes of `m` only; the lane
+// condition is an execution mask inside the block, so a step has no divergent
+// branch.  Left to the compiler (branches on the condition, results in
+// registers of their own), every step's results were copied back where the
+// steps' branches join: 241 registers and two wavefronts a SIMD for KH = 2 in
+// complex128, a third of the instructions moves.  All 64 lanes are active
+// around every block.
+__device__ __forceinline__ void rt_into(uint64_t m, double2 &a, double u, double tx, double ty) {
+    asm("s_mov_b64 exec, %2\n\t"
+        "v_fma_f64 %0, %3, %0, %4\n\t"
+        "v_fma_f64 %1, %3, %1, %5\n\t"
+        "s_mov_b64 exec, -1"
+        : "+v"(a.x), "+v"(a.y)
+        : "s"(m), "v"(u), "v"(tx), "v"(ty));
+}
+__device__ __forceinline__ void rt_into2(uint64_t m, double2 &a, double2 &b, double ua, double ub, double t0,
+                                            double t1, double t2, double t3) {
+    asm("s_mov_b64 exec, %4\n\t"
+        "v_fma_f64 %0, %5, %0, %7\n\t"
+        "v_fma_f64 %1, %5, %1, %8\n\t"
+        "v_fma_f64 %2, %6, %2, %9\n\t"
+        "v_fma_f64 %3, %6, %3, %10\n\t"
+        "s_mov_b64 exec, -1"
+        : "+v"(a.x), "+v"(a.y), "+v"(b.x), "+v"(b.y)
+        : "s"(m), "s"(ua), "s"(ub), "v"(t0), "v"(t1), "v"(t2), "v"(t3));
+}
+// a <-> b in the lanes of m
+__device__ __forceinline__ void rt_exchange(uint64_t m, double2 &a, double2 &b) {
+    double t;
+    asm("s_mov_b64 exec, %5\n\t"
+        "v_mov_b64 %4, %0\n\t"
+        "v_mov_b64 %0, %2\n\t"
+        "v_mov_b64 %2, %4\n\t"
+        "v_mov_b64 %4, %1\n\t"
+        "v_mov_b64 %1, %3\n\t"
+        "v_mov_b64 %3, %4\n\t"
+        "s_mov_b64 exec, -1"
+        : "+v"(a.x), "+v"(a.y), "+v"(b.x), "+v"(b.y), "=&v"(t)
+        : "s"(m));
+}
+
+// (a, b) <- u (a, b) in the lanes of m, 16 multiply-adds
+__device__ __forceinline__ void rt_apply2(uint64_t m, const dcx<double> *u, double2 &a, double2 &b) {
+    const double t0 = rt_fma(-u[0].i, a.y, rt_fma(u[1].r, b.x, -u[1].i * b.y));
+    const double t1 = rt_fma(u[0].i, a.x, rt_fma(u[1].r, b.y, u[1].i * b.x));
+    const double t2 = rt_fma(-u[3].i, b.y, rt_fma(u[2].r, a.x, -u[2].i * a.y));
+    const double t3 = rt_fma(u[3].i, b.x, rt_fma(u[2].r, a.y, u[2].i * a.x));
+    rt_into2(m, a, b, u[0].r, u[3].r, t0, t1, t2, t3);
+}
+
+// (a, b) <- u (a, b), left to the compiler: for code without a step's branches
+__device__ __forceinline__ void rt_mul2(const dcx<double> *u, double2 &a, double2 &b) {
+    const double ax = a.x, ay = a.y, bx = b.x, by = b.y;
+    a.x = rt_fma(u[0].r, ax, rt_fma(-u[0].i, ay, rt_fma(u[1].r, bx, -u[1].i * by)));
+    a.y = rt_fma(u[0].r, ay, rt_fma(u[0].i, ax, rt_fma(u[1].r, by, u[1].i * bx)));
+    b.x = rt_fma(u[2].r, ax, rt_fma(-u[2].i, ay, rt_fma(u[3].r, bx, -u[3].i * by)));
+    b.y = rt_fma(u[2].r, ay, rt_fma(u[2].i, ax, rt_fma(u[3].r, by, u[3].i * bx)));
+}
+
+// The S states of a tile moved from window `from` to window `to` through
+// `buf` (2^(TB + RB) real parts, then as many imaginary parts), one state at a
+// time.  All threads of the workgroup call it.
+template <int TB, int RB, int S>
+__device__ __forceinline__ void rt_window(double2 (&x)[S][1 << RB], double *buf, uint32_t tid, uint32_t from,
+                                          uint32_t to) {
+    constexpr uint32_t IM = 1U << (TB + RB);
+    const uint32_t tf = rt_place(rt_thread_part<RB>(tid, from));
+    const uint32_t tt = rt_place(rt_thread_part<RB>(tid, to));
+    // the register index's part, from its bits' parts (uniform): computed per
+    // register instead, it costs more scalar instructions than the step's
+    // multiply-adds
+    uint32_t fb[RB], ob[RB];
+#pragma unroll
+    for (int j = 0; j < RB; j++) {
+        fb[j] = rt_place(1U << ((from >> (4 * j)) & 15U));
+        ob[j] = rt_place(1U << ((to >> (4 * j)) & 15U));
+    }
+    auto part = [](int r, const uint32_t (&v)[RB]) {
+        uint32_t e = 0;
+#pragma unroll
+        for (int j = 0; j < RB; j++) {
+            e ^= ((r >> j) & 1) ? v[j] : 0U;
+        }
+        return e;
+    };
+#pragma unroll
+    for (int i = 0; i < S; i++) {
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < (1 << RB); r++) {
+            const uint32_t p = tf ^ part(r, fb);
+            buf[p] = x[i][r].x;
+            buf[p + IM] = x[i][r].y;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < (1 << RB); r++) {
+            const uint32_t p = tt ^ part(r, ob);
+            x[i][r].x = buf[p];
+            x[i][r].y = buf[p + IM];
+        }
+    }
+}
+
+} // namespace plamd
