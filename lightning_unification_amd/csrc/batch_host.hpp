@@ -338,7 +338,7 @@ template <class T> struct BatchPlan final : BatchPlanBase {
     template <bool ADJ> void stage(const LaunchSpec &ls, int lb, int hb, int gl, int gh) {
         auto go = [&](auto nw) {
             constexpr int NW = decltype(nw)::value;
-            const size_t lds = sizeof(double2) * 8 * 64 * NW;
+            const size_t lds = (ADJ ? sizeof(double2) : sizeof(double)) * 8 * 64 * NW;
             hipLaunchKernelGGL((k_batch_stage<T, NW, ADJ>), dim3(static_cast<unsigned>(ls.blocks)), dim3(64 * NW), lds,
                                stream, arena, dcircs, ls.L, W, ls.stage, ls.layer, lb, hb, gl, gh, npat, pat, dmats,
                                dcs, dgrads);

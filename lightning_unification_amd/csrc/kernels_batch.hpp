@@ -295,7 +295,7 @@ __global__ __launch_bounds__(kBlock) void k_batch_obs(v2<T> *__restrict__ arena,
 // are rotated in double: a stage rounds an amplitude once.
 // BATCH_FIGURES
 template <class T, int NW, bool ADJ>
-__global__ __launch_bounds__(64 * NW, NW == 16 ? 4 : ADJ ? 4 : 6) void k_batch_stage(
+__global__ __launch_bounds__(64 * NW, NW == 16 || ADJ ? 4 : 8) void k_batch_stage(
     v2<T> *__restrict__ arena, const BCirc *__restrict__ circs, const BLaunch L, int W, int stage, int layer, int lb,
     int hb, int gl, int gh, int npat, int4 pat, const BMat *__restrict__ mats, const double2 *__restrict__ cs,
     double *__restrict__ grads) {
@@ -349,7 +349,7 @@ __global__ __launch_bounds__(64 * NW, NW == 16 ? 4 : ADJ ? 4 : 6) void k_batch_s
     for (int top = kb; top > ka;) { // target bits at and above `top` are done
         const int p = top >= 3 ? top - 3 : 0;
         if (window_at(p) != win) {
-            rt_window<TB, RB>(x, buf, tid, win, window_at(p));
+            rt_window<TB, RB, S, !ADJ>(x, buf, tid, win, window_at(p));
             win = window_at(p);
         }
         auto bit = [&](auto jt) {
@@ -401,7 +401,7 @@ __global__ __launch_bounds__(64 * NW, NW == 16 ? 4 : ADJ ? 4 : 6) void k_batch_s
         top = p > ka ? p : ka;
     }
     if (win != HOME) {
-        rt_window<TB, RB>(x, buf, tid, win, HOME);
+        rt_window<TB, RB, S, !ADJ>(x, buf, tid, win, HOME);
     }
 #pragma unroll
     for (int r = 0; r < R; r++) {

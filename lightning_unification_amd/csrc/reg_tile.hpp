@@ -57,14 +57,12 @@ __device__ __forceinline__ double rt_sum4(double v0, double v1, double v2, doubl
 }
 __device__ __forceinline__ int rt_row(int r) { return ((r & 1) << 1) | (r >> 1); }
 
-// Local index -> place in the LDS buffer, linear in its bits.  With a window
-// bit among the lowest, neighbouring lanes hold every other amplitude of 128
-// bytes; flipping the bits inside 128 bytes where the next bit is set spreads
-// them over all banks again.
-__device__ __forceinline__ uint32_t rt_place(uint32_t e) {
-    constexpr int b = 4; // 16 doubles
-    return e ^ (((e >> b) & 1U) * ((1U << b) - 1));
-}
+// Local index -> place in the LDS buffer, linear in its bits.  With window bits
+// p .. p + 2, consecutive lanes differ in the local bits around them; the map
+// folds bits 4..7 into the low five so that for every p the first four lane
+// bits give 16 different places mod 16 and the first five 32 mod 32 (doubles:
+// no two lanes of an access share a bank).
+__device__ __forceinline__ uint32_t rt_place(uint32_t e) { return e ^ ((e >> 3) & 30U) ^ ((e >> 6) & 1U); }
 
 // thread bits spread over the local bits outside the window
 template <int RB> __device__ __forceinline__ uint32_t rt_thread_part(uint32_t t, uint32_t win) {
@@ -138,9 +136,10 @@ __device__ __forceinline__ void rt_mul2(const dcx<double> *u, double2 &a, double
 }
 
 // The S states of a tile moved from window `from` to window `to` through
-// `buf` (2^(TB + RB) real parts, then as many imaginary parts), one state at a
-// time.  All threads of the workgroup call it.
-template <int TB, int RB, int S>
+// `buf`, one state at a time: 2^(TB + RB) real parts, then as many imaginary
+// parts; HALF: the parts take turns in a buffer of half that size, for two
+// more barriers a state.  All threads of the workgroup call it.
+template <int TB, int RB, int S, bool HALF = false>
 __device__ __forceinline__ void rt_window(double2 (&x)[S][1 << RB], double *buf, uint32_t tid, uint32_t from,
                                           uint32_t to) {
     constexpr uint32_t IM = 1U << (TB + RB);
@@ -165,19 +164,26 @@ __device__ __forceinline__ void rt_window(double2 (&x)[S][1 << RB], double *buf,
     };
 #pragma unroll
     for (int i = 0; i < S; i++) {
-        __syncthreads();
 #pragma unroll
-        for (int r = 0; r < (1 << RB); r++) {
-            const uint32_t p = tf ^ part(r, fb);
-            buf[p] = x[i][r].x;
-            buf[p + IM] = x[i][r].y;
-        }
-        __syncthreads();
+        for (int h = 0; h < (HALF ? 2 : 1); h++) {
+            __syncthreads();
 #pragma unroll
-        for (int r = 0; r < (1 << RB); r++) {
-            const uint32_t p = tt ^ part(r, ob);
-            x[i][r].x = buf[p];
-            x[i][r].y = buf[p + IM];
+            for (int r = 0; r < (1 << RB); r++) {
+                const uint32_t p = tf ^ part(r, fb);
+                buf[p] = h ? x[i][r].y : x[i][r].x;
+                if constexpr (!HALF) {
+                    buf[p + IM] = x[i][r].y;
+                }
+            }
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < (1 << RB); r++) {
+                const uint32_t p = tt ^ part(r, ob);
+                (h ? x[i][r].y : x[i][r].x) = buf[p];
+                if constexpr (!HALF) {
+                    x[i][r].y = buf[p + IM];
+                }
+            }
         }
     }
 }
