@@ -226,6 +226,11 @@ struct pl_sv {
     size_t staging_bytes = 0;
     std::vector<hipEvent_t> slots; // pl_event_record slots
     std::vector<std::pair<void *, size_t>> bufs; // grow-only device buffers by purpose (plamd::Buf)
+    // pinned copy of the programs of the last call's passes (ProgramBuffer)
+    void *prog_host = nullptr;
+    size_t prog_host_bytes = 0;
+    hipEvent_t prog_ev = nullptr;
+    bool prog_busy = false; // prog_ev is recorded behind copies from prog_host
     // gates queued while deferral is on (pl_sv_set_deferred), in the tape
     // encoding of pl_sv_apply_ops; applied as tile passes before anything
     // else reads or changes the state

@@ -161,6 +161,73 @@ static void download_host(pl_sv_t h, void *dst, const void *src, size_t bytes) {
     drain(nchunks - 1);
 }
 
+template <class T> constexpr int kSweepLow = std::is_same_v<T, double> ? 3 : 4; // one 128-byte line
+
+// The programs of one call's passes on their way to the device: appended to
+// the handle's pinned buffer and copied from there without waiting.  The
+// buffer is taken again once the last call's copies have left it (an event);
+// where it cannot be pinned, each copy is waited for.
+class ProgramBuffer {
+  public:
+    ProgramBuffer(pl_sv *h, size_t steps) : h_(h) {
+        const size_t bytes = steps * sizeof(SweepStep);
+        if (h->prog_busy) {
+            HIP_OK(hipEventSynchronize(h->prog_ev));
+            h->prog_busy = false;
+        }
+        if (h->prog_host_bytes < bytes) {
+            if (h->prog_host) {
+                HIP_OK(hipHostFree(h->prog_host));
+                h->prog_host = nullptr;
+                h->prog_host_bytes = 0;
+            }
+            const size_t sz = std::max<size_t>(bytes, 1 << 16);
+            if (hipHostMalloc(&h->prog_host, sz, hipHostMallocDefault) == hipSuccess) {
+                h->prog_host_bytes = sz;
+            } else {
+                (void)hipGetLastError();
+                h->prog_host = nullptr;
+            }
+        }
+        if (!h->prog_ev) {
+            HIP_OK(hipEventCreateWithFlags(&h->prog_ev, hipEventDisableTiming));
+        }
+        dev_ = static_cast<SweepStep *>(buf(h, kBufSweepProg, std::max<size_t>(bytes, 1 << 16)));
+        cap_ = steps;
+    }
+    ~ProgramBuffer() {
+        if (used_ > 0 && h_->prog_host) {
+            h_->prog_busy = hipEventRecord(h_->prog_ev, h_->stream) == hipSuccess;
+            if (!h_->prog_busy) {
+                (void)hipStreamSynchronize(h_->stream);
+            }
+        }
+    }
+    // the device address of the steps, in place for work queued after this
+    const SweepStep *put(const std::vector<SweepStep> &steps) {
+        if (used_ + steps.size() > cap_) {
+            throw std::logic_error("a program longer than its steps and windows");
+        }
+        SweepStep *to = dev_ + used_;
+        const size_t bytes = steps.size() * sizeof(SweepStep);
+        if (h_->prog_host) {
+            SweepStep *from = static_cast<SweepStep *>(h_->prog_host) + used_;
+            std::memcpy(from, steps.data(), bytes);
+            HIP_OK(hipMemcpyAsync(to, from, bytes, hipMemcpyHostToDevice, h_->stream));
+        } else {
+            HIP_OK(hipMemcpyAsync(to, steps.data(), bytes, hipMemcpyHostToDevice, h_->stream));
+            HIP_OK(hipStreamSynchronize(h_->stream));
+        }
+        used_ += steps.size();
+        return to;
+    }
+
+  private:
+    pl_sv *h_;
+    SweepStep *dev_ = nullptr;
+    size_t used_ = 0, cap_ = 0;
+};
+
 template <class T> struct Engine {
     using V = v2<T>;
     using Scalar = T;
@@ -684,6 +751,82 @@ template <class T> struct Engine {
         }
         HIP_OK(hipStreamSynchronize(h->stream));
         return npasses;
+    }
+
+    // ---- forward passes on register tiles (kernels_pass.hpp) ------------------
+    // Applies a tape; returns the number of launches.  The operations before
+    // one that does not lower are applied before its error leaves, as gate by
+    // gate.  The steps of every pass go through the handle's pinned program
+    // buffer, so nothing waits for the device.
+    int apply_passes(V *sv, const TapeView &t, int max_waves = 8) {
+        SweepSteps builder;
+        std::vector<SweepOp> parts;
+        std::vector<int> woff(t.nops + 1, 0), poff(t.nops + 1, 0);
+        std::exception_ptr refused;
+        for (int i = 0; i < t.nops; i++) {
+            woff[i + 1] = woff[i] + t.nwires[i];
+            poff[i + 1] = poff[i] + t.nparams[i];
+            if (t.ids[i] == -1) {
+                continue;
+            }
+            const int *w = t.wires + woff[i];
+            GroupOp<double> g;
+            try {
+                g = lower_gate<double>(n(), t.ids[i], w, t.nwires[i], t.inverse[i] != 0, t.params + poff[i],
+                                       t.nparams[i]);
+            } catch (...) {
+                refused = std::current_exception();
+                break;
+            }
+            if (g.kind == GroupOp<double>::Noop) {
+                continue;
+            }
+            if (!sweep_expand_op(g, nullptr, SweepTrain{}, parts)) {
+                SweepOp op;
+                op.big = true;
+                op.tape = i;
+                for (int j = 0; j < t.nwires[i]; j++) {
+                    op.extra |= uint64_t{1} << (n() - 1 - w[j]);
+                }
+                parts.assign(1, op);
+            }
+            for (const SweepOp &op : parts) {
+                builder.add(op);
+            }
+        }
+        builder.finish();
+        const auto &steps = builder.steps;
+        int launches = 0;
+        if (!steps.empty()) {
+            constexpr int RB = kPassRegBits;
+            const int lw = std::clamp(n() - 6 - RB, 0, max_waves == 8 ? 3 : 2);
+            const int tb = 6 + lw, bits = std::min(n(), tb + RB), low = std::min(n(), kSweepLow<T>);
+            SweepScheduler sched(n(), bits, low, steps);
+            SweepPass ps;
+            std::vector<SweepStep> prog;
+            ProgramBuffer pb(h, 2 * steps.size());
+            SweepGeom geo{};
+            geo.bits = bits;
+            geo.low = low;
+            while (sched.next(ps)) {
+                launches++;
+                if (ps.big) {
+                    const int i = steps[ps.ops[0]].tape;
+                    gate(sv, t.ids[i], t.wires + woff[i], t.nwires[i], t.inverse[i] != 0, t.params + poff[i],
+                         t.nparams[i]);
+                    continue;
+                }
+                prog.clear();
+                sweep_program(steps, ps, low, tb, RB, prog);
+                std::copy(ps.hb.begin(), ps.hb.end(), geo.hb);
+                HIP_OK(launch_pass<T>(1 << lw, sv, len() >> bits, geo, pb.put(prog), static_cast<int>(prog.size()),
+                                      h->stream));
+            }
+        }
+        if (refused) {
+            std::rethrow_exception(refused);
+        }
+        return launches;
     }
 
     // ---- reductions ----------------------------------------------------------
@@ -1339,6 +1482,10 @@ void defer_gate(pl_sv_t h, int id, const int *wires, int nw, bool inverse, const
     }
 }
 
+// Tapes of at least this many operations run as passes on register tiles;
+// shorter ones gate by gate: KPASS_WHY
+constexpr int kPassMinOps = 4;
+
 // Engine of the handle's precision, exceptions propagate
 template <class F> void dispatch_or_throw(pl_sv_t h, F &&f) {
     flush_deferred(h);
@@ -1385,7 +1532,6 @@ struct SweepTape {
     const double *params;
 };
 
-template <class T> constexpr int kSweepLow = std::is_same_v<T, double> ? 3 : 4; // one 128-byte line
 // States up to this size keep a second lambda, so that every observable group
 // of a pass can run at once; larger ones fill the device group by group.
 constexpr size_t kSweepTwoLambdas = size_t{64} << 20;
@@ -1487,10 +1633,9 @@ void backward_sweep(Engine<T> &E, const SweepTape &t, v2<T> *lam, const std::vec
     V *mu = nullptr;
     auto **dhs = static_cast<V **>(buf(h, kBufSweepStates, K * sizeof(V *)));
     HIP_OK(hipMemcpyAsync(dhs, hs.data(), K * sizeof(V *), hipMemcpyHostToDevice, h->stream));
-    auto *dprog = static_cast<SweepStep *>(buf(h, kBufSweepProg, 2 * steps.size() * sizeof(SweepStep)));
+    ProgramBuffer pb(h, 2 * steps.size());
     std::vector<SweepStep> prog;
-    prog.reserve(2 * steps.size()); // steps and windows; never moves: copies may still read it
-    struct Drain { // nor does it end before them when a call below fails
+    struct Drain { // hs outlives the copy of its pointers when a call below fails
         hipStream_t s;
         ~Drain() { (void)hipStreamSynchronize(s); }
     } drain{h->stream};
@@ -1541,7 +1686,6 @@ void backward_sweep(Engine<T> &E, const SweepTape &t, v2<T> *lam, const std::vec
             }
             continue;
         }
-        const size_t p0 = prog.size();
         size_t mine = 0;
         for (int i : ps.ops) {
             mine += steps[i].train.empty() ? 0 : 1;
@@ -1555,11 +1699,10 @@ void backward_sweep(Engine<T> &E, const SweepTape &t, v2<T> *lam, const std::vec
                 slot_step.push_back(i);
             }
         }
-        sweep_program(steps, ps, low, tb, prog);
-        const int ns = static_cast<int>(prog.size() - p0);
-        HIP_OK(hipMemcpyAsync(dprog + p0, prog.data() + p0, ns * sizeof(SweepStep), hipMemcpyHostToDevice,
-                              h->stream));
-        SweepArgs<T> a{lam, other, dhs, K, 0, 0, ngrp - 1, W, ntiles, {}, dprog + p0, ns, static_cast<int>(mine),
+        prog.clear();
+        sweep_program(steps, ps, low, tb, RB, prog);
+        const int ns = static_cast<int>(prog.size());
+        SweepArgs<T> a{lam, other, dhs, K, 0, 0, ngrp - 1, W, ntiles, {}, pb.put(prog), ns, static_cast<int>(mine),
                        static_cast<int>(slot0), part};
         a.geo.bits = bits;
         a.geo.low = low;
@@ -1576,7 +1719,7 @@ void backward_sweep(Engine<T> &E, const SweepTape &t, v2<T> *lam, const std::vec
     if (!sums.empty()) {
         HIP_OK(hipMemcpyAsync(sums.data(), dsums, sums.size() * sizeof(double), hipMemcpyDeviceToHost, h->stream));
     }
-    HIP_OK(hipStreamSynchronize(h->stream)); // also ends every copy from prog and hs
+    HIP_OK(hipStreamSynchronize(h->stream));
     for (size_t sl = 0; sl < slot_step.size(); sl++) {
         const SweepOp &op = steps[slot_step[sl]];
         for (int k = 0; k < K; k++) {
@@ -1750,6 +1893,12 @@ int pl_sv_destroy(pl_sv_t h) {
         for (void *p : h->pool) {
             (void)hipFree(p);
         }
+        if (h->prog_host) {
+            (void)hipHostFree(h->prog_host);
+        }
+        if (h->prog_ev) {
+            (void)hipEventDestroy(h->prog_ev);
+        }
         (void)hipFree(h->red);
         (void)hipFree(h->staging);
         for (auto &b : h->bufs) {
@@ -1903,6 +2052,10 @@ int pl_sv_apply_ops(pl_sv_t h, int nops, const int *ids, const int *nwires, cons
         });
     }
     return dispatch(h, [&](auto &E) {
+        if (nops >= kPassMinOps) {
+            E.apply_passes(E.psi(), TapeView{nops, ids, nwires, wires, inverse, nparams, params});
+            return;
+        }
         for (int i = 0, wo = 0, po = 0; i < nops; i++) {
             if (ids[i] != -1) {
                 E.gate(E.psi(), ids[i], wires + wo, nwires[i], inverse[i] != 0, params + po,

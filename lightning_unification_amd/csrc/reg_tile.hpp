@@ -58,11 +58,14 @@ __device__ __forceinline__ double rt_sum4(double v0, double v1, double v2, doubl
 __device__ __forceinline__ int rt_row(int r) { return ((r & 1) << 1) | (r >> 1); }
 
 // Local index -> place in the LDS buffer, linear in its bits.  With window bits
-// p .. p + 2, consecutive lanes differ in the local bits around them; the map
-// folds bits 4..7 into the low five so that for every p the first four lane
-// bits give 16 different places mod 16 and the first five 32 mod 32 (doubles:
-// no two lanes of an access share a bank).
-__device__ __forceinline__ uint32_t rt_place(uint32_t e) { return e ^ ((e >> 3) & 30U) ^ ((e >> 6) & 1U); }
+// p .. p + RB - 1, consecutive lanes differ in the local bits around them; the
+// map folds bits 4..8 into the low five so that for windows of three and four
+// neighbouring bits the first four lane bits give 16 places that differ mod 16
+// and the first five 32 mod 32 (all but one case): no two lanes of an access
+// share a bank.  Found by trying every such map.
+__device__ __forceinline__ uint32_t rt_place(uint32_t e) {
+    return e ^ ((e >> 4) & 1U) ^ ((e >> 3) & 4U) ^ (((e >> 6) & 1U) * 10U) ^ (((e >> 7) & 1U) * 28U) ^ ((e >> 4) & 16U);
+}
 
 // thread bits spread over the local bits outside the window
 template <int RB> __device__ __forceinline__ uint32_t rt_thread_part(uint32_t t, uint32_t win) {

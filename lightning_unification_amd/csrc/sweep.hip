@@ -1,8 +1,9 @@
-// The backward sweep's pass kernel, one translation unit per precision
+// The pass kernels of the backward sweep and of forward tapes, one translation unit per precision
 // (PL_SWEEP_DOUBLE), compiled like the tile passes with uniform regions left
 // unstructured: a step's branches are all on scalars, and structuring them
 // makes the compiler copy the register tile at every join.
 #include "kernels_adjoint.hpp"
+#include "kernels_pass.hpp"
 
 namespace plamd {
 
@@ -29,7 +30,27 @@ template <class T> hipError_t launch_sweep(int waves, int kh, bool full, const S
     return waves == 4 ? go(I4{}, I1{}, I0{}) : waves == 2 ? go(I2{}, I1{}, I0{}) : go(I1{}, I1{}, I0{});
 }
 
+template <class T>
+hipError_t launch_pass(int waves, v2<T> *sv, uint64_t ntiles, const SweepGeom &geo, const SweepStep *prog, int nsteps,
+                       hipStream_t s) {
+    auto go = [&](auto nw) {
+        constexpr int NW = decltype(nw)::value;
+        constexpr size_t lds = sizeof(double) << (6 + kPassRegBits + (NW == 8 ? 3 : NW == 4 ? 2 : NW == 2 ? 1 : 0));
+        hipLaunchKernelGGL((k_pass<T, NW>), dim3(static_cast<unsigned>(ntiles)), dim3(64 * NW), lds, s, sv, ntiles, geo,
+                           prog, nsteps);
+        return hipGetLastError();
+    };
+    switch (waves) {
+    case 8: return go(std::integral_constant<int, 8>{});
+    case 4: return go(std::integral_constant<int, 4>{});
+    case 2: return go(std::integral_constant<int, 2>{});
+    default: return go(std::integral_constant<int, 1>{});
+    }
+}
+
 #if PL_SWEEP_DOUBLE
+template hipError_t launch_pass<double>(int, v2<double> *, uint64_t, const SweepGeom &, const SweepStep *, int,
+                                        hipStream_t);
 template hipError_t launch_sweep<double>(int, int, bool, const SweepArgs<double> &, hipStream_t);
 
 hipError_t launch_sweep_sums(const double *partial, int W, unsigned count, double *out, hipStream_t s) {
@@ -37,6 +58,8 @@ hipError_t launch_sweep_sums(const double *partial, int W, unsigned count, doubl
     return hipGetLastError();
 }
 #else
+template hipError_t launch_pass<float>(int, v2<float> *, uint64_t, const SweepGeom &, const SweepStep *, int,
+                                       hipStream_t);
 template hipError_t launch_sweep<float>(int, int, bool, const SweepArgs<float> &, hipStream_t);
 #endif
 

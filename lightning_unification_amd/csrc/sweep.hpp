@@ -454,9 +454,8 @@ class SweepScheduler {
 // followed by the steps it can hold (those whose mixing bit is in the window
 // and which touch no bit of a step held back).  tb: thread bits of the tile;
 // local bits are numbered from the lowest, the first window is the highest RB.
-inline void sweep_program(const std::vector<SweepOp> &steps, const SweepPass &ps, int low, int tb,
+inline void sweep_program(const std::vector<SweepOp> &steps, const SweepPass &ps, int low, int tb, int RB,
                           std::vector<SweepStep> &prog) {
-    constexpr int RB = kSweepRegBits;
     const int bits = tb + RB;
     uint64_t tile = (uint64_t{1} << low) - 1;
     for (int b : ps.hb) {

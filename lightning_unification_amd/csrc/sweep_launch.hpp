@@ -40,9 +40,10 @@ struct SweepStep {
 //   4 Re M00, 5 Re M11, 6 Re(M01 + M10), 7 Im(M01 - M10).
 constexpr int kSweepReal = 4, kSweepFull = 8;
 constexpr int kSweepSlots = 64;    // trainable steps per pass
-constexpr int kSweepMaxBits = 11;  // widest tile
+constexpr int kSweepMaxBits = 13;  // widest tile
 
-constexpr int kSweepRegBits = 3;   // register bits of a tile: 8 amplitudes a thread and state
+constexpr int kSweepRegBits = 3;   // register bits of a sweep tile: 8 amplitudes a thread and state
+constexpr int kPassRegBits = 4;    // of a forward pass's: 16 amplitudes a thread
 
 struct SweepGeom {
     int bits;              // local bits of the state: min(n, the tile's)
@@ -67,6 +68,10 @@ template <class T> struct SweepArgs {
 // One launch of args.ngrp observable groups (kh observables each) with `waves`
 // (1, 2 or 4) wavefronts per tile; full: the complex sums too.
 template <class T> hipError_t launch_sweep(int waves, int kh, bool full, const SweepArgs<T> &args, hipStream_t s);
+// One forward pass (kernels_pass.hpp) of `waves` (1, 2, 4 or 8) wavefronts a tile.
+template <class T>
+hipError_t launch_pass(int waves, v2<T> *sv, uint64_t ntiles, const SweepGeom &geo, const SweepStep *prog, int nsteps,
+                       hipStream_t s);
 // out[v] = sum of partial[v W .. (v + 1) W), v < count
 hipError_t launch_sweep_sums(const double *partial, int W, unsigned count, double *out, hipStream_t s);
 
