@@ -828,7 +828,8 @@ def main():
 
     sv = capi.DeviceStateVector(n, np.complex128)
     for _ in range(args.warmup):
-        sv.apply_tape(tape)
+        for op in tape.ops:  # the timed region's launches, one per gate
+            sv.apply(op[0], op[1], op[2], op[3])
     sv.synchronize()
     log("warmup done")
 

@@ -9,7 +9,11 @@
 // of four bits holds more steps than the sweep's three, and one state leaves
 // the registers for it.  complex64 states are updated in double: a pass rounds
 // each amplitude once.
-// PASS_FIGURES
+// Bound: HBM for shallow passes (1.9 ms a pass of 4 GiB at the copy rate), FP64
+// issue from about twenty steps a pass on.  28 qubits complex128: 19 gates 22.4 ->
+// 3.5 ms against a launch each; 220 gates 28.2 -> 17.6 ms against the
+// wavefront tiles of kernels_tile.hpp, whose 2^11 amplitudes take 16 passes
+// where 2^13 take 7.  13 qubits complex64, 90 gates: 275 -> 65 us a call.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -24,7 +28,7 @@ template <class T, int NW>
 __global__ __launch_bounds__(64 * NW, 4) void k_pass(v2<T> *__restrict__ sv, uint64_t ntiles, const SweepGeom geo,
                                                      const SweepStep *__restrict__ prog, int nsteps) {
     constexpr int RB = kPassRegBits, R = 1 << RB;
-    static_assert(RB == 4, "the steps' switches name four register bits");
+    static_assert(RB == 4, "rt_pairs4 names four register bits");
     constexpr int TB = 6 + (NW == 8 ? 3 : NW == 4 ? 2 : NW == 2 ? 1 : 0);
     constexpr uint32_t HOME = TB | (TB + 1) << 4 | (TB + 2) << 8 | (TB + 3) << 12;
     extern __shared__ unsigned char smem_raw[];
@@ -96,50 +100,56 @@ __global__ __launch_bounds__(64 * NW, 4) void k_pass(v2<T> *__restrict__ sv, uin
             for (int i = 0; i < 4; i++) {
                 u[i] = st.u[i];
             }
-            auto dense = [&](auto jt) {
-                constexpr int J = decltype(jt)::value;
+            auto each = [&](auto apply) {
+                rt_pairs4(st.j, [&](auto jt, auto j2t) {
+                    constexpr int J = decltype(jt)::value, J2 = decltype(j2t)::value;
 #pragma unroll
-                for (int p = 0; p < R / 2; p++) {
-                    const int i0 = ((p >> J) << (J + 1)) | (p & ((1 << J) - 1)), i1 = i0 | (1 << J);
-                    if ((static_cast<uint32_t>(i0) & rm) == rv) {
-                        rt_apply2(lanes, u, x[0][i0], x[0][i1]);
+                    for (int p = 0; p < R / 2; p++) {
+                        const int i0 = rt_member<J>(p), i1 = rt_partner<J, J2>(i0);
+                        if ((static_cast<uint32_t>(i0) & rm) == rv) {
+                            apply(x[0][i0], x[0][i1]);
+                        }
                     }
-                }
+                });
             };
-            switch (st.j) {
-            case 0: dense(std::integral_constant<int, 0>{}); break;
-            case 1: dense(std::integral_constant<int, 1>{}); break;
-            case 2: dense(std::integral_constant<int, 2>{}); break;
-            default: dense(std::integral_constant<int, 3>{}); break;
+            if (st.form == kSweepReal2) {
+                each([&](double2 &a, double2 &b) { rt_apply2_real(lanes, u, a, b); });
+            } else if (st.form == kSweepCross2) {
+                each([&](double2 &a, double2 &b) { rt_apply2_cross(lanes, u, a, b); });
+            } else {
+                each([&](double2 &a, double2 &b) { rt_apply2(lanes, u, a, b); });
             }
         } else if (kind == kSweepFlip) {
-            auto flip = [&](auto jt) {
-                constexpr int J = decltype(jt)::value;
+            rt_pairs4(st.j, [&](auto jt, auto j2t) {
+                constexpr int J = decltype(jt)::value, J2 = decltype(j2t)::value;
 #pragma unroll
                 for (int p = 0; p < R / 2; p++) {
-                    const int i0 = ((p >> J) << (J + 1)) | (p & ((1 << J) - 1)), i1 = i0 | (1 << J);
+                    const int i0 = rt_member<J>(p), i1 = rt_partner<J, J2>(i0);
                     if ((static_cast<uint32_t>(i0) & rm) == rv) {
                         rt_exchange(lanes, x[0][i0], x[0][i1]);
                     }
                 }
-            };
-            switch (st.j) {
-            case 0: flip(std::integral_constant<int, 0>{}); break;
-            case 1: flip(std::integral_constant<int, 1>{}); break;
-            case 2: flip(std::integral_constant<int, 2>{}); break;
-            default: flip(std::integral_constant<int, 3>{}); break;
-            }
+            });
         } else { // kSweepDiag
             const uint32_t rp = st.rp;
             const uint32_t tpar = (__popc(tid & st.lp) + __popcll(base & st.op)) & 1U;
             const dcx<double> u0 = st.u[0], u1 = st.u[1];
             const dcx<double> ue{tpar ? u1.r : u0.r, tpar ? u1.i : u0.i}, uo{tpar ? u0.r : u1.r, tpar ? u0.i : u1.i};
+            if (rp == 0) { // one phase a lane
 #pragma unroll
-            for (int r = 0; r < R; r++) {
-                if ((static_cast<uint32_t>(r) & rm) == rv) {
-                    const bool odd = __popc(static_cast<uint32_t>(r) & rp) & 1U; // uniform
-                    const dcx<double> u{odd ? uo.r : ue.r, odd ? uo.i : ue.i};
-                    rt_into(lanes, x[0][r], u.r, -u.i * x[0][r].y, u.i * x[0][r].x);
+                for (int r = 0; r < R; r++) {
+                    if ((static_cast<uint32_t>(r) & rm) == rv) {
+                        rt_into(lanes, x[0][r], ue.r, -ue.i * x[0][r].y, ue.i * x[0][r].x);
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int r = 0; r < R; r++) {
+                    if ((static_cast<uint32_t>(r) & rm) == rv) {
+                        const bool odd = __popc(static_cast<uint32_t>(r) & rp) & 1U; // uniform
+                        const dcx<double> u{odd ? uo.r : ue.r, odd ? uo.i : ue.i};
+                        rt_into(lanes, x[0][r], u.r, -u.i * x[0][r].y, u.i * x[0][r].x);
+                    }
                 }
             }
         }

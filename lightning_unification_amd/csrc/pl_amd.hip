@@ -192,9 +192,14 @@ class ProgramBuffer {
         if (!h->prog_ev) {
             HIP_OK(hipEventCreateWithFlags(&h->prog_ev, hipEventDisableTiming));
         }
-        dev_ = static_cast<SweepStep *>(buf(h, kBufSweepProg, std::max<size_t>(bytes, 1 << 16)));
-        cap_ = steps;
+        try {
+            dev_ = static_cast<SweepStep *>(buf(h, kBufSweepProg, std::max<size_t>(bytes, 1 << 16)));
+            cap_ = steps;
+        } catch (const DeviceError &) { // the device is full: ok() is false
+            (void)hipGetLastError();
+        }
     }
+    bool ok() const { return dev_ != nullptr; }
     ~ProgramBuffer() {
         if (used_ > 0 && h_->prog_host) {
             h_->prog_busy = hipEventRecord(h_->prog_ev, h_->stream) == hipSuccess;
@@ -623,6 +628,7 @@ template <class T> struct Engine {
     // wins (fewer passes outweigh the lower occupancy)
     static constexpr int kTileDefaultBits = std::is_same_v<T, double> ? 11 : 12;
     static constexpr int kTileMaxBitsC128 = 11;
+    static constexpr int kTileFloatQubits = 23;
     static constexpr int kTileDefaultLow = std::is_same_v<T, double> ? 3 : 4;
 
     // Applies a tape as tile passes (tile.hpp); returns the number of launches.
@@ -637,6 +643,18 @@ template <class T> struct Engine {
             poff[i + 1] = poff[i] + t.nparams[i];
         }
         if (k == 0) {
+            // the default is the faster executor: passes on workgroup tiles
+            // (apply_passes), except for complex64 states of
+            // kTileFloatQubits or more, where this one's FP32 arithmetic and
+            // 2^12-amplitude wavefront tiles win (28 qubits, 185 gates: 11.8
+            // against 16.5 ms; 20 qubits, 133 gates: 0.45 against 0.26 ms;
+            // complex128 at 28 qubits: 24.2 against 16.4 ms)
+            if (std::is_same_v<T, double> || n() < kTileFloatQubits) {
+                const int launches = apply_passes(sv, t);
+                if (launches >= 0) {
+                    return launches;
+                }
+            }
             if (n() < kTpMinBits) {
                 int launches = 0;
                 for (int i = 0; i < t.nops; i++) {
@@ -754,11 +772,11 @@ template <class T> struct Engine {
     }
 
     // ---- forward passes on register tiles (kernels_pass.hpp) ------------------
-    // Applies a tape; returns the number of launches.  The operations before
-    // one that does not lower are applied before its error leaves, as gate by
-    // gate.  The steps of every pass go through the handle's pinned program
-    // buffer, so nothing waits for the device.
-    int apply_passes(V *sv, const TapeView &t, int max_waves = 8) {
+    // Applies a tape; returns the number of launches, or -1, with nothing done,
+    // where there is no memory for the passes' programs.  The operations
+    // before one that does not lower are applied before its error leaves, as
+    // gate by gate.  Nothing here waits for the device's passes.
+    int apply_passes(V *sv, const TapeView &t) {
         SweepSteps builder;
         std::vector<SweepOp> parts;
         std::vector<int> woff(t.nops + 1, 0), poff(t.nops + 1, 0);
@@ -799,12 +817,15 @@ template <class T> struct Engine {
         int launches = 0;
         if (!steps.empty()) {
             constexpr int RB = kPassRegBits;
-            const int lw = std::clamp(n() - 6 - RB, 0, max_waves == 8 ? 3 : 2);
+            const int lw = std::clamp(n() - 6 - RB, 0, 3); // the widest tile the state fills
             const int tb = 6 + lw, bits = std::min(n(), tb + RB), low = std::min(n(), kSweepLow<T>);
             SweepScheduler sched(n(), bits, low, steps);
             SweepPass ps;
             std::vector<SweepStep> prog;
-            ProgramBuffer pb(h, 2 * steps.size());
+            ProgramBuffer pb(h, 2 * steps.size()); // a step and its window
+            if (!pb.ok()) {
+                return -1;
+            }
             SweepGeom geo{};
             geo.bits = bits;
             geo.low = low;
@@ -817,7 +838,7 @@ template <class T> struct Engine {
                     continue;
                 }
                 prog.clear();
-                sweep_program(steps, ps, low, tb, RB, prog);
+                sweep_program(steps, ps, low, tb, RB, true, prog);
                 std::copy(ps.hb.begin(), ps.hb.end(), geo.hb);
                 HIP_OK(launch_pass<T>(1 << lw, sv, len() >> bits, geo, pb.put(prog), static_cast<int>(prog.size()),
                                       h->stream));
@@ -1482,8 +1503,10 @@ void defer_gate(pl_sv_t h, int id, const int *wires, int nw, bool inverse, const
     }
 }
 
-// Tapes of at least this many operations run as passes on register tiles;
-// shorter ones gate by gate: KPASS_WHY
+// Tapes of at least this many operations run as passes on register tiles
+// (apply_passes); shorter ones gate by gate, a launch each and no program to
+// upload.  Three gates at 6 qubits: 34 us by either; five at 9 qubits 40 us
+// gate by gate, 38 us as a pass; 19 at 28 qubits 22.5 and 3.5 ms.
 constexpr int kPassMinOps = 4;
 
 // Engine of the handle's precision, exceptions propagate
@@ -1633,7 +1656,10 @@ void backward_sweep(Engine<T> &E, const SweepTape &t, v2<T> *lam, const std::vec
     V *mu = nullptr;
     auto **dhs = static_cast<V **>(buf(h, kBufSweepStates, K * sizeof(V *)));
     HIP_OK(hipMemcpyAsync(dhs, hs.data(), K * sizeof(V *), hipMemcpyHostToDevice, h->stream));
-    ProgramBuffer pb(h, 2 * steps.size());
+    ProgramBuffer pb(h, 4 * steps.size()); // a step with two flips, and its window
+    if (!pb.ok()) {
+        throw DeviceError("no device memory for the sweep's programs");
+    }
     std::vector<SweepStep> prog;
     struct Drain { // hs outlives the copy of its pointers when a call below fails
         hipStream_t s;
@@ -1700,7 +1726,7 @@ void backward_sweep(Engine<T> &E, const SweepTape &t, v2<T> *lam, const std::vec
             }
         }
         prog.clear();
-        sweep_program(steps, ps, low, tb, RB, prog);
+        sweep_program(steps, ps, low, tb, RB, false, prog);
         const int ns = static_cast<int>(prog.size());
         SweepArgs<T> a{lam, other, dhs, K, 0, 0, ngrp - 1, W, ntiles, {}, pb.put(prog), ns, static_cast<int>(mine),
                        static_cast<int>(slot0), part};
@@ -2052,8 +2078,8 @@ int pl_sv_apply_ops(pl_sv_t h, int nops, const int *ids, const int *nwires, cons
         });
     }
     return dispatch(h, [&](auto &E) {
-        if (nops >= kPassMinOps) {
-            E.apply_passes(E.psi(), TapeView{nops, ids, nwires, wires, inverse, nparams, params});
+        if (nops >= kPassMinOps &&
+            E.apply_passes(E.psi(), TapeView{nops, ids, nwires, wires, inverse, nparams, params}) >= 0) {
             return;
         }
         for (int i = 0, wo = 0, po = 0; i < nops; i++) {

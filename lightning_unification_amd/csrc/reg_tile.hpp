@@ -12,6 +12,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "kernels_gate.hpp"
 
 namespace plamd {
@@ -120,6 +122,37 @@ __device__ __forceinline__ void rt_exchange(uint64_t m, double2 &a, double2 &b) 
         : "s"(m));
 }
 
+// Partner of register index i0 in the pairs that differ in bit J, or in J and J2.
+template <int J, int J2> __device__ __forceinline__ constexpr int rt_partner(int i0) {
+    return i0 ^ (1 << J) ^ (J2 >= 0 ? 1 << J2 : 0);
+}
+// The p-th register index with bit J clear.
+template <int J> __device__ __forceinline__ constexpr int rt_member(int p) {
+    return ((p >> J) << (J + 1)) | (p & ((1 << J) - 1));
+}
+// f(J, J2) for a step's j (SweepStep) with four register bits: a single one
+// (J2 = -1) or two.
+template <class F> __device__ __forceinline__ void rt_pairs4(int j, F &&f) {
+    using std::integral_constant;
+    integral_constant<int, -1> none;
+    integral_constant<int, 0> b0;
+    integral_constant<int, 1> b1;
+    integral_constant<int, 2> b2;
+    integral_constant<int, 3> b3;
+    switch (j) {
+    case 0: f(b0, none); break;
+    case 1: f(b1, none); break;
+    case 2: f(b2, none); break;
+    case 3: f(b3, none); break;
+    case 4: f(b0, b1); break;
+    case 5: f(b0, b2); break;
+    case 6: f(b0, b3); break;
+    case 7: f(b1, b2); break;
+    case 8: f(b1, b3); break;
+    default: f(b2, b3); break;
+    }
+}
+
 // (a, b) <- u (a, b) in the lanes of m, 16 multiply-adds
 __device__ __forceinline__ void rt_apply2(uint64_t m, const dcx<double> *u, double2 &a, double2 &b) {
     const double t0 = rt_fma(-u[0].i, a.y, rt_fma(u[1].r, b.x, -u[1].i * b.y));
@@ -129,13 +162,13 @@ __device__ __forceinline__ void rt_apply2(uint64_t m, const dcx<double> *u, doub
     rt_into2(m, a, b, u[0].r, u[3].r, t0, t1, t2, t3);
 }
 
-// (a, b) <- u (a, b), left to the compiler: for code without a step's branches
-__device__ __forceinline__ void rt_mul2(const dcx<double> *u, double2 &a, double2 &b) {
-    const double ax = a.x, ay = a.y, bx = b.x, by = b.y;
-    a.x = rt_fma(u[0].r, ax, rt_fma(-u[0].i, ay, rt_fma(u[1].r, bx, -u[1].i * by)));
-    a.y = rt_fma(u[0].r, ay, rt_fma(u[0].i, ax, rt_fma(u[1].r, by, u[1].i * bx)));
-    b.x = rt_fma(u[2].r, ax, rt_fma(-u[2].i, ay, rt_fma(u[3].r, bx, -u[3].i * by)));
-    b.y = rt_fma(u[2].r, ay, rt_fma(u[2].i, ax, rt_fma(u[3].r, by, u[3].i * bx)));
+// the same for a real u, and for one with a real diagonal and imaginary others:
+// 8 multiply-adds
+__device__ __forceinline__ void rt_apply2_real(uint64_t m, const dcx<double> *u, double2 &a, double2 &b) {
+    rt_into2(m, a, b, u[0].r, u[3].r, u[1].r * b.x, u[1].r * b.y, u[2].r * a.x, u[2].r * a.y);
+}
+__device__ __forceinline__ void rt_apply2_cross(uint64_t m, const dcx<double> *u, double2 &a, double2 &b) {
+    rt_into2(m, a, b, u[0].r, u[3].r, -u[1].i * b.y, u[1].i * b.x, -u[2].i * a.y, u[2].i * a.x);
 }
 
 // The S states of a tile moved from window `from` to window `to` through

@@ -2,11 +2,11 @@
 // operation first, becomes steps; steps become passes; a pass becomes a
 // program of register windows.
 //
-// Step: a 2x2 on one bit, or phases by the parity of some bits, where other
-// bits have given values.  Every gate of at most four members is a product of
-// such steps and CNOTs: members that differ in several bits are brought
-// together by CNOTs from one of those bits to the others (IsingXX is RX
-// between two CNOTs), undone after.  A step merges into the last one that
+// Step: a 2x2 on pairs that differ in one bit or two, or phases by the parity
+// of some bits, where other bits have given values.  Every gate of at most four
+// members is one or two such steps (IsingXX: one on pairs that differ in both
+// bits); members that differ in more bits (DoubleExcitation) are brought
+// together by CNOTs from one of those bits to the others, undone after.  A step merges into the last one that
 // touched any of its bits when that has the same geometry: nothing in between
 // touches those bits, so it commutes back.  The merged step keeps the product
 // U^dagger = U_m^dagger .. U_1^dagger (U_1 the tape's last) and, for the j-th
@@ -39,17 +39,18 @@ struct SweepTrain {
 struct SweepOp { // one step before it is placed on a tile
     bool big = false;  // applied state by state: operation `tape` of the tape
     int tape = -1;
-    uint64_t bit = 0;  // the bit a 2x2 mixes; 0: phases only
+    uint64_t bit = 0;  // the bit a 2x2 mixes (the lower of two); 0: phases only
+    uint64_t bit2 = 0; // a second bit its pairs differ in; tests are on the member with `bit` clear
     uint64_t par = 0;  // phases: u[0] or u[3] by the parity of these bits
     uint64_t test = 0, value = 0; // bits tested, and their values
     std::complex<double> u[4] = {1, 0, 0, 1};
     std::vector<SweepTrain> train;
 
-    uint64_t touch() const { return bit | par | test | extra; }
+    uint64_t touch() const { return bit | bit2 | par | test | extra; }
     uint64_t extra = 0; // big operations: all their bits
-    uint64_t need() const { return bit; }
+    uint64_t need() const { return bit | bit2; }
     bool same_place(const SweepOp &o) const {
-        return !big && !o.big && bit == o.bit && par == o.par && test == o.test && value == o.value;
+        return !big && !o.big && bit == o.bit && bit2 == o.bit2 && par == o.par && test == o.test && value == o.value;
     }
     bool diagonal() const { return u[1] == 0.0 && u[2] == 0.0; }
     bool identity() const { return diagonal() && u[0] == 1.0 && u[3] == 1.0; }
@@ -142,9 +143,9 @@ inline bool sweep_expand_op(const GroupOp<double> &ud, const GroupOp<double> *g,
         out.push_back(proto);
         return true;
     }
-    // CNOTs from bit t to the other bits of `bits`
+    // CNOTs from bit t to `bits`
     auto frame = [&](uint64_t t, uint64_t bits) {
-        for (uint64_t b = bits & ~t; b; b &= b - 1) {
+        for (uint64_t b = bits; b; b &= b - 1) {
             SweepOp c;
             c.bit = b & (~b + 1);
             c.test = c.value = t;
@@ -153,17 +154,17 @@ inline bool sweep_expand_op(const GroupOp<double> &ud, const GroupOp<double> *g,
             out.push_back(c);
         }
     };
-    // the 2x2 of members p and q, which differ in the bits `mix`, t among
-    // them, inside the frame of t and mix
-    auto pair = [&](int p, int q, uint64_t t, uint64_t mix) {
+    // the 2x2 of members p and q, which differ in t, t2 and bits brought
+    // together by the frame of t (which leaves the member with t clear alone)
+    auto pair = [&](int p, int q, uint64_t t, uint64_t t2) {
         if (mem[p] & t) {
             std::swap(p, q);
         }
         SweepOp s = proto;
         s.bit = t;
+        s.bit2 = t2;
         s.test = touch & ~t;
-        s.value = mem[p] & s.test; // member p has t clear: the frame leaves it alone
-        (void)mix;
+        s.value = mem[p] & s.test;
         s.u[0] = U(p, p);
         s.u[1] = U(p, q);
         s.u[2] = U(q, p);
@@ -178,10 +179,10 @@ inline bool sweep_expand_op(const GroupOp<double> &ud, const GroupOp<double> *g,
         return s;
     };
     if (M == 2) {
-        const uint64_t t = vary & (~vary + 1);
-        frame(t, vary);
+        const uint64_t t = vary & (~vary + 1), up = vary & ~t, t2 = up & (~up + 1);
+        frame(t, up & ~t2);
         const size_t nf = out.size();
-        out.push_back(pair(0, 1, t, vary));
+        out.push_back(pair(0, 1, t, t2));
         for (size_t j = 0; j < nf; j++) {
             const SweepOp c = out[j];
             out.push_back(c);
@@ -230,11 +231,9 @@ inline bool sweep_expand_op(const GroupOp<double> &ud, const GroupOp<double> *g,
         }
         mix = lo;
     }
-    const uint64_t t = mix & (~mix + 1);
-    frame(t, mix);
-    const size_t nf = out.size();
+    const uint64_t t = mix & (~mix + 1), t2 = mix & ~t;
     const int a = at(0), b = at(mix), c = at(t == mix ? vary & ~mix : hi), d = at(t == mix ? vary : lo);
-    SweepOp s0 = pair(a, b, t, mix), s1 = pair(c, d, t, mix);
+    SweepOp s0 = pair(a, b, t, t2), s1 = pair(c, d, t, t2);
     auto same = [](const SweepOp &x, const SweepOp &y) {
         bool eq = std::equal(x.u, x.u + 4, y.u) && x.train.size() == y.train.size();
         for (size_t j = 0; eq && j < x.train.size(); j++) {
@@ -249,10 +248,6 @@ inline bool sweep_expand_op(const GroupOp<double> &ud, const GroupOp<double> *g,
     } else {
         out.push_back(s0);
         out.push_back(s1);
-    }
-    for (size_t j = 0; j < nf; j++) {
-        const SweepOp x = out[j];
-        out.push_back(x);
     }
     return true;
 }
@@ -296,13 +291,13 @@ class SweepSteps {
             if (!s.big && s.identity() && s.train.empty()) {
                 continue;
             }
-            bool diag = !s.big && s.bit && s.diagonal();
+            bool diag = !s.big && s.bit && s.diagonal() && !(s.test & s.bit2);
             for (const auto &t : s.train) {
                 diag = diag && t.w01 == 0.0;
             }
             if (diag) {
                 s.par = s.bit;
-                s.bit = 0;
+                s.bit = s.bit2 = 0;
             }
             kept.push_back(std::move(s));
         }
@@ -454,7 +449,10 @@ class SweepScheduler {
 // followed by the steps it can hold (those whose mixing bit is in the window
 // and which touch no bit of a step held back).  tb: thread bits of the tile;
 // local bits are numbered from the lowest, the first window is the highest RB.
-inline void sweep_program(const std::vector<SweepOp> &steps, const SweepPass &ps, int low, int tb, int RB,
+// two: the kernel takes pairs that differ in two register bits (k_pass); else
+// such a step runs on its lower bit between CNOTs from it to the other
+// (k_sweep, whose registers the further pair patterns would not fit).
+inline void sweep_program(const std::vector<SweepOp> &steps, const SweepPass &ps, int low, int tb, int RB, bool two,
                           std::vector<SweepStep> &prog) {
     const int bits = tb + RB;
     uint64_t tile = (uint64_t{1} << low) - 1;
@@ -509,10 +507,18 @@ inline void sweep_program(const std::vector<SweepOp> &steps, const SweepPass &ps
         auto cast = [](const std::complex<double> &z) { return dcx<double>{z.real(), z.imag()}; };
         if (s.bit) {
             d.kind = s.flip() && s.train.empty() ? kSweepFlip : kSweepDense;
-            d.j = __builtin_ctz(reg(local(s.bit)));
+            const int j1 = __builtin_ctz(reg(local(s.bit)));
+            d.j = j1;
+            if (s.bit2 && two) { // the pairs (0,1) (0,2) .. (1,2) .. of register bits, after the single ones
+                const int j2 = __builtin_ctz(reg(local(s.bit2)));
+                d.j = RB + j1 * (2 * RB - j1 - 1) / 2 + (j2 - j1 - 1);
+            }
             for (int j = 0; j < 4; j++) {
                 d.u[j] = cast(s.u[j]);
             }
+            const bool real = s.u[0].imag() == 0 && s.u[1].imag() == 0 && s.u[2].imag() == 0 && s.u[3].imag() == 0;
+            const bool cross = s.u[0].imag() == 0 && s.u[1].real() == 0 && s.u[2].real() == 0 && s.u[3].imag() == 0;
+            d.form = real ? kSweepReal2 : cross ? kSweepCross2 : kSweepFull2;
         } else {
             d.kind = kSweepDiag;
             d.op = s.par & ~tile;
@@ -521,7 +527,18 @@ inline void sweep_program(const std::vector<SweepOp> &steps, const SweepPass &ps
             d.u[0] = cast(s.u[0]);
             d.u[1] = cast(s.u[3]);
         }
+        SweepStep f{};
+        if (s.bit2 && !two) {
+            f.kind = kSweepFlip;
+            f.slot = -1;
+            f.j = __builtin_ctz(reg(local(s.bit2)));
+            f.rm = f.rv = reg(local(s.bit));
+            prog.push_back(f);
+        }
         prog.push_back(d);
+        if (s.bit2 && !two) {
+            prog.push_back(f);
+        }
     };
     while (!pending.empty()) {
         // steps the window w would take; claim: w grows to RB bits in step order

@@ -12,15 +12,21 @@ namespace plamd {
 
 enum SweepKind : int {
     kSweepWindow = 0, // other local bits become register bits
-    kSweepDense,      // a 2x2 on register bit j
-    kSweepFlip,       // an X on register bit j (CNOT, Toffoli)
+    kSweepDense,      // a 2x2 on the pairs of j
+    kSweepFlip,       // the pairs of j exchanged (CNOT, Toffoli, SWAP)
     kSweepDiag,       // phase u[0] or u[1] by the parity of masked bits
 };
+
+// Entries of a kSweepDense step's 2x2 that vanish: none; the imaginary parts (RY,
+// Hadamard); the diagonal's imaginary and the others' real parts (RX, IsingXX).
+enum SweepForm : int { kSweepFull2 = 0, kSweepReal2, kSweepCross2 };
 
 // One step on a tile whose local index is split into register bits (the
 // window) and thread bits (the others, ascending).  It acts where all tested
 // bits have their values: (register index & rm) == rv, (thread & lm) == lv and
-// (bits outside the tile & omask) == oval.  kSweepDiag: the phase is u[parity
+// (bits outside the tile & omask) == oval, of a pair at the member with the lower
+// bit clear.  j: the pairs differ in register bit j (j < RB, the number of
+// register bits), or in two: the j - RB-th of (0,1) (0,2) .. (1,2) ..  kSweepDiag: the phase is u[parity
 // of register & rp, thread & lp and outside & op].  kSweepWindow: rp holds the
 // new window's positions, four bits each.
 struct SweepStep {
@@ -28,7 +34,7 @@ struct SweepStep {
     int j;
     uint32_t rm, rv, lm, lv, rp, lp;
     int slot; // accumulation slot of the pass, -1: not trainable
-    int pad;
+    int form; // kSweepDense: SweepForm
     uint64_t omask, oval, op;
     dcx<double> u[4];
 };
