@@ -231,6 +231,10 @@ struct pl_sv {
     size_t prog_host_bytes = 0;
     hipEvent_t prog_ev = nullptr;
     bool prog_busy = false; // prog_ev is recorded behind copies from prog_host
+    // small pinned area, host memory the device writes results to and tables
+    // are uploaded from (io_area)
+    void *io_host = nullptr;
+    bool io_refused = false;
     // gates queued while deferral is on (pl_sv_set_deferred), in the tape
     // encoding of pl_sv_apply_ops; applied as tile passes before anything
     // else reads or changes the state
@@ -284,6 +288,20 @@ inline void *buf(pl_sv *h, Buf purpose, size_t bytes) {
     return b.first;
 }
 
+// The handle's pinned area (kIoBytes), nullptr where none can be had.  Used
+// within one call that ends by waiting for the stream.
+constexpr size_t kIoBytes = size_t{64} << 10;
+inline unsigned char *io_area(pl_sv *h) {
+    if (!h->io_host && !h->io_refused) {
+        if (hipHostMalloc(&h->io_host, kIoBytes, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            h->io_host = nullptr;
+            h->io_refused = true;
+        }
+    }
+    return static_cast<unsigned char *>(h->io_host);
+}
+
 inline double *reduce_buf(pl_sv *h, size_t bytes) {
     if (h->red_bytes < bytes) {
         if (h->red) {
@@ -297,9 +315,8 @@ inline double *reduce_buf(pl_sv *h, size_t bytes) {
     return h->red;
 }
 
-// Copy host bytes to the handle's device staging area and wait for the copy,
-// so the host buffer may be released as soon as this returns.
-inline void *stage(pl_sv *h, const void *src, size_t bytes) {
+// The handle's device staging area, at least `bytes` long.
+inline void *staging_area(pl_sv *h, size_t bytes) {
     if (h->staging_bytes < bytes) {
         HIP_OK(hipStreamSynchronize(h->stream));
         if (h->staging) {
@@ -310,9 +327,16 @@ inline void *stage(pl_sv *h, const void *src, size_t bytes) {
         HIP_OK(hipMalloc(&h->staging, sz));
         h->staging_bytes = sz;
     }
-    HIP_OK(hipMemcpyAsync(h->staging, src, bytes, hipMemcpyHostToDevice, h->stream));
-    HIP_OK(hipStreamSynchronize(h->stream));
     return h->staging;
+}
+
+// Copy host bytes to the staging area and wait for the copy, so the host
+// buffer may be released as soon as this returns.
+inline void *stage(pl_sv *h, const void *src, size_t bytes) {
+    void *to = staging_area(h, bytes);
+    HIP_OK(hipMemcpyAsync(to, src, bytes, hipMemcpyHostToDevice, h->stream));
+    HIP_OK(hipStreamSynchronize(h->stream));
+    return to;
 }
 
 } // namespace plamd

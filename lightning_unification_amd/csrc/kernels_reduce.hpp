@@ -137,6 +137,53 @@ __global__ __launch_bounds__(kBlock) void k_pauli_expval(const v2<T> *__restrict
     }
 }
 
+// Pauli sum over a small state in one workgroup: the terms travel in the kernel
+// arguments, the state is read once into LDS, and the sum goes to `out`, which
+// may be host memory, so a call is one launch and one wait.  The tile passes
+// (k_pauli_tile) need a table upload, a reduction launch and a read-back, which
+// at 6 qubits were 45 of an expectation's 55 us.  Bound: the launch; the
+// arithmetic is a few multiply-adds per amplitude and term.
+constexpr int kSmallPauliQubits = 12;  // 64 KiB of complex128 in LDS
+constexpr int kSmallPauliTerms = 128;  // 2 KiB of arguments
+constexpr uint64_t kSmallPauliWork = uint64_t{1} << 16; // amplitudes times terms: about 10 us of one workgroup
+constexpr int kSmallPauliThreads = 512;
+struct SmallPauliTerm {
+    double coeff;
+    uint16_t x, zy;
+    uint32_t ny;
+};
+struct SmallPauliSum {
+    int n;
+    SmallPauliTerm t[kSmallPauliTerms];
+};
+template <class T>
+__global__ __launch_bounds__(kSmallPauliThreads) void k_pauli_small(const v2<T> *__restrict__ sv, uint32_t len,
+                                                                    const SmallPauliSum sum, double2 *out) {
+    extern __shared__ unsigned char smem_raw[];
+    v2<T> *psi = reinterpret_cast<v2<T> *>(smem_raw);
+    for (uint32_t i = threadIdx.x; i < len; i += kSmallPauliThreads) {
+        psi[i] = sv[i];
+    }
+    __syncthreads();
+    double acc = 0;
+    for (uint32_t i = threadIdx.x; i < len; i += kSmallPauliThreads) {
+        const v2<T> a = psi[i];
+        for (int k = 0; k < sum.n; k++) {
+            const SmallPauliTerm t = sum.t[k];
+            const v2<T> c = psi[i ^ t.x];
+            // Re[(-i)^ny conj(a) c]
+            double v = (t.ny & 1) ? double(a.x) * double(c.y) - double(a.y) * double(c.x)
+                                  : double(a.x) * double(c.x) + double(a.y) * double(c.y);
+            const bool minus = ((__popc(i & t.zy) & 1) != 0) != ((t.ny & 2) != 0);
+            acc += t.coeff * (minus ? -v : v);
+        }
+    }
+    const double2 r = block_sum2<kSmallPauliThreads>(double2{acc, 0});
+    if (threadIdx.x == 0) {
+        out[0] = r;
+    }
+}
+
 // dst[i] (+)= c * (-i)^ny * (-1)^popcount(i & zy) * src[i ^ x]
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_apply_pauli(const v2<T> *__restrict__ src,

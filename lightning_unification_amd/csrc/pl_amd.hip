@@ -885,6 +885,22 @@ template <class T> struct Engine {
     double pauli_expval(const V *sv, const std::vector<PauliWord> &words,
                         const std::vector<double> &coeffs, unsigned char *ext = nullptr,
                         size_t ext_bytes = 0) {
+        unsigned char *io = ext ? nullptr : io_area(h); // the result's place, then the tables'
+        if (io && n() <= kSmallPauliQubits && words.size() <= static_cast<size_t>(kSmallPauliTerms) &&
+            len() * words.size() <= kSmallPauliWork) {
+            SmallPauliSum sum{};
+            for (size_t t = 0; t < words.size(); t++) {
+                sum.t[sum.n++] = SmallPauliTerm{coeffs[t], static_cast<uint16_t>(words[t].x),
+                                                static_cast<uint16_t>(words[t].zy),
+                                                static_cast<uint32_t>(words[t].ny & 3)};
+            }
+            auto *out = reinterpret_cast<double2 *>(io);
+            hipLaunchKernelGGL((k_pauli_small<T>), dim3(1), dim3(kSmallPauliThreads), len() * sizeof(V), h->stream, sv,
+                               static_cast<uint32_t>(len()), sum, out);
+            HIP_OK(hipGetLastError());
+            HIP_OK(hipStreamSynchronize(h->stream));
+            return out->x;
+        }
         std::map<uint64_t, std::vector<PauliTerm>> groups;
         for (size_t t = 0; t < words.size(); t++) {
             groups[words[t].x].push_back(PauliTerm{words[t].zy, coeffs[t], words[t].ny & 3, 0});
@@ -1029,7 +1045,14 @@ template <class T> struct Engine {
             dev = ext;
             part = reinterpret_cast<double2 *>(ext + part_off);
         } else {
-            dev = static_cast<unsigned char *>(stage(h, blob.data(), blob.size()));
+            constexpr size_t at = 256; // behind the result
+            if (io && at + blob.size() <= kIoBytes) {
+                std::memcpy(io + at, blob.data(), blob.size());
+                dev = static_cast<unsigned char *>(staging_area(h, blob.size()));
+                HIP_OK(hipMemcpyAsync(dev, io + at, blob.size(), hipMemcpyHostToDevice, h->stream));
+            } else {
+                dev = static_cast<unsigned char *>(stage(h, blob.data(), blob.size()));
+            }
             part = reinterpret_cast<double2 *>(reduce_buf(h, part_bytes));
         }
         const auto *dgroups = reinterpret_cast<const PauliTileGroup *>(dev);
@@ -1079,6 +1102,13 @@ template <class T> struct Engine {
                                part + total);
             HIP_OK(hipGetLastError());
             total += grid;
+        }
+        if (io) {
+            auto *out = reinterpret_cast<double2 *>(io);
+            hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(kBlock), 0, h->stream, part, total, out);
+            HIP_OK(hipGetLastError());
+            HIP_OK(hipStreamSynchronize(h->stream));
+            return out->x;
         }
         hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(kBlock), 0, h->stream, part, total,
                            part + nlaunch * kReduceBlocks);
@@ -1921,6 +1951,9 @@ int pl_sv_destroy(pl_sv_t h) {
         }
         if (h->prog_host) {
             (void)hipHostFree(h->prog_host);
+        }
+        if (h->io_host) {
+            (void)hipHostFree(h->io_host);
         }
         if (h->prog_ev) {
             (void)hipEventDestroy(h->prog_ev);
