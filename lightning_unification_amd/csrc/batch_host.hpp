@@ -84,9 +84,9 @@ template <class T> struct BatchPlan final : BatchPlanBase {
     int nc = 0, npat = 0, entangler = 0;
     int4 pat{0, 0, 0, 0};
     std::vector<int> nq, depth;
-    std::vector<PauliTerm> terms;
-    std::vector<uint64_t> xmasks;
-    std::vector<uint32_t> term_off, term_cnt;
+    std::vector<BTerm> terms;
+    std::vector<BGroup> groups;
+    std::vector<uint32_t> group_off, group_cnt;
     std::vector<uint64_t> par_off;
     uint64_t npar = 0;
     std::vector<double> norms; // <psi|psi> of each circuit's final state, last replay
@@ -95,8 +95,8 @@ template <class T> struct BatchPlan final : BatchPlanBase {
     hipStream_t stream = nullptr;
     V *arena = nullptr;
     BCirc *dcircs = nullptr;
-    PauliTerm *dterms = nullptr;
-    uint64_t *dxm = nullptr;
+    BTerm *dterms = nullptr;
+    BGroup *dgroups = nullptr;
     double *dparams = nullptr, *dgrads = nullptr, *denergy = nullptr;
     double2 *dcs = nullptr; // (cos, sin) of every half angle, refreshed each replay
     BMat *dmats = nullptr;  // every wire's 2x2 per layer, refreshed each replay
@@ -135,17 +135,30 @@ template <class T> struct BatchPlan final : BatchPlanBase {
             depth.push_back(d[j]);
             par_off.push_back(npar);
             npar += static_cast<uint64_t>(d[j]) * n[j] * npat;
-            term_off.push_back(static_cast<uint32_t>(terms.size()));
-            term_cnt.push_back(static_cast<uint32_t>(t[j].size()));
             // group the circuit's terms by x-mask: one amplitude load per mask
             std::vector<size_t> order(t[j].size());
             std::iota(order.begin(), order.end(), size_t{0});
             std::stable_sort(order.begin(), order.end(),
                              [&](size_t a, size_t b) { return x[j][a] < x[j][b]; });
+            group_off.push_back(static_cast<uint32_t>(groups.size()));
             for (size_t k : order) {
-                terms.push_back(t[j][k]);
-                xmasks.push_back(x[j][k]);
+                const auto at = static_cast<uint32_t>(terms.size());
+                const auto xm = static_cast<uint32_t>(x[j][k]);
+                if (groups.size() == group_off.back() || groups.back().x != xm) {
+                    groups.push_back(BGroup{xm, at, at});
+                }
+                groups.back().last = at + 1;
+                const PauliTerm &p = t[j][k];
+                BTerm b{0, 0, static_cast<uint32_t>(p.zy), 0};
+                switch (p.ny & 3) { // coeff (-i)^ny
+                case 0: b.cr = p.coeff; break;
+                case 1: b.ci = -p.coeff; break;
+                case 2: b.cr = -p.coeff; break;
+                default: b.ci = p.coeff; break;
+                }
+                terms.push_back(b);
             }
+            group_cnt.push_back(static_cast<uint32_t>(groups.size()) - group_off.back());
         }
         int dev = 0;
         HIP_OK(hipGetDevice(&dev));
@@ -160,16 +173,16 @@ template <class T> struct BatchPlan final : BatchPlanBase {
         }
         HIP_OK(hipMalloc(&arena, std::max<uint64_t>(amps, 1) * sizeof(V)));
         HIP_OK(hipMalloc(&dcircs, std::max(nc, 1) * sizeof(BCirc)));
-        HIP_OK(hipMalloc(&dterms, std::max<size_t>(terms.size(), 1) * sizeof(PauliTerm)));
-        HIP_OK(hipMalloc(&dxm, std::max<size_t>(xmasks.size(), 1) * sizeof(uint64_t)));
+        HIP_OK(hipMalloc(&dterms, std::max<size_t>(terms.size(), 1) * sizeof(BTerm)));
+        HIP_OK(hipMalloc(&dgroups, std::max<size_t>(groups.size(), 1) * sizeof(BGroup)));
         HIP_OK(hipMalloc(&dparams, std::max<uint64_t>(npar, 1) * sizeof(double)));
         HIP_OK(hipMalloc(&dgrads, std::max<uint64_t>(npar, 1) * sizeof(double)));
         HIP_OK(hipMalloc(&dcs, std::max<uint64_t>(npar, 1) * sizeof(double2)));
         HIP_OK(hipMalloc(&dmats, std::max<uint64_t>(npar / npat, 1) * sizeof(BMat)));
         HIP_OK(hipMalloc(&denergy, 2 * std::max(nc, 1) * sizeof(double))); // energies, then <psi|psi>
         if (!terms.empty()) {
-            HIP_OK(hipMemcpy(dterms, terms.data(), terms.size() * sizeof(PauliTerm), hipMemcpyHostToDevice));
-            HIP_OK(hipMemcpy(dxm, xmasks.data(), xmasks.size() * sizeof(uint64_t), hipMemcpyHostToDevice));
+            HIP_OK(hipMemcpy(dterms, terms.data(), terms.size() * sizeof(BTerm), hipMemcpyHostToDevice));
+            HIP_OK(hipMemcpy(dgroups, groups.data(), groups.size() * sizeof(BGroup), hipMemcpyHostToDevice));
         }
         if (tile_width > 0) {
             configure(tile_width);
@@ -186,7 +199,7 @@ template <class T> struct BatchPlan final : BatchPlanBase {
             (void)hipGraphDestroy(graph);
         }
         for (void *p : {static_cast<void *>(arena), static_cast<void *>(dcircs),
-                        static_cast<void *>(dterms), static_cast<void *>(dxm),
+                        static_cast<void *>(dterms), static_cast<void *>(dgroups),
                         static_cast<void *>(dparams), static_cast<void *>(dgrads), static_cast<void *>(dcs),
                         static_cast<void *>(dmats), static_cast<void *>(denergy), static_cast<void *>(dcirc_lists),
                         static_cast<void *>(dprefix)}) {
@@ -229,11 +242,11 @@ template <class T> struct BatchPlan final : BatchPlanBase {
             c.n = nq[j];
             c.depth = depth[j];
             c.nstage = stages(nq[j], W);
-            c.nterms = static_cast<int>(term_cnt[j]);
+            c.ngroups = static_cast<int>(group_cnt[j]);
             c.off = off;
             off += uint64_t{4} << nq[j];
             c.par = static_cast<uint32_t>(par_off[j]);
-            c.term = term_off[j];
+            c.group = group_off[j];
             Gf2Map m(nq[j]);
             if (entangler && nq[j] > 1) {
                 const int last = entangler == 2 ? nq[j] : nq[j] - 1;
@@ -379,7 +392,7 @@ template <class T> struct BatchPlan final : BatchPlanBase {
                 break;
             case LaunchSpec::Obs:
                 hipLaunchKernelGGL((k_batch_obs<T>), grid, dim3(kBlock), 0, stream, arena, dcircs,
-                                   ls.L, entangler ? 1 : 0, dterms, dxm, denergy,
+                                   ls.L, entangler ? 1 : 0, dterms, dgroups, denergy,
                                    denergy + nc);
                 break;
             case LaunchSpec::RotAdj:

@@ -34,10 +34,10 @@ struct BCirc {
     int n;           // qubits
     int depth;       // layers
     int nstage;      // rotation stages per layer
-    int nterms;      // Pauli terms of the observable
+    int ngroups;     // x-masks of the observable
     uint64_t off;    // amplitude offset of buffer 0 (buffers k at off + k * 2^n)
     uint32_t par;    // offset of this circuit's angles / gradients
-    uint32_t term;   // offset of its Pauli terms
+    uint32_t group;  // offset of its groups
     uint32_t fwd_rows[kBatchMaxQubits]; // entangler gather:  src bit b = parity(y & fwd_rows[b])
     uint32_t adj_rows[kBatchMaxQubits]; // inverse entangler gather
 };
@@ -209,15 +209,29 @@ __global__ __launch_bounds__(kBlock) void k_batch_init(v2<T> *__restrict__ arena
     }
 }
 
+// A term's coefficient with its (-i)^ny, and its Z/Y bits.
+struct BTerm {
+    double cr, ci;
+    uint32_t zy, pad;
+};
+// The terms of one circuit that share an x-mask: terms [first, last).
+struct BGroup {
+    uint32_t x, first, last;
+};
+
 // H psi into buffer 2 + f, E += Re<psi|H psi> and N += <psi|psi> (FP64
 // atomics per block), where psi sits in buffer f = depth mod 2 when layers
 // end with an entangler (each one flips the buffer) and f = 0 otherwise.
+// The amplitudes of four groups are loaded together (one at a time, a 20-qubit
+// Ising sum was twenty dependent loads a thread), and a group's signed
+// coefficients are added before its one complex product: 512 circuits, 3.07 ->
+// 2.33 ms a replay; what is left are the L1 and L2 reads.
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_batch_obs(v2<T> *__restrict__ arena,
                                                       const BCirc *__restrict__ circs,
                                                       const BLaunch L, int ent,
-                                                      const PauliTerm *__restrict__ terms,
-                                                      const uint64_t *__restrict__ xmasks,
+                                                      const BTerm *__restrict__ terms,
+                                                      const BGroup *__restrict__ groups,
                                                       double *__restrict__ energy,
                                                       double *__restrict__ norm2) {
     uint64_t q;
@@ -230,30 +244,31 @@ __global__ __launch_bounds__(kBlock) void k_batch_obs(v2<T> *__restrict__ arena,
     double e = 0, pn = 0;
     if (y < len) {
         const v2<T> *psi = arena + c.off + pbuf * len;
+        const uint32_t yb = static_cast<uint32_t>(y);
         double hr = 0, hi = 0;
-        uint64_t xm_prev = ~uint64_t{0};
-        v2<T> a{};
-        for (int t = 0; t < c.nterms; t++) { // terms arrive grouped by x-mask
-            const PauliTerm &pt = terms[c.term + t];
-            const uint64_t xm = xmasks[c.term + t];
-            if (xm != xm_prev) {
-                a = psi[y ^ xm];
-                xm_prev = xm;
+        for (int g0 = 0; g0 < c.ngroups; g0 += 4) {
+            v2<T> a[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                if (g0 + j < c.ngroups) {
+                    a[j] = psi[yb ^ groups[c.group + g0 + j].x];
+                }
             }
-            // coeff * (-i)^ny * (-1)^popcount(y & zy) * a
-            double cr = pt.coeff, ci2 = 0;
-            switch (pt.ny & 3) {
-            case 1: ci2 = -cr; cr = 0; break;
-            case 2: cr = -cr; break;
-            case 3: ci2 = cr; cr = 0; break;
-            default: break;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                if (g0 + j < c.ngroups) {
+                    const BGroup &g = groups[c.group + g0 + j];
+                    double cr = 0, ci2 = 0;
+                    for (uint32_t t = g.first; t < g.last; t++) {
+                        const BTerm &tm = terms[t];
+                        const bool minus = __popc(yb & tm.zy) & 1;
+                        cr += minus ? -tm.cr : tm.cr;
+                        ci2 += minus ? -tm.ci : tm.ci;
+                    }
+                    hr += cr * double(a[j].x) - ci2 * double(a[j].y);
+                    hi += cr * double(a[j].y) + ci2 * double(a[j].x);
+                }
             }
-            if (__popcll(y & pt.zy) & 1) {
-                cr = -cr;
-                ci2 = -ci2;
-            }
-            hr += cr * double(a.x) - ci2 * double(a.y);
-            hi += cr * double(a.y) + ci2 * double(a.x);
         }
         v2<T> hv;
         hv.x = T(hr);
@@ -293,7 +308,9 @@ __global__ __launch_bounds__(kBlock) void k_batch_obs(v2<T> *__restrict__ arena,
 // A trip through LDS and a barrier per wire, as before, left the stages at 2.6
 // (adjoint) and 3.3 TB/s; windows take a third of the trips.  complex64 states
 // are rotated in double: a stage rounds an amplitude once.
-// BATCH_FIGURES
+// 512 circuits of 8-20 qubits complex128: 63.4 -> 32.3 ms a replay, the widest
+// adjoint launch 1.67 ms -> 0.81 (3.8 TB/s, a large copy 4.35); one circuit of
+// 16 qubits 485 -> 390 us.
 template <class T, int NW, bool ADJ>
 __global__ __launch_bounds__(64 * NW, NW == 16 || ADJ ? 4 : 8) void k_batch_stage(
     v2<T> *__restrict__ arena, const BCirc *__restrict__ circs, const BLaunch L, int W, int stage, int layer, int lb,
@@ -310,8 +327,17 @@ __global__ __launch_bounds__(64 * NW, NW == 16 || ADJ ? 4 : 8) void k_batch_stag
     const BCirc &c = circs[find_circ(L, blockIdx.x, q)];
     int bits[16];
     int alo, ahi;
+    const uint32_t tid = threadIdx.x;
+    const BMat *lm = mats + c.par / npat + static_cast<uint64_t>(layer) * c.n;
+    // the layer's matrices and the circuit's index rows into the caches at
+    // once: the scalar loads of each wire and row would meet memory one after
+    // another (half of a small circuit's stage)
+    if (tid < static_cast<uint32_t>(c.n)) {
+        asm volatile("" ::"v"(*reinterpret_cast<const int *>(lm + tid)),
+                     "v"((ADJ ? c.adj_rows : c.fwd_rows)[tid]));
+    }
     const int Tn = stage_bits(c.n, W, stage, bits, alo, ahi);
-    const uint32_t tid = threadIdx.x, size = 1U << Tn;
+    const uint32_t size = 1U << Tn;
     const uint64_t len = uint64_t{1} << c.n;
     v2<T> *st[2] = {arena + c.off + lb * len, arena + c.off + (ADJ ? hb : lb) * len};
     const uint64_t base = tile_base(q, bits, Tn);
@@ -343,7 +369,6 @@ __global__ __launch_bounds__(64 * NW, NW == 16 || ADJ ? 4 : 8) void k_batch_stag
     // local positions of the target bits: [ka, kb)
     const int shift = stage == 0 ? 0 : bits[3] - 3;
     const int ka = alo - shift, kb = ahi - shift;
-    const BMat *lm = mats + c.par / npat + static_cast<uint64_t>(layer) * c.n;
     const int lane = tid & 63, wave = tid >> 6;
     uint32_t win = HOME;
     for (int top = kb; top > ka;) { // target bits at and above `top` are done
