@@ -266,7 +266,8 @@ struct ScratchScope {
 
 // Device buffers kept by a handle between calls, one per purpose.
 enum Buf { kBufUniforms, kBufIndices, kBufBits, kBufCdfGroups, kBufCdfPrefix, kBufCdfTiles, kBufChainStart,
-           kBufScalar, kBufSweepProg, kBufSweepPart, kBufSweepSums, kBufSweepStates, kBufCount };
+           kBufScalar, kBufSweepProg, kBufSweepPart, kBufSweepSums, kBufSweepStates, kBufProbs, kBufCount };
+constexpr uint64_t kProbsKept = 4096; // bins of a marginal whose buffer stays with the handle
 
 // The handle's buffer for `purpose`, at least `bytes` long (grown when
 // needed, after the handle's queued work, which may still use the old one).

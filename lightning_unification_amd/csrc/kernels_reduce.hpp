@@ -265,21 +265,30 @@ __device__ __forceinline__ uint64_t bin_bits(uint64_t bin, const MarginalGeom &m
     return r;
 }
 
-// Marginal probabilities, bin bit j taken from bit position bitpos[j].  Grid: blockIdx.y
-// = bin, blockIdx.x = chunk of the remaining index space; partial[bin][chunk].
+// Marginal probabilities, bin bit j taken from bit position bitpos[j], no
+// marginal bit below 3.  Grid: blockIdx.y = bin, blockIdx.x = chunk of the
+// remaining index space; partial[bin][chunk].  A thread takes four consecutive
+// amplitudes per expanded index: one at a time, inserting the marginal bits
+// cost more issue slots than the reads took (27 qubits complex64, 8 wires:
+// 275 us for 1 GiB -> 195, 5.5 TB/s).
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_marginal(const v2<T> *__restrict__ sv,
                                                      uint64_t nrest, MarginalGeom m,
                                                      double *__restrict__ partial) {
     const uint64_t bin = blockIdx.y;
     const uint64_t bb = bin_bits(bin, m);
-    double acc = 0;
-    const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kBlock;
-    for (uint64_t r = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x; r < nrest; r += stride) {
-        const v2<T> a = sv[expand(r, m.rest) | bb];
-        acc += double(a.x * a.x + a.y * a.y);
+    double acc[4] = {0, 0, 0, 0};
+    const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kBlock * 4;
+    // nrest is a multiple of 8: the three lowest bits are free
+    for (uint64_t r = (static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x) * 4; r < nrest; r += stride) {
+        const v2<T> *at = sv + (expand(r, m.rest) | bb);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const v2<T> a = at[k];
+            acc[k] += double(a.x) * double(a.x) + double(a.y) * double(a.y);
+        }
     }
-    const double2 s = block_sum2(double2{acc, 0});
+    const double2 s = block_sum2(double2{(acc[0] + acc[1]) + (acc[2] + acc[3]), 0});
     if (threadIdx.x == 0) {
         partial[bin * gridDim.x + blockIdx.x] = s.x;
     }
@@ -320,7 +329,7 @@ __global__ __launch_bounds__(kBlock) void k_marginal_lo(const v2<T> *__restrict_
 #pragma unroll
         for (int c = 0; c < C; c++) {
             const v2<T> a = sv[base | off[c]];
-            acc[c] += double(a.x * a.x + a.y * a.y);
+            acc[c] += double(a.x) * double(a.x) + double(a.y) * double(a.y);
         }
     }
 #pragma unroll

@@ -15,9 +15,11 @@
 //       tile's own scan offset by its total's prefix, tpre[t] = gpre[t * kCdfTile]);
 //   (3) k_cdf_search: one thread per sample bisects tpre, then gpre inside the
 //       tile, for the last group with C_{64 g} < U; its wavefront then walks
-//       its 64 samples one after another, each time loading the chosen group
-//       (one amplitude per lane) and counting with a wavefront scan the C_k
-//       below U.
+//       its 64 samples, four a step, each loading the chosen group (sixteen
+//       lanes, four amplitudes a lane) and counting the C_k below U.  A
+//       million samples of 27 qubits complex64: 257 us with one
+//       sample a step over 64 lanes (twelve LDS shuffles a sample), 232 so:
+//       the reads of 512 bytes a sample at random places bound it.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -173,25 +175,14 @@ __global__ __launch_bounds__(1024) void k_scan_exclusive(const double *__restric
     }
 }
 
-__device__ __forceinline__ double wave_incl_scan(double x, int lane) {
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const double y = __shfl_up(x, o, 64);
-        if (lane >= o) {
-            x += y;
-        }
-    }
-    return x;
+// value of the lane N below in the row of 16 lanes (0 where there is none)
+template <int N> __device__ __forceinline__ int row_shr_i(int x) {
+    return __builtin_amdgcn_update_dpp(0, x, 0x110 + N, 0xf, 0xf, true);
 }
-
-// value of lane `lane` (uniform) of a 64-bit register
-__device__ __forceinline__ uint64_t readlane_u64(uint64_t x, int lane) {
-    const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(static_cast<uint32_t>(x)), lane));
-    const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(static_cast<uint32_t>(x >> 32)), lane));
-    return (static_cast<uint64_t>(hi) << 32) | lo;
-}
-__device__ __forceinline__ double readlane_d(double x, int lane) {
-    return __longlong_as_double(static_cast<long long>(readlane_u64(static_cast<uint64_t>(__double_as_longlong(x)), lane)));
+template <int N> __device__ __forceinline__ double row_shr(double x) {
+    const long long v = __double_as_longlong(x);
+    const int lo = row_shr_i<N>(static_cast<int>(v)), hi = row_shr_i<N>(static_cast<int>(v >> 32));
+    return __longlong_as_double((static_cast<long long>(hi) << 32) | static_cast<uint32_t>(lo));
 }
 
 // idx[s] = (#{k : C_k < u[s]}) - 1 clamped to [0, len - 1]
@@ -233,32 +224,60 @@ __global__ __launch_bounds__(kBlock) void k_cdf_search(const v2<T> *__restrict__
         g = static_cast<int64_t>(a) - 1;
         base = gpre[g];
     }
-    // the wavefront scans its samples' groups one after another
+    // the wavefront scans its samples' groups, four samples a step (sixteen
+    // lanes a sample, four amplitudes a lane), the loads of four steps in flight
+    constexpr int B = 4;
     const int64_t wave0 = s - lane;
     const int nv = m - wave0 < 64 ? static_cast<int>(m - wave0) : 64;
+    const int row = lane >> 4, rl = lane & 15;
     int64_t my = 0;
-    for (int i = 0; i < nv; i++) {
-        const int64_t gi = static_cast<int64_t>(readlane_u64(static_cast<uint64_t>(g), i));
-        if (gi < 0) {
-            if (lane == i) {
-                my = 0;
+    for (int i0 = 0; i0 < nv; i0 += 4 * B) {
+        int64_t gi[B];
+        v2<T> a[B][4];
+#pragma unroll
+        for (int j = 0; j < B; j++) {
+            gi[j] = __shfl(g, i0 + 4 * j + row, 64); // past nv: a lane whose g is -1
+            const uint64_t e = static_cast<uint64_t>(gi[j] < 0 ? 0 : gi[j]) * kCdfGroup + 4 * rl;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                a[j][k].x = a[j][k].y = 0;
+                if (e + k < len) {
+                    a[j][k] = sv[e + k];
+                }
             }
-            continue;
         }
-        const double Ui = readlane_d(U, i);
-        const double bi = readlane_d(base, i);
-        const uint64_t e = static_cast<uint64_t>(gi) * kCdfGroup + lane;
-        double p = 0;
-        if (e < len) {
-            const v2<T> a = sv[e];
-            p = double(a.x) * double(a.x) + double(a.y) * double(a.y);
-        }
-        const double c = bi + (wave_incl_scan(p, lane) - p);
-        const uint64_t below = __ballot(e < len && c < Ui);
-        int64_t r = static_cast<int64_t>(gi) * kCdfGroup + __popcll(below) - 1;
-        r = r < 0 ? 0 : (r > static_cast<int64_t>(len) - 1 ? static_cast<int64_t>(len) - 1 : r);
-        if (lane == i) {
-            my = r;
+#pragma unroll
+        for (int j = 0; j < B; j++) {
+            const double Ui = __shfl(U, i0 + 4 * j + row, 64), bi = __shfl(base, i0 + 4 * j + row, 64);
+            const uint64_t e = static_cast<uint64_t>(gi[j] < 0 ? 0 : gi[j]) * kCdfGroup + 4 * rl;
+            double p[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                p[k] = double(a[j][k].x) * double(a[j][k].x) + double(a[j][k].y) * double(a[j][k].y);
+            }
+            const double own = (p[0] + p[1]) + (p[2] + p[3]);
+            double in = own;
+            in += row_shr<1>(in);
+            in += row_shr<2>(in);
+            in += row_shr<4>(in);
+            in += row_shr<8>(in);
+            double c = in - own;
+            int below = 0;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                below += e + k < len && bi + c < Ui ? 1 : 0;
+                c += p[k];
+            }
+            below += row_shr_i<1>(below);
+            below += row_shr_i<2>(below);
+            below += row_shr_i<4>(below);
+            below += row_shr_i<8>(below);
+            int64_t r = gi[j] * kCdfGroup + below - 1; // the row's count is in its lane 15
+            r = r < 0 ? 0 : (r > static_cast<int64_t>(len) - 1 ? static_cast<int64_t>(len) - 1 : r);
+            r = __shfl(r, 16 * (lane & 3) + 15, 64);
+            if ((lane >> 2) == (i0 >> 2) + j && g >= 0) {
+                my = r; // g = -1 (U <= 0): index 0
+            }
         }
     }
     if (valid) {

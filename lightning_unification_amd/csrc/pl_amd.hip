@@ -1261,11 +1261,16 @@ template <class T> struct Engine {
         m.free_mask = (len() - 1) & ~pinned;
         const uint64_t nbins = uint64_t{1} << nw, nrest = len() >> nw;
         double *d = nullptr;
-        HIP_OK(hipMalloc(reinterpret_cast<void **>(&d), nbins * sizeof(double)));
         struct FreeD {
-            double *p;
+            double *p = nullptr;
             ~FreeD() { (void)hipFree(p); }
-        } free_d{d};
+        } free_d;
+        if (nbins <= kProbsKept) { // kept with the handle: an allocation and its free cost tens of us
+            d = static_cast<double *>(buf(h, kBufProbs, nbins * sizeof(double)));
+        } else {
+            HIP_OK(hipMalloc(reinterpret_cast<void **>(&d), nbins * sizeof(double)));
+            free_d.p = d;
+        }
         if (nw <= 12 && nrest >= 4096) {
             m.rest.nb = nw;
             m.rest.fixed = 0;
@@ -1327,8 +1332,8 @@ template <class T> struct Engine {
         return {gpre, tpre, ngroups, ntiles};
     }
     // didx[s] for the uniforms du[s], both in device memory (queued, no wait)
-    void sample_device(const double *du, int64_t m, int64_t *didx) {
-        const CdfTables c = cdf_tables();
+    void sample_device(const double *du, int64_t m, int64_t *didx) { search_device(cdf_tables(), du, m, didx); }
+    void search_device(const CdfTables &c, const double *du, int64_t m, int64_t *didx) {
         hipLaunchKernelGGL((k_cdf_search<T>), dim3(static_cast<unsigned>((m + kBlock - 1) / kBlock)), dim3(kBlock),
                            0, h->stream, psi(), len(), c.ngroups, c.ntiles, c.tpre, c.gpre, du, m, didx);
         HIP_OK(hipGetLastError());
@@ -1340,6 +1345,7 @@ template <class T> struct Engine {
                 uint64_t *host_bits) {
         auto *du = static_cast<double *>(buf(h, kBufUniforms, m * sizeof(double)));
         auto *didx = static_cast<int64_t *>(buf(h, kBufIndices, m * sizeof(int64_t)));
+        const CdfTables c = cdf_tables(); // queued first: the uniforms are staged meanwhile
         if (host_u) {
             upload_host(h, du, host_u, m * sizeof(double));
         } else {
@@ -1347,7 +1353,7 @@ template <class T> struct Engine {
                                h->stream, seed, m, du);
             HIP_OK(hipGetLastError());
         }
-        sample_device(du, m, didx);
+        search_device(c, du, m, didx);
         if (host_idx) {
             download_host(h, host_idx, didx, m * sizeof(int64_t));
         }
