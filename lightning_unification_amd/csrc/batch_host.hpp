@@ -214,7 +214,7 @@ template <class T> struct BatchPlan final : BatchPlanBase {
 
     int lds_limit = 65536; // bytes of LDS a workgroup may use (device attribute)
 
-    // widest tile whose adjoint stage (two tiles + its 2 KiB of reduction slots) fits
+    // widest tile two of which, with 2 KiB of reduction slots, fit the LDS
     int max_tile() const {
         int w = 4;
         while (w < kBatchMaxTile && (size_t{2} << (w + 1)) * sizeof(V) + 2048 <= static_cast<size_t>(lds_limit)) {
@@ -319,7 +319,7 @@ template <class T> struct BatchPlan final : BatchPlanBase {
         }
         add(LaunchSpec::Obs, 0, 0, [&](int) { return true; }, elem_blocks);
         // the entangler of each layer is undone inside its first adjoint
-        // rotation stage (k_batch_rot_adj gathers lambda and H)
+        // rotation stage (k_batch_stage gathers lambda and H)
         for (int l = dmax - 1; l >= 0; l--) {
             for (int s = smax - 1; s >= 0; s--) {
                 add(LaunchSpec::RotAdj, l, s,
