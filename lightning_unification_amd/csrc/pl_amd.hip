@@ -631,7 +631,9 @@ template <class T> struct Engine {
     static constexpr int kTileFloatQubits = 23;
     static constexpr int kTileDefaultLow = std::is_same_v<T, double> ? 3 : 4;
 
-    // Applies a tape as tile passes (tile.hpp); returns the number of launches.
+    // Applies a tape as tile passes (tile.hpp); returns the number of launches,
+    // with the state final: the deferred gates' flush behind pl_sv_device_ptr
+    // and the callers of pl_sv_apply_ops_tiled hand the memory to other streams.
     // k = 0 / low < 0 pick the measured defaults of the precision; with k = 0
     // a state narrower than the smallest tile runs gate by gate.  Each pass is
     // planned, compiled and launched before the next is planned, so the host's
@@ -652,6 +654,7 @@ template <class T> struct Engine {
             if (std::is_same_v<T, double> || n() < kTileFloatQubits) {
                 const int launches = apply_passes(sv, t);
                 if (launches >= 0) {
+                    HIP_OK(hipStreamSynchronize(h->stream));
                     return launches;
                 }
             }
