@@ -1594,6 +1594,13 @@ struct SweepTape {
     const double *params;
 };
 
+// Waits for the stream on the way out: declared after host memory that queued
+// copies read and before the first of them, it outlasts them on every path.
+struct Drain {
+    hipStream_t s;
+    ~Drain() { (void)hipStreamSynchronize(s); }
+};
+
 // States up to this size keep a second lambda, so that every observable group
 // of a pass can run at once; larger ones fill the device group by group.
 constexpr size_t kSweepTwoLambdas = size_t{64} << 20;
@@ -1694,16 +1701,13 @@ void backward_sweep(Engine<T> &E, const SweepTape &t, v2<T> *lam, const std::vec
     V *other = two ? static_cast<V *>(sc.get()) : lam;
     V *mu = nullptr;
     auto **dhs = static_cast<V **>(buf(h, kBufSweepStates, K * sizeof(V *)));
+    Drain drain{h->stream}; // hs
     HIP_OK(hipMemcpyAsync(dhs, hs.data(), K * sizeof(V *), hipMemcpyHostToDevice, h->stream));
     ProgramBuffer pb(h, 4 * steps.size()); // a step with two flips, and its window
     if (!pb.ok()) {
         throw DeviceError("no device memory for the sweep's programs");
     }
     std::vector<SweepStep> prog;
-    struct Drain { // hs outlives the copy of its pointers when a call below fails
-        hipStream_t s;
-        ~Drain() { (void)hipStreamSynchronize(s); }
-    } drain{h->stream};
     // slots in flight: partial sums of `cap` slots before a reduction
     size_t nslots_all = 0;
     for (const auto &s : steps) {
@@ -1873,6 +1877,7 @@ void vjp_sweep(Engine<T> &E, const SweepTape &t, const double *dy, int ntp, cons
     V *mu = static_cast<V *>(sc.get());
     E.copy(lam, E.psi());
     std::vector<V> host;
+    Drain drain{h->stream}; // dy and host: the sweep may refuse the tape with the upload queued
     if constexpr (std::is_same_v<T, double>) {
         upload_host(h, mu, dy, E.len() * sizeof(V)); // the same layout
     } else {

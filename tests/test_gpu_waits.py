@@ -1,11 +1,17 @@
-"""Calls after which the state's memory may be read from any stream: the tiled
+"""Waits that calls owe their callers.
+
+Calls after which the state's memory may be read from any stream: the tiled
 executor and pl_sv_device_ptr with gates queued.  The engine's stream does not
 order itself against others, so the amplitudes copied on torch's stream right
-behind the call must be the ones the engine's own wait gives."""
+behind the call must be the ones the engine's own wait gives.
+
+Calls that refuse their input with a copy of the caller's memory queued: the
+next call on the handle gives the oracle's result."""
 import numpy as np
 import pytest
 
-from lightning_unification_amd.circuits import random_layers
+from conftest import random_state, rel_err
+from lightning_unification_amd.circuits import Tape, random_layers
 
 pytestmark = pytest.mark.gpu
 
@@ -39,3 +45,24 @@ def test_state_is_final_when_the_call_returns(dtype, n, how):
         sv.synchronize()
         assert torch.equal(got, view)
         assert abs(float(torch.linalg.vector_norm(got.abs().double())) - 1) < 1e-4
+
+
+@pytest.mark.parametrize("dtype", [np.complex128, np.complex64])
+def test_vjp_that_refuses_its_tape_has_finished_its_upload(oracle, dtype):
+    from lightning_unification_amd import capi
+    n = 15
+    good, bad, wrong = Tape(), Tape(), Tape()
+    for w in range(n):
+        good.add("RX", [w], [0.1 + w])
+    bad.add("Rot", [0], [0.1, 0.2, 0.3])  # more than one parameter
+    bad.ops += good.ops
+    wrong.ops = [("RY", [n], False, [0.3])] + list(good.ops)  # no such wire
+    tol = 1e-12 if dtype == np.complex128 else 5e-5
+    s, dy = random_state(n, 1, dtype), random_state(n, 2, dtype)
+    with capi.DeviceStateVector.from_array(s) as sv:
+        for tape in (bad, wrong):
+            with pytest.raises(ValueError):
+                sv.vjp(tape, random_state(n, 3, dtype), list(range(n + 1)))
+            got = sv.vjp(good, dy, list(range(n)))
+            exp = oracle.vjp(s.astype(np.complex128), good, dy.astype(np.complex128), list(range(n)))
+            assert rel_err(got, exp) < tol
