@@ -281,7 +281,11 @@ int pl_fuse_tape(int num_qubits, int nops, const int *ids, const int *nwires,
  * [0, 6].  tile_bits = 0 and low_bits = -1 run the passes of pl_sv_apply_ops
  * (tiles of a workgroup, held in double) for complex128 states and complex64
  * ones below 23 qubits; larger complex64 states take 2^12 amplitudes and 4 low
- * bits.  flags: PL_FUSE_RENORM rescales
+ * bits.  tile_bits = 0 with low_bits given takes the wavefront's tiles of
+ * those widths.  A tape with an operation that cannot be applied fails with
+ * the state untouched (below 9 qubits with tile_bits = 0: with the operations
+ * before it applied).  The state is final when the call returns.
+ * flags: PL_FUSE_RENORM rescales
  * the state to unit norm at the end, the norm accumulated in FP64 (the
  * precision form's renormalisation for complex64 states).  *npasses (may be
  * NULL) receives the number of launches. */

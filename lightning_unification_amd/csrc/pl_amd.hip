@@ -650,9 +650,11 @@ template <class T> struct Engine {
             // kTileFloatQubits or more, where this one's FP32 arithmetic and
             // 2^12-amplitude wavefront tiles win (28 qubits, 185 gates: 11.8
             // against 16.5 ms; 20 qubits, 133 gates: 0.45 against 0.26 ms;
-            // complex128 at 28 qubits: 24.2 against 16.4 ms)
-            if (std::is_same_v<T, double> || n() < kTileFloatQubits) {
-                const int launches = apply_passes(sv, t);
+            // complex128 at 28 qubits: 24.2 against 16.4 ms).  A caller's
+            // low_bits is for the wavefront tiles.  Like their scheduler, the
+            // passes refuse a tape as a whole, except below the smallest tile.
+            if (low < 0 && (std::is_same_v<T, double> || n() < kTileFloatQubits)) {
+                const int launches = apply_passes(sv, t, n() >= kTpMinBits);
                 if (launches >= 0) {
                     HIP_OK(hipStreamSynchronize(h->stream));
                     return launches;
@@ -778,12 +780,17 @@ template <class T> struct Engine {
     // Applies a tape; returns the number of launches, or -1, with nothing done,
     // where there is no memory for the passes' programs.  The operations
     // before one that does not lower are applied before its error leaves, as
-    // gate by gate.  Nothing here waits for the device's passes.
-    int apply_passes(V *sv, const TapeView &t) {
+    // gate by gate, or none (whole).  Nothing here waits for the device's passes.
+    int apply_passes(V *sv, const TapeView &t, bool whole = false) {
         SweepSteps builder;
         std::vector<SweepOp> parts;
         std::vector<int> woff(t.nops + 1, 0), poff(t.nops + 1, 0);
         std::exception_ptr refused;
+        for (int i = 0; whole && i < t.nops; i++) {
+            if (t.nwires[i] < 0 || t.nparams[i] < 0) {
+                throw InvalidArg("negative wire or parameter count");
+            }
+        }
         for (int i = 0; i < t.nops; i++) {
             woff[i + 1] = woff[i] + t.nwires[i];
             poff[i + 1] = poff[i] + t.nparams[i];
@@ -796,6 +803,9 @@ template <class T> struct Engine {
                 g = lower_gate<double>(n(), t.ids[i], w, t.nwires[i], t.inverse[i] != 0, t.params + poff[i],
                                        t.nparams[i]);
             } catch (...) {
+                if (whole) {
+                    throw;
+                }
                 refused = std::current_exception();
                 break;
             }

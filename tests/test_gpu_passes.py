@@ -71,3 +71,27 @@ def test_four_bit_members_at_every_window(oracle):
     with capi.DeviceStateVector.from_array(s) as sv:
         sv.apply_tape(tape)
         assert rel_err(sv.state(), exp, floor=0.1) < 1e-12
+
+
+@pytest.mark.parametrize("dtype", [np.complex128, np.complex64])
+@pytest.mark.parametrize("n", [9, 14])
+def test_default_tiles_refuse_a_tape_whole(dtype, n):
+    """The tiled executor leaves the state alone where an operation cannot be
+    applied, wherever it stands in the tape; a low-bit count out of range is
+    refused, one in range is the tiles'."""
+    from lightning_unification_amd import capi
+    good = random_layers(n, 2, seed=4)
+    s = random_state(n, 8, dtype)
+    with capi.DeviceStateVector.from_array(s) as sv:
+        for op in (("RX", [n], False, [0.3]), ("RX", [-1], False, [0.3]), ("CNOT", [1], False, [])):
+            for at in (0, 5, len(good.ops)):
+                tape = Tape()
+                tape.ops = list(good.ops[:at]) + [op] + list(good.ops[at:])
+                with pytest.raises(ValueError):
+                    sv.apply_tape_tiled(tape)
+                assert np.array_equal(sv.state(), s)
+        with pytest.raises(ValueError):
+            sv.apply_tape_tiled(good, 0, 7)
+        assert np.array_equal(sv.state(), s)
+        k = min(n, 11 if dtype == np.complex128 else 12)
+        assert sv.apply_tape_tiled(good, 0, 2) == len(capi.tile_plan(n, good, k, 2))
