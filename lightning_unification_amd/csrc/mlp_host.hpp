@@ -71,7 +71,7 @@ struct Mlp {
             nbf += static_cast<size_t>(ld[l]) * ld[l + 1];
         }
         alloc(&pbf, nbf);
-        HIP_OK(hipMemset(pbf, 0, nbf * sizeof(uint16_t))); // the padding stays zero
+        HIP_OK(hipMemsetAsync(pbf, 0, nbf * sizeof(uint16_t), stream)); // the padding stays zero
         const size_t B = row_pad(maxb), nblk = B / 32;
         alloc(&xf, static_cast<size_t>(maxb) * d0);
         alloc(&xb, B * ld[0]);

@@ -62,3 +62,16 @@ def test_rows_past_the_batch_stay_out():
         net.close()
     assert np.isfinite(got[1][0]) and got[0][0] == got[1][0]
     assert np.array_equal(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("seed", range(4))
+def test_initial_weights_are_in_place(seed):
+    """A network answers from its initial weights as soon as it exists."""
+    from lightning_unification_amd import capi
+    dims, b = (192, 512, 512, 193), 64
+    x = np.random.default_rng(seed).uniform(-1, 1, (b, dims[0])).astype(np.float32)
+    net = capi.Mlp(dims, max_batch=b, seed=seed)
+    y = net.predict(x)
+    y_ref = torch_reference(net, net.params(), x, np.zeros((b, dims[3]), np.float32), np.ones(dims[3], np.float32))[0]
+    assert np.max(np.abs(y - y_ref)) < 2e-3 * np.max(np.abs(y_ref))
+    net.close()
