@@ -210,12 +210,15 @@ template <bool TRA, bool TRB> __device__ void mlp_gemm(const GemmArgs &g, unsign
         }
         const size_t o = static_cast<size_t>(row) * g.ldact + col, oc = static_cast<size_t>(row) * g.N + col;
         switch (g.epi) {
-        case kEpiGelu: // padded columns: zero in, GELU(0) = 0 out
+        case kEpiGelu:
+            // padded columns stay zero: zero weights give NaN where an
+            // activation has overflowed, and the next layer reads them
+            z = in ? z : 0.0f;
             g.Z[o] = z;
             g.act[o] = f32_to_bf16(gelu(z));
             break;
         case kEpiGeluGrad:
-            z *= gelu_grad(g.Z[o]);
+            z = in ? z * gelu_grad(g.Z[o]) : 0.0f;
             csum += z;
             g.act[o] = f32_to_bf16(z);
             break;

@@ -75,3 +75,25 @@ def test_initial_weights_are_in_place(seed):
     y_ref = torch_reference(net, net.params(), x, np.zeros((b, dims[3]), np.float32), np.ones(dims[3], np.float32))[0]
     assert np.max(np.abs(y - y_ref)) < 2e-3 * np.max(np.abs(y_ref))
     net.close()
+
+
+def test_an_overflowed_activation_stays_infinite():
+    """All weights positive and one hidden value past the largest float: its
+    row's outputs are +inf as the product has them, not NaN from the zeros that
+    widths of 17 are padded with; the other rows are untouched."""
+    from lightning_unification_amd import capi
+    dims, b = (3, 17, 17, 5), 33
+    net = capi.Mlp(dims, max_batch=b, seed=3)
+    p = np.full(net.params().size, 0.25, np.float32)
+    p[:dims[1]] = 0.0
+    p[0] = 16.0  # feature 0 reaches hidden value 0 only
+    net.set_params(p)
+    x = np.full((b, 3), 0.5, np.float32)
+    x[7, 0] = 3e38
+    y = net.predict(x)
+    x[7, 0] = 0.5
+    ref = torch_reference(net, p, x, np.zeros((b, 5), np.float32), np.ones(5, np.float32))[0]
+    assert np.all(np.isposinf(y[7]))
+    rest = np.arange(b) != 7
+    assert np.max(np.abs(y[rest] - ref[rest])) < 2e-3 * np.max(np.abs(ref))
+    net.close()
