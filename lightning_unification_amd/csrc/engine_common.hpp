@@ -210,6 +210,18 @@ template <class F> int guarded(F &&f) {
 
 } // namespace plamd
 
+// The passes' programs on their way to the device (ProgramBuffer): kSegs
+// segments of pinned memory, each copied to the same place of a device buffer.
+struct ProgramRing {
+    static constexpr int kSegs = 4;
+    static constexpr size_t kSegBytes = size_t{32} << 10; // at first: about 240 steps
+    void *host = nullptr, *dev = nullptr; // host: nullptr where it cannot be pinned
+    size_t seg_bytes = 0, used = 0;       // used: bytes of the current segment
+    int seg = 0;
+    hipEvent_t ev[kSegs] = {}; // recorded behind the segment's copies when it was left
+    bool busy[kSegs] = {};
+};
+
 struct pl_sv {
     int n = 0;
     int dtype = PL_C128;
@@ -226,11 +238,7 @@ struct pl_sv {
     size_t staging_bytes = 0;
     std::vector<hipEvent_t> slots; // pl_event_record slots
     std::vector<std::pair<void *, size_t>> bufs; // grow-only device buffers by purpose (plamd::Buf)
-    // pinned copy of the programs of the last call's passes (ProgramBuffer)
-    void *prog_host = nullptr;
-    size_t prog_host_bytes = 0;
-    hipEvent_t prog_ev = nullptr;
-    bool prog_busy = false; // prog_ev is recorded behind copies from prog_host
+    ProgramRing ring;
     // small pinned area, host memory the device writes results to and tables
     // are uploaded from (io_area)
     void *io_host = nullptr;
@@ -266,7 +274,7 @@ struct ScratchScope {
 
 // Device buffers kept by a handle between calls, one per purpose.
 enum Buf { kBufUniforms, kBufIndices, kBufBits, kBufCdfGroups, kBufCdfPrefix, kBufCdfTiles, kBufChainStart,
-           kBufScalar, kBufSweepProg, kBufSweepPart, kBufSweepSums, kBufSweepStates, kBufProbs, kBufCount };
+           kBufScalar, kBufSweepPart, kBufSweepSums, kBufSweepStates, kBufProbs, kBufCount };
 constexpr uint64_t kProbsKept = 4096; // bins of a marginal whose buffer stays with the handle
 
 // The handle's buffer for `purpose`, at least `bytes` long (grown when

@@ -163,74 +163,90 @@ static void download_host(pl_sv_t h, void *dst, const void *src, size_t bytes) {
 
 template <class T> constexpr int kSweepLow = std::is_same_v<T, double> ? 3 : 4; // one 128-byte line
 
-// The programs of one call's passes on their way to the device: appended to
-// the handle's pinned buffer and copied from there without waiting.  The
-// buffer is taken again once the last call's copies have left it (an event);
-// where it cannot be pinned, each copy is waited for.
+// The passes' programs on their way to the device: appended to the current
+// segment of the handle's pinned ring and copied from there without waiting.
+// A full segment is left with an event behind its copies (and the passes
+// between them) and taken again once that event has come, so calls run ahead of the device by
+// up to three segments; the device side of a segment is safe by the stream's
+// order.  A call whose longest program may not fit a segment grows the ring,
+// after a wait.  Where the ring cannot be pinned, each copy is waited for.
+// With one buffer for a whole call, taken again when the call's last pass had
+// ended, a tape right behind another waited for it.
 class ProgramBuffer {
   public:
-    ProgramBuffer(pl_sv *h, size_t steps) : h_(h) {
-        const size_t bytes = steps * sizeof(SweepStep);
-        if (h->prog_busy) {
-            HIP_OK(hipEventSynchronize(h->prog_ev));
-            h->prog_busy = false;
-        }
-        if (h->prog_host_bytes < bytes) {
-            if (h->prog_host) {
-                HIP_OK(hipHostFree(h->prog_host));
-                h->prog_host = nullptr;
-                h->prog_host_bytes = 0;
-            }
-            const size_t sz = std::max<size_t>(bytes, 1 << 16);
-            if (hipHostMalloc(&h->prog_host, sz, hipHostMallocDefault) == hipSuccess) {
-                h->prog_host_bytes = sz;
-            } else {
-                (void)hipGetLastError();
-                h->prog_host = nullptr;
-            }
-        }
-        if (!h->prog_ev) {
-            HIP_OK(hipEventCreateWithFlags(&h->prog_ev, hipEventDisableTiming));
-        }
-        try {
-            dev_ = static_cast<SweepStep *>(buf(h, kBufSweepProg, std::max<size_t>(bytes, 1 << 16)));
-            cap_ = steps;
-        } catch (const DeviceError &) { // the device is full: ok() is false
-            (void)hipGetLastError();
+    // longest: steps of any one program of the call, at most
+    ProgramBuffer(pl_sv *h, size_t longest) : h_(h), r_(h->ring) {
+        const size_t bytes = longest * sizeof(SweepStep);
+        if (r_.seg_bytes < bytes) {
+            reserve(std::max(bytes, ProgramRing::kSegBytes));
         }
     }
-    bool ok() const { return dev_ != nullptr; }
-    ~ProgramBuffer() {
-        if (used_ > 0 && h_->prog_host) {
-            h_->prog_busy = hipEventRecord(h_->prog_ev, h_->stream) == hipSuccess;
-            if (!h_->prog_busy) {
-                (void)hipStreamSynchronize(h_->stream);
-            }
-        }
-    }
+    bool ok() const { return r_.dev != nullptr; } // false: the device is full
     // the device address of the steps, in place for work queued after this
     const SweepStep *put(const std::vector<SweepStep> &steps) {
-        if (used_ + steps.size() > cap_) {
+        const size_t bytes = steps.size() * sizeof(SweepStep);
+        if (bytes > r_.seg_bytes) {
             throw std::logic_error("a program longer than its steps and windows");
         }
-        SweepStep *to = dev_ + used_;
-        const size_t bytes = steps.size() * sizeof(SweepStep);
-        if (h_->prog_host) {
-            SweepStep *from = static_cast<SweepStep *>(h_->prog_host) + used_;
+        if (r_.used + bytes > r_.seg_bytes) {
+            next();
+        }
+        const size_t at = r_.seg * r_.seg_bytes + r_.used;
+        auto *to = static_cast<unsigned char *>(r_.dev) + at;
+        if (r_.host) {
+            auto *from = static_cast<unsigned char *>(r_.host) + at;
             std::memcpy(from, steps.data(), bytes);
             HIP_OK(hipMemcpyAsync(to, from, bytes, hipMemcpyHostToDevice, h_->stream));
         } else {
             HIP_OK(hipMemcpyAsync(to, steps.data(), bytes, hipMemcpyHostToDevice, h_->stream));
             HIP_OK(hipStreamSynchronize(h_->stream));
         }
-        used_ += steps.size();
-        return to;
+        r_.used += bytes;
+        return reinterpret_cast<const SweepStep *>(to);
     }
 
   private:
+    void next() {
+        if (!r_.ev[r_.seg]) {
+            HIP_OK(hipEventCreateWithFlags(&r_.ev[r_.seg], hipEventDisableTiming));
+        }
+        HIP_OK(hipEventRecord(r_.ev[r_.seg], h_->stream));
+        r_.busy[r_.seg] = true;
+        r_.seg = (r_.seg + 1) % ProgramRing::kSegs;
+        r_.used = 0;
+        if (r_.busy[r_.seg]) {
+            HIP_OK(hipEventSynchronize(r_.ev[r_.seg]));
+            r_.busy[r_.seg] = false;
+        }
+    }
+    // new segments of `bytes`; none where the device is full
+    void reserve(size_t bytes) {
+        if (r_.dev) {
+            HIP_OK(hipStreamSynchronize(h_->stream));
+            (void)hipFree(r_.dev);
+            if (r_.host) {
+                (void)hipHostFree(r_.host);
+            }
+            r_.dev = r_.host = nullptr;
+        }
+        r_.seg_bytes = bytes;
+        r_.seg = 0;
+        r_.used = 0;
+        std::fill(r_.busy, r_.busy + ProgramRing::kSegs, false);
+        if (hipMalloc(&r_.dev, ProgramRing::kSegs * bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            r_.dev = nullptr;
+            r_.seg_bytes = 0;
+            return;
+        }
+        if (hipHostMalloc(&r_.host, ProgramRing::kSegs * bytes, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            r_.host = nullptr;
+        }
+    }
+
     pl_sv *h_;
-    SweepStep *dev_ = nullptr;
-    size_t used_ = 0, cap_ = 0;
+    ProgramRing &r_;
 };
 
 template <class T> struct Engine {
@@ -780,7 +796,8 @@ template <class T> struct Engine {
     // Applies a tape; returns the number of launches, or -1, with nothing done,
     // where there is no memory for the passes' programs.  The operations
     // before one that does not lower are applied before its error leaves, as
-    // gate by gate, or none (whole).  Nothing here waits for the device's passes.
+    // gate by gate, or none (whole).  The device is waited for only
+    // where the program ring has gone round (ProgramBuffer).
     int apply_passes(V *sv, const TapeView &t, bool whole = false) {
         SweepSteps builder;
         std::vector<SweepOp> parts;
@@ -835,7 +852,7 @@ template <class T> struct Engine {
             SweepScheduler sched(n(), bits, low, steps);
             SweepPass ps;
             std::vector<SweepStep> prog;
-            ProgramBuffer pb(h, 2 * steps.size()); // a step and its window
+            ProgramBuffer pb(h, 2 * std::min(steps.size(), kSweepLookahead)); // a step and its window
             if (!pb.ok()) {
                 return -1;
             }
@@ -1713,7 +1730,7 @@ void backward_sweep(Engine<T> &E, const SweepTape &t, v2<T> *lam, const std::vec
     auto **dhs = static_cast<V **>(buf(h, kBufSweepStates, K * sizeof(V *)));
     Drain drain{h->stream}; // hs
     HIP_OK(hipMemcpyAsync(dhs, hs.data(), K * sizeof(V *), hipMemcpyHostToDevice, h->stream));
-    ProgramBuffer pb(h, 4 * steps.size()); // a step with two flips, and its window
+    ProgramBuffer pb(h, 4 * std::min(steps.size(), kSweepLookahead)); // a step with two flips, and its window
     if (!pb.ok()) {
         throw DeviceError("no device memory for the sweep's programs");
     }
@@ -1973,14 +1990,17 @@ int pl_sv_destroy(pl_sv_t h) {
         for (void *p : h->pool) {
             (void)hipFree(p);
         }
-        if (h->prog_host) {
-            (void)hipHostFree(h->prog_host);
+        (void)hipFree(h->ring.dev);
+        if (h->ring.host) {
+            (void)hipHostFree(h->ring.host);
+        }
+        for (hipEvent_t e : h->ring.ev) {
+            if (e) {
+                (void)hipEventDestroy(e);
+            }
         }
         if (h->io_host) {
             (void)hipHostFree(h->io_host);
-        }
-        if (h->prog_ev) {
-            (void)hipEventDestroy(h->prog_ev);
         }
         (void)hipFree(h->red);
         (void)hipFree(h->staging);

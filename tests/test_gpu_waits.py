@@ -66,3 +66,35 @@ def test_vjp_that_refuses_its_tape_has_finished_its_upload(oracle, dtype):
             got = sv.vjp(good, dy, list(range(n)))
             exp = oracle.vjp(s.astype(np.complex128), good, dy.astype(np.complex128), list(range(n)))
             assert rel_err(got, exp) < tol
+
+
+def test_tapes_run_ahead_of_the_device():
+    """A tape's call does not wait for the tape before it: three queued behind
+    each other take a fraction of their run time to submit, and many short ones,
+    whose programs go round the upload ring several times, give the oracle's state."""
+    import time
+    from lightning_unification_amd import capi
+    tape = random_layers(28, 4, seed=6)
+    with capi.DeviceStateVector(28) as sv:
+        sv.apply_tape(tape)
+        sv.synchronize()
+        t0 = time.perf_counter()
+        for _ in range(3):
+            sv.apply_tape(tape)
+        queued = time.perf_counter() - t0
+        sv.synchronize()
+        assert queued < 0.5 * (time.perf_counter() - t0)
+
+
+@pytest.mark.parametrize("n,layers,times", [(6, 2, 60), (12, 25, 4), (14, 120, 2)])
+def test_programs_round_the_ring(oracle, n, layers, times):
+    """Short programs many times round the ring, and tapes whose programs grow it."""
+    from lightning_unification_amd import capi
+    s = random_state(n, 3)
+    exp = s.copy()
+    with capi.DeviceStateVector.from_array(s) as sv:
+        for i in range(times):
+            tape = random_layers(n, layers, seed=i)
+            sv.apply_tape(tape)
+            oracle.apply_tape(exp, tape)
+        assert rel_err(sv.state(), exp, floor=0.1) < 1e-12 * times
