@@ -222,6 +222,22 @@ struct ProgramRing {
     bool busy[kSegs] = {};
 };
 
+// What a handle's first tape and first expectation value would pin and
+// allocate (about 40 us each): taken from the handles destroyed before it, of
+// which up to kKits are kept, rings at their first size only; one when the
+// last handle goes.  A kit enters when its handle's stream has drained, so
+// nothing queued touches it.
+struct HandleKit {
+    ProgramRing ring;
+    void *io = nullptr;
+};
+struct HandleKits {
+    static constexpr size_t kKits = 4; // 192 KiB pinned and 128 KiB of device memory each
+    std::mutex mu;
+    std::vector<HandleKit> kept;
+    int live = 0; // handles
+};
+
 struct pl_sv {
     int n = 0;
     int dtype = PL_C128;
@@ -295,6 +311,63 @@ inline void *buf(pl_sv *h, Buf purpose, size_t bytes) {
         b.second = sz;
     }
     return b.first;
+}
+
+inline HandleKits &handle_kits() {
+    static HandleKits *kits = new HandleKits; // never destroyed: the runtime may be gone by then
+    return *kits;
+}
+inline void free_kit(HandleKit &k) {
+    (void)hipFree(k.ring.dev);
+    for (void *p : {k.ring.host, k.io}) {
+        if (p) {
+            (void)hipHostFree(p);
+        }
+    }
+    for (hipEvent_t e : k.ring.ev) {
+        if (e) {
+            (void)hipEventDestroy(e);
+        }
+    }
+    k = HandleKit{};
+}
+inline void take_kit(pl_sv *h) {
+    HandleKits &kits = handle_kits();
+    const std::lock_guard<std::mutex> lock(kits.mu);
+    kits.live++;
+    if (!kits.kept.empty()) {
+        h->ring = kits.kept.back().ring;
+        h->io_host = kits.kept.back().io;
+        kits.kept.pop_back();
+    }
+}
+// drained: nothing queued on h's stream uses the kit any more
+inline void return_kit(pl_sv *h, bool drained) {
+    HandleKit k{h->ring, h->io_host};
+    k.ring.seg = 0;
+    k.ring.used = 0;
+    std::fill(k.ring.busy, k.ring.busy + ProgramRing::kSegs, false);
+    h->ring = ProgramRing{};
+    h->io_host = nullptr;
+    const bool usual = drained && k.ring.seg_bytes <= ProgramRing::kSegBytes && (k.ring.dev || k.io);
+    std::vector<HandleKit> out;
+    HandleKits &kits = handle_kits();
+    {
+        const std::lock_guard<std::mutex> lock(kits.mu);
+        kits.live--;
+        if (usual && kits.kept.size() < (kits.live > 0 ? HandleKits::kKits : 1)) {
+            kits.kept.push_back(k);
+        } else {
+            out.push_back(k);
+        }
+        while (kits.live == 0 && kits.kept.size() > 1) {
+            out.push_back(kits.kept.back());
+            kits.kept.pop_back();
+        }
+    }
+    for (HandleKit &o : out) {
+        free_kit(o);
+    }
 }
 
 // The handle's pinned area (kIoBytes), nullptr where none can be had.  Used

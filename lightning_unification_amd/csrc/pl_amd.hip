@@ -1972,6 +1972,7 @@ int pl_sv_create(int num_qubits, int dtype, pl_sv_t *out) {
             throw DeviceError(std::string("hipMalloc of the state failed: ") + hipGetErrorString(e));
         }
         pl_sv *raw = h.release();
+        take_kit(raw);
         if (pl_sv_reset(raw) != PL_OK) {
             const std::string msg = g_err;
             pl_sv_destroy(raw);
@@ -1986,22 +1987,11 @@ int pl_sv_destroy(pl_sv_t h) {
         if (!h) {
             return;
         }
-        (void)hipStreamSynchronize(h->stream);
+        const bool drained = hipStreamSynchronize(h->stream) == hipSuccess;
         for (void *p : h->pool) {
             (void)hipFree(p);
         }
-        (void)hipFree(h->ring.dev);
-        if (h->ring.host) {
-            (void)hipHostFree(h->ring.host);
-        }
-        for (hipEvent_t e : h->ring.ev) {
-            if (e) {
-                (void)hipEventDestroy(e);
-            }
-        }
-        if (h->io_host) {
-            (void)hipHostFree(h->io_host);
-        }
+        return_kit(h, drained);
         (void)hipFree(h->red);
         (void)hipFree(h->staging);
         for (auto &b : h->bufs) {

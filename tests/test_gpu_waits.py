@@ -2,7 +2,7 @@
 
 Calls after which the state's memory may be read from any stream: the tiled
 executor and pl_sv_device_ptr with gates queued.  The engine's stream does not
-order itself against others, so the amplitudes copied on torch's stream right
+order itself against others, so the amplitudes copied on the null stream right
 behind the call must be the ones the engine's own wait gives.
 
 Calls that refuse their input with a copy of the caller's memory queued: the
@@ -16,35 +16,30 @@ from lightning_unification_amd.circuits import Tape, random_layers
 pytestmark = pytest.mark.gpu
 
 
-class _Memory:
-    def __init__(self, sv, ptr):
-        self.sv = sv
-        self.__cuda_array_interface__ = {"shape": (sv.size,), "typestr": sv.dtype.str, "version": 3,
-                                         "data": (ptr, False)}
-
-
 @pytest.mark.parametrize("dtype,n", [(np.complex128, 25), (np.complex64, 22), (np.complex64, 24)])
 @pytest.mark.parametrize("how", ["tiled", "deferred"])
 def test_state_is_final_when_the_call_returns(dtype, n, how):
-    import torch
+    import ctypes
     from lightning_unification_amd import capi
+    hip = ctypes.CDLL("libamdhip64.so")
+    hip.hipMemcpy.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int]
     tape = random_layers(n, 8, seed=3)
     print(f"final on return: {how} n={n} {np.dtype(dtype).name}", flush=True)
-    with capi.DeviceStateVector(n, dtype) as sv:
-        view = torch.as_tensor(_Memory(sv, sv.device_ptr()), device="cuda")
-        view.clone()  # torch's allocation for the copy below
-        torch.cuda.synchronize()
+    with capi.DeviceStateVector(n, dtype) as sv, capi.DeviceStateVector(n, dtype) as copy:
+        to = copy.device_ptr()
+        copy.synchronize()
+        at = sv.device_ptr()
         if how == "tiled":
             sv.apply_tape_tiled(tape)
         else:
             sv.set_deferred(True)
             sv.apply_tape(tape)
-            sv.device_ptr()
-        got = view.clone()
-        torch.cuda.synchronize()
-        sv.synchronize()
-        assert torch.equal(got, view)
-        assert abs(float(torch.linalg.vector_norm(got.abs().double())) - 1) < 1e-4
+            at = sv.device_ptr()
+        # on the null stream, which the engine's streams do not wait for
+        assert hip.hipMemcpy(to, at, sv.size * np.dtype(dtype).itemsize, 3) == 0  # hipMemcpyDeviceToDevice
+        assert hip.hipDeviceSynchronize() == 0
+        assert copy.distance(sv) == 0
+        assert abs(copy.norm2() - 1) < 1e-4
 
 
 @pytest.mark.parametrize("dtype", [np.complex128, np.complex64])
@@ -98,3 +93,27 @@ def test_programs_round_the_ring(oracle, n, layers, times):
             sv.apply_tape(tape)
             oracle.apply_tape(exp, tape)
         assert rel_err(sv.state(), exp, floor=0.1) < 1e-12 * times
+
+
+def test_a_handle_per_circuit_in_several_threads(oracle):
+    """Handles that come and go take over the upload ring and the pinned area of
+    earlier ones; four threads at once, tapes that grow the ring among them,
+    give the oracle's states and expectation values."""
+    from concurrent.futures import ThreadPoolExecutor
+    from lightning_unification_amd import capi
+    from lightning_unification_amd.circuits import random_hamiltonian
+
+    def circuit(i):
+        n = 4 + i % 9
+        tape, ham = random_layers(n, 40 if i % 8 == 7 else 2, seed=i), random_hamiltonian(n, 6, seed=i)
+        exp = np.zeros(1 << n, np.complex128)
+        exp[0] = 1
+        oracle.apply_tape(exp, tape)
+        with capi.DeviceStateVector(n) as sv:
+            sv.apply_tape(tape)
+            e = sv.expval(ham)
+            return rel_err(sv.state(), exp, floor=0.1), abs(e - oracle.expval(exp, ham))
+
+    with ThreadPoolExecutor(4) as pool:
+        for err, de in pool.map(circuit, range(64)):
+            assert err < 1e-12 and de < 1e-12
