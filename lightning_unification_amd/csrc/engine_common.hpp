@@ -313,6 +313,15 @@ inline void *buf(pl_sv *h, Buf purpose, size_t bytes) {
     return b.first;
 }
 
+// Gives a buffer back that has grown past `keep` bytes.
+inline void trim_buf(pl_sv *h, Buf purpose, size_t keep) {
+    if (h->bufs.size() > static_cast<size_t>(purpose) && h->bufs[purpose].second > keep) {
+        (void)hipStreamSynchronize(h->stream);
+        (void)hipFree(h->bufs[purpose].first);
+        h->bufs[purpose] = {nullptr, 0};
+    }
+}
+
 inline HandleKits &handle_kits() {
     static HandleKits *kits = new HandleKits; // never destroyed: the runtime may be gone by then
     return *kits;

@@ -39,7 +39,7 @@ namespace plamd {
 // walker on one XCD where the grid allows it, since they read the same lambda
 // tiles.  Group grp takes KH observables.  The group numbered `writer` writes
 // lambda to lam_out (which may be lam_in when no other group reads it).
-// partial[(((slot0 + slot) * NC + c) * K + k) * W + w], W walkers.
+// partial[(((slot0 + slot) * NC + c) * pk + k - pk0) * W + w], W walkers.
 template <class T, int NW, int KH, bool FULL>
 __global__ __launch_bounds__(64 * NW, 4) void k_sweep(const SweepArgs<T> A, const SweepStep *__restrict__ prog) {
     constexpr int NC = FULL ? kSweepFull : kSweepReal;
@@ -312,14 +312,18 @@ __global__ __launch_bounds__(64 * NW, 4) void k_sweep(const SweepArgs<T> A, cons
             t += sums[v * nsum + i];
         }
         if (kk < nk) {
-            A.partial[((static_cast<uint64_t>(A.slot0 + slot) * NC + c) * A.K + k0 + kk) * A.W + w] = t;
+            A.partial[((static_cast<uint64_t>(A.slot0 + slot) * NC + c) * A.pk + k0 - A.pk0 + kk) * A.W + w] = t;
         }
     }
 }
 
-// out[v] = sum of partial[v * W .. + W), one wavefront per value, fixed order
-static __global__ __launch_bounds__(64) void k_sweep_sums(const double *__restrict__ partial, int W,
+// launch_sweep_sums: one wavefront per value, fixed order
+static __global__ __launch_bounds__(64) void k_sweep_sums(const double *__restrict__ partial, int W, int pk, int pk0, int K,
                                                           double *__restrict__ out) {
+    const int sc = static_cast<int>(blockIdx.x) / pk, k = pk0 + static_cast<int>(blockIdx.x) % pk;
+    if (k >= K) {
+        return;
+    }
     const double *p = partial + static_cast<uint64_t>(blockIdx.x) * W;
     double s = 0;
     for (int i = threadIdx.x; i < W; i += 64) {
@@ -327,7 +331,7 @@ static __global__ __launch_bounds__(64) void k_sweep_sums(const double *__restri
     }
     s = wave_sum(s);
     if (threadIdx.x == 0) {
-        out[blockIdx.x] = s;
+        out[static_cast<uint64_t>(sc) * K + k] = s;
     }
 }
 

@@ -1631,7 +1631,11 @@ struct Drain {
 // States up to this size keep a second lambda, so that every observable group
 // of a pass can run at once; larger ones fill the device group by group.
 constexpr size_t kSweepTwoLambdas = size_t{64} << 20;
-constexpr size_t kSweepPartBytes = size_t{64} << 20; // partial sums held before they are added up
+// Partial sums: those of one pass's slots, or of more where they are small,
+// are held before they are added up.  Observables beyond what a launch takes
+// share their space, so it stays below 32 MiB whatever their number.
+constexpr size_t kSweepPartBytes = size_t{4} << 20;
+constexpr size_t kSweepKeptBytes = size_t{32} << 20; // of a buffer, between calls
 
 template <class T, bool FULL, class Emit>
 void backward_sweep(Engine<T> &E, const SweepTape &t, v2<T> *lam, const std::vector<v2<T> *> &hs, int ntp,
@@ -1740,19 +1744,34 @@ void backward_sweep(Engine<T> &E, const SweepTape &t, v2<T> *lam, const std::vec
     for (const auto &s : steps) {
         nslots_all += !s.big && !s.train.empty() ? 1 : 0;
     }
-    const size_t slot_bytes = size_t(NC) * K * W * sizeof(double);
+    // where the groups of a pass share its launch (or there is one), every
+    // observable has its place in the partial sums and they are added up when
+    // `cap` slots are full; else after each launch
+    const bool shared = two || ngrp == 1;
+    const int pk = shared ? K : KH;
+    const size_t slot_bytes = size_t(NC) * pk * W * sizeof(double);
     const size_t cap = std::min<size_t>(std::max<size_t>(nslots_all, 1),
                                         std::max<size_t>(kSweepSlots, kSweepPartBytes / slot_bytes));
     auto *part = static_cast<double *>(buf(h, kBufSweepPart, cap * slot_bytes));
     auto *dsums = static_cast<double *>(buf(h, kBufSweepSums, std::max<size_t>(nslots_all, 1) * NC * K * sizeof(double)));
+    struct Trim {
+        pl_sv *h;
+        ~Trim() {
+            trim_buf(h, kBufSweepPart, kSweepKeptBytes);
+            trim_buf(h, kBufSweepSums, kSweepKeptBytes);
+        }
+    } trim{h};
     std::vector<int> slot_step; // step of every slot so far
     size_t reduced = 0;         // slots already added up
+    auto add_up = [&](size_t first, size_t m, int pk0) {
+        HIP_OK(launch_sweep_sums(part, W, static_cast<unsigned>(m * NC), pk, pk0, K, dsums + first * NC * K, h->stream));
+    };
     auto reduce = [&] {
         const size_t m = slot_step.size() - reduced;
-        if (m > 0) {
-            HIP_OK(launch_sweep_sums(part, W, static_cast<unsigned>(m * NC * K), dsums + reduced * NC * K, h->stream));
-            reduced = slot_step.size();
+        if (shared && m > 0) {
+            add_up(reduced, m, 0);
         }
+        reduced = slot_step.size();
     };
 
     SweepScheduler sched(E.n(), bits, low, steps);
@@ -1799,14 +1818,21 @@ void backward_sweep(Engine<T> &E, const SweepTape &t, v2<T> *lam, const std::vec
         sweep_program(steps, ps, low, tb, RB, false, prog);
         const int ns = static_cast<int>(prog.size());
         SweepArgs<T> a{lam, other, dhs, K, 0, 0, ngrp - 1, W, ntiles, {}, pb.put(prog), ns, static_cast<int>(mine),
-                       static_cast<int>(slot0), part};
+                       static_cast<int>(slot0), part, pk, 0};
         a.geo.bits = bits;
         a.geo.low = low;
         std::copy(ps.hb.begin(), ps.hb.end(), a.geo.hb);
         for (int g0 = 0; g0 < ngrp; g0 += per_launch) {
             a.grp0 = g0;
             a.ngrp = std::min(per_launch, ngrp - g0);
+            a.pk0 = shared ? 0 : g0 * KH;
             HIP_OK(launch_sweep<T>(waves, KH, FULL, a, h->stream));
+            if (!shared && mine > 0) {
+                add_up(reduced, mine, a.pk0);
+            }
+        }
+        if (!shared) {
+            reduced = slot_step.size();
         }
         std::swap(lam, other);
     }

@@ -53,8 +53,9 @@ template hipError_t launch_pass<double>(int, v2<double> *, uint64_t, const Sweep
                                         hipStream_t);
 template hipError_t launch_sweep<double>(int, int, bool, const SweepArgs<double> &, hipStream_t);
 
-hipError_t launch_sweep_sums(const double *partial, int W, unsigned count, double *out, hipStream_t s) {
-    hipLaunchKernelGGL(k_sweep_sums, dim3(count), dim3(64), 0, s, partial, W, out);
+hipError_t launch_sweep_sums(const double *partial, int W, unsigned count, int pk, int pk0, int K, double *out,
+                             hipStream_t s) {
+    hipLaunchKernelGGL(k_sweep_sums, dim3(count * static_cast<unsigned>(pk)), dim3(64), 0, s, partial, W, pk, pk0, K, out);
     return hipGetLastError();
 }
 #else

@@ -69,6 +69,7 @@ template <class T> struct SweepArgs {
     const SweepStep *prog;
     int nsteps, nslots, slot0;
     double *partial;
+    int pk, pk0; // observables per slot of `partial`, the first one's number
 };
 
 // One launch of args.ngrp observable groups (kh observables each) with `waves`
@@ -78,7 +79,9 @@ template <class T> hipError_t launch_sweep(int waves, int kh, bool full, const S
 template <class T>
 hipError_t launch_pass(int waves, v2<T> *sv, uint64_t ntiles, const SweepGeom &geo, const SweepStep *prog, int nsteps,
                        hipStream_t s);
-// out[v] = sum of partial[v W .. (v + 1) W), v < count
-hipError_t launch_sweep_sums(const double *partial, int W, unsigned count, double *out, hipStream_t s);
+// Sums over the W walkers of partial[sc][k][W], sc < count, k < pk:
+// out[sc K + pk0 + k] where that is an observable
+hipError_t launch_sweep_sums(const double *partial, int W, unsigned count, int pk, int pk0, int K, double *out,
+                             hipStream_t s);
 
 } // namespace plamd

@@ -74,3 +74,79 @@ def test_more_trainable_steps_than_a_pass_has_slots(oracle):
     obs = [pauli_word("XX", [0, 3]), Obs.named("PauliY", [5])]
     with capi.DeviceStateVector.from_array(s) as sv:
         assert rel_err(sv.adjoint_jacobian(tape, obs, tp), oracle.adjoint(s, tape, obs, tp)) < 1e-12
+
+
+def _wide_tape(n, nops, seed):
+    """Entangled, with a parametrised gate in every step."""
+    rs, tape = np.random.default_rng(seed), Tape()
+    for i in range(nops):
+        a, b = rs.choice(n, 2, replace=False).tolist()
+        g = ["CRX", "IsingXX", "CRZ", "CRY"][i % 4]
+        tape.add(g, [a, b], [0.2 + 0.1 * i])
+    return tape
+
+
+def _adjoint_pairwise(oracle, lam, tape, words):
+    """The Jacobian of Pauli words (letters, wires), one parameter an operation,
+    summed pairwise: at 2^23 coherent terms the oracle's running sum is 1e-11 off."""
+    def gates(ops):
+        t = Tape()
+        for op in ops:
+            t.add(*op)
+        return t
+
+    hs = []
+    for letters, wires in words:
+        hs.append(lam.copy())
+        oracle.apply_tape(hs[-1], gates([("Pauli" + a, [w]) for a, w in zip(letters, wires)]))
+    lam, jac = lam.copy(), np.zeros((len(words), len(tape.ops)))
+    for i in reversed(range(len(tape.ops))):
+        name, wires, _, params = tape.ops[i]
+        mu = lam.copy()
+        scale = oracle.apply_generator(mu, name, wires)
+        jac[:, i] = [-2 * scale * np.sum(np.conj(h) * mu).imag for h in hs]
+        for v in [lam] + hs:
+            oracle.apply_tape(v, gates([(name, wires, params, True)]))
+    return jac
+
+
+@pytest.mark.parametrize("dtype,n", [(np.complex128, 23), (np.complex64, 24)])
+def test_groups_of_a_large_state_one_by_one(oracle, dtype, n):
+    """Past 64 MiB a state has one lambda: each group of observables is swept
+    from it and the last one writes it.  Three and five observables, in pairs
+    with one left over, over several passes, on a state whose wires all differ."""
+    from lightning_unification_amd import capi
+    prep, tape = Tape(), _wide_tape(n, 8, 5)
+    for w in range(n):
+        prep.add("RY", [w], [0.4 + 0.1 * w])
+        prep.add("RZ", [w], [0.3 * w])
+    s = np.zeros(1 << n, np.complex128)
+    s[0] = 1
+    oracle.apply_tape(s, prep)
+    oracle.apply_tape(s, tape)
+    used = [w for op in tape.ops for w in op[1]]
+    words = [("Z", [used[1]]), ("XZ", [used[2], used[5]]), ("Y", [used[7]]), ("X", [used[9]]),
+             ("YX", [used[12], used[15]])]
+    exp = _adjoint_pairwise(oracle, s, tape, words)
+    assert np.sum(np.abs(exp) > 1e-3) >= 5  # something to compare
+    tol = 1e-12 if dtype == np.complex128 else 5e-5
+    print(f"group by group: n={n} {np.dtype(dtype).name}", flush=True)
+    obs = [pauli_word(letters, wires) for letters, wires in words]
+    with capi.DeviceStateVector.from_array(s.astype(dtype)) as sv:
+        for k in (3, 5):
+            assert np.max(np.abs(sv.adjoint_jacobian(tape, obs[:k], list(range(8))) - exp[:k])) < tol
+
+
+def test_partial_sums_are_added_up_during_the_sweep(oracle):
+    """More trainable steps than the partial sums of 64 observables have room
+    for at once."""
+    from lightning_unification_amd import capi
+    n = 16
+    tape = _wide_tape(n, 100, 8)
+    s = random_state(n, 4)
+    oracle.apply_tape(s, tape)
+    obs = [Obs.named("PauliZ", [k % n]) if k < n else pauli_word("XY", [k % n, (k + 1 + k // n) % n])
+           for k in range(64)]
+    with capi.DeviceStateVector.from_array(s) as sv:
+        assert rel_err(sv.adjoint_jacobian(tape, obs, list(range(100))),
+                       oracle.adjoint(s, tape, obs, list(range(100)))) < 1e-12
