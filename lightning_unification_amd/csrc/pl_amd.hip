@@ -895,6 +895,16 @@ template <class T> struct Engine {
         return {r.x, r.y};
     }
 
+    // <a|b> left in device memory at *slot, ordered on the engine's stream with
+    // no wait; part holds kReduceBlocks partials and must not overlap slot.
+    void dot_to(const V *a, const V *b, double2 *part, double2 *slot) {
+        const unsigned grid = std::min<unsigned>(grid_for(len(), 1, 4), kReduceBlocks);
+        hipLaunchKernelGGL((k_dot<T>), dim3(grid), dim3(kBlock), 0, h->stream, a, b, len(), part);
+        HIP_OK(hipGetLastError());
+        hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(kBlock), 0, h->stream, part, (int)grid, slot);
+        HIP_OK(hipGetLastError());
+    }
+
     // sum_t c_t <psi|P_t|psi> over Pauli words, grouped by x-mask
     // High bits per Pauli tile: 10 where a workgroup's LDS holds a tile of
     // 2^13 amplitudes (fewer passes), else 8.
@@ -1761,6 +1771,17 @@ void backward_sweep(Engine<T> &E, const SweepTape &t, v2<T> *lam, const std::vec
             trim_buf(h, kBufSweepSums, kSweepKeptBytes);
         }
     } trim{h};
+    // <h_k|G lambda> of operations applied state by state, read back at the end
+    // with the sums: a wait each would cost what their launches do
+    size_t ndots = 0;
+    for (const auto &s : steps) {
+        ndots += s.big ? s.train.size() * K : 0;
+    }
+    double2 *dots = nullptr;
+    if (ndots > 0) {
+        dots = reinterpret_cast<double2 *>(reduce_buf(h, (kReduceBlocks + ndots) * sizeof(double2)));
+    }
+    std::vector<SweepTrain> dot_train; // K dots each
     std::vector<int> slot_step; // step of every slot so far
     size_t reduced = 0;         // slots already added up
     auto add_up = [&](size_t first, size_t m, int pk0) {
@@ -1792,8 +1813,9 @@ void backward_sweep(Engine<T> &E, const SweepTape &t, v2<T> *lam, const std::vec
                 T s = 0;
                 E.apply(lower_generator<T>(E.n(), t.ids[i], w, t.nwires[i], false, &s), mu);
                 for (int k = 0; k < K; k++) {
-                    emit(tr.row, k, E.dot(hs[k], mu), tr.scale);
+                    E.dot_to(hs[k], mu, dots, dots + kReduceBlocks + dot_train.size() * K + k);
                 }
+                dot_train.push_back(tr);
             }
             E.apply(ud, lam);
             for (V *s : hs) {
@@ -1841,7 +1863,17 @@ void backward_sweep(Engine<T> &E, const SweepTape &t, v2<T> *lam, const std::vec
     if (!sums.empty()) {
         HIP_OK(hipMemcpyAsync(sums.data(), dsums, sums.size() * sizeof(double), hipMemcpyDeviceToHost, h->stream));
     }
+    std::vector<double2> z(ndots);
+    if (ndots > 0) {
+        HIP_OK(hipMemcpyAsync(z.data(), dots + kReduceBlocks, ndots * sizeof(double2), hipMemcpyDeviceToHost,
+                              h->stream));
+    }
     HIP_OK(hipStreamSynchronize(h->stream));
+    for (size_t i = 0; i < dot_train.size(); i++) {
+        for (int k = 0; k < K; k++) {
+            emit(dot_train[i].row, k, std::complex<double>(z[i * K + k].x, z[i * K + k].y), dot_train[i].scale);
+        }
+    }
     for (size_t sl = 0; sl < slot_step.size(); sl++) {
         const SweepOp &op = steps[slot_step[sl]];
         for (int k = 0; k < K; k++) {
