@@ -290,7 +290,7 @@ struct ScratchScope {
 
 // Device buffers kept by a handle between calls, one per purpose.
 enum Buf { kBufUniforms, kBufIndices, kBufBits, kBufCdfGroups, kBufCdfPrefix, kBufCdfTiles, kBufChainStart,
-           kBufScalar, kBufSweepPart, kBufSweepSums, kBufSweepStates, kBufProbs, kBufCount };
+           kBufScalar, kBufSweepPart, kBufSweepSums, kBufProbs, kBufCount };
 constexpr uint64_t kProbsKept = 4096; // bins of a marginal whose buffer stays with the handle
 
 // The handle's buffer for `purpose`, at least `bytes` long (grown when

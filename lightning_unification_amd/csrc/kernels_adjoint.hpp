@@ -317,6 +317,117 @@ __global__ __launch_bounds__(64 * NW, 4) void k_sweep(const SweepArgs<T> A, cons
     }
 }
 
+// One step by itself (SweepStepArgs), as it touches a part of the amplitudes
+// only and a pass would read and write them all, or where a launch costs less
+// than a pass's program.  Four states' loads are in flight before the stores.
+// OBS: states with room for their sums; four are an instance of their own, whose
+// registers let more wavefronts run.
+template <class T, int OBS, bool FULL, bool DENSE, bool TRAIN>
+__global__ __launch_bounds__(kBlock, 4) void k_sweep_step(const SweepStepArgs<T> A) {
+    constexpr int NC = FULL ? kSweepFull : kSweepReal;
+    constexpr int CH = OBS < 4 ? OBS : 4;
+    double acc[OBS][NC] = {};
+    auto mul2 = [](const dcx<double> &p, const double2 &x, const dcx<double> &q, const double2 &y) {
+        return v2<T>{static_cast<T>(rt_fma(p.r, x.x, rt_fma(-p.i, x.y, rt_fma(q.r, y.x, -q.i * y.y)))),
+                     static_cast<T>(rt_fma(p.r, x.y, rt_fma(p.i, x.x, rt_fma(q.r, y.y, q.i * y.x))))};
+    };
+    auto mul1 = [](const dcx<double> &p, const double2 &x) {
+        return v2<T>{static_cast<T>(rt_fma(p.r, x.x, -p.i * x.y)), static_cast<T>(rt_fma(p.r, x.y, p.i * x.x))};
+    };
+    const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kBlock;
+    for (uint64_t g = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x; g < A.nwork; g += stride) {
+        const uint64_t i0 = expand(g, A.geo), i1 = i0 ^ A.flip;
+        const bool odd = !DENSE && (__popcll(i0 & A.par) & 1);
+        const dcx<double> ph = odd ? A.u[3] : A.u[0];
+        const v2<T> a0 = A.lam[i0], b0 = DENSE ? A.lam[i1] : v2<T>{0, 0};
+        const double2 a{a0.x, a0.y}, b{b0.x, b0.y};
+        if (A.write_lam) {
+            if constexpr (DENSE) {
+                A.lam[i0] = mul2(A.u[0], a, A.u[1], b);
+                A.lam[i1] = mul2(A.u[2], a, A.u[3], b);
+            } else {
+                A.lam[i0] = mul1(ph, a);
+            }
+        }
+#pragma unroll
+        for (int k0 = 0; k0 < OBS; k0 += CH) {
+            v2<T> c0[CH], d0[CH];
+#pragma unroll
+            for (int j = 0; j < CH; j++) {
+                if (k0 + j < A.nk) {
+                    c0[j] = A.h[k0 + j][i0];
+                    if constexpr (DENSE) {
+                        d0[j] = A.h[k0 + j][i1];
+                    }
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < CH; j++) {
+                if (k0 + j >= A.nk) {
+                    continue;
+                }
+                const double2 c{c0[j].x, c0[j].y};
+                double *t = acc[k0 + j];
+                if constexpr (DENSE) {
+                    const double2 d{d0[j].x, d0[j].y};
+                    if constexpr (TRAIN) {
+                        t[0] = rt_fma(c.x, a.y, rt_fma(-c.y, a.x, t[0]));
+                        t[1] = rt_fma(d.x, b.y, rt_fma(-d.y, b.x, t[1]));
+                        t[2] = rt_fma(c.x, b.y, rt_fma(-c.y, b.x, rt_fma(d.x, a.y, rt_fma(-d.y, a.x, t[2]))));
+                        t[3] = rt_fma(c.x, b.x, rt_fma(c.y, b.y, rt_fma(-d.x, a.x, rt_fma(-d.y, a.y, t[3]))));
+                        if constexpr (FULL) {
+                            t[4] = rt_fma(c.x, a.x, rt_fma(c.y, a.y, t[4]));
+                            t[5] = rt_fma(d.x, b.x, rt_fma(d.y, b.y, t[5]));
+                            t[6] = rt_fma(c.x, b.x, rt_fma(c.y, b.y, rt_fma(d.x, a.x, rt_fma(d.y, a.y, t[6]))));
+                            t[7] = rt_fma(c.x, b.y, rt_fma(-c.y, b.x, rt_fma(-d.x, a.y, rt_fma(d.y, a.x, t[7]))));
+                        }
+                    }
+                    A.h[k0 + j][i0] = mul2(A.u[0], c, A.u[1], d);
+                    A.h[k0 + j][i1] = mul2(A.u[2], c, A.u[3], d);
+                } else {
+                    if constexpr (TRAIN) {
+                        const double im = rt_fma(c.x, a.y, -c.y * a.x);
+                        t[0] += odd ? 0.0 : im;
+                        t[1] += odd ? im : 0.0;
+                        if constexpr (FULL) {
+                            const double re = rt_fma(c.x, a.x, c.y * a.y);
+                            t[4] += odd ? 0.0 : re;
+                            t[5] += odd ? re : 0.0;
+                        }
+                    }
+                    A.h[k0 + j][i0] = mul1(ph, c);
+                }
+            }
+        }
+    }
+    if constexpr (TRAIN) {
+        __shared__ double wpart[kBlock / 64][OBS * NC];
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+        for (int k = 0; k < OBS; k++) {
+            if (k < A.nk) { // uniform
+#pragma unroll
+                for (int c = 0; c < NC; c += 4) {
+                    const double s = rt_sum4(acc[k][c], acc[k][c + 1], acc[k][c + 2], acc[k][c + 3]);
+                    if ((lane & 15) == 0) {
+                        wpart[wave][k * NC + c + rt_row(lane >> 4)] = s;
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        for (int i = threadIdx.x; i < A.nk * NC; i += kBlock) {
+            double s = wpart[0][i];
+#pragma unroll
+            for (int w = 1; w < kBlock / 64; w++) {
+                s += wpart[w][i];
+            }
+            const int k = i / NC, c = i % NC;
+            A.partial[((static_cast<uint64_t>(A.slot) * NC + c) * A.pk + A.k0 + k) * gridDim.x + blockIdx.x] = s;
+        }
+    }
+}
+
 // launch_sweep_sums: one wavefront per value, fixed order
 static __global__ __launch_bounds__(64) void k_sweep_sums(const double *__restrict__ partial, int W, int pk, int pk0, int K,
                                                           double *__restrict__ out) {

@@ -8,6 +8,9 @@
 // HIP stream.  There is no CPU compute path: if the device work cannot be
 // enqueued the call fails with PL_ERR_DEVICE.
 #include "engine_common.hpp"
+
+#include <optional>
+
 #include "sweep.hpp"
 #include "kernels_reduce.hpp"
 #include "kernels_sample.hpp"
@@ -174,17 +177,19 @@ template <class T> constexpr int kSweepLow = std::is_same_v<T, double> ? 3 : 4; 
 // ended, a tape right behind another waited for it.
 class ProgramBuffer {
   public:
-    // longest: steps of any one program of the call, at most
-    ProgramBuffer(pl_sv *h, size_t longest) : h_(h), r_(h->ring) {
-        const size_t bytes = longest * sizeof(SweepStep);
+    // longest: steps of any one program of the call, at most; more: bytes
+    // that go with each
+    ProgramBuffer(pl_sv *h, size_t longest, size_t more = 0) : h_(h), r_(h->ring) {
+        const size_t bytes = longest * sizeof(SweepStep) + more;
         if (r_.seg_bytes < bytes) {
             reserve(std::max(bytes, ProgramRing::kSegBytes));
         }
     }
     bool ok() const { return r_.dev != nullptr; } // false: the device is full
-    // the device address of the steps, in place for work queued after this
-    const SweepStep *put(const std::vector<SweepStep> &steps) {
-        const size_t bytes = steps.size() * sizeof(SweepStep);
+    // the device address of the steps and, behind them, `more` (of a size that
+    // keeps the next program aligned), in place for work queued after this
+    const SweepStep *put(const std::vector<SweepStep> &steps, const void *more = nullptr, size_t more_bytes = 0) {
+        const size_t head = steps.size() * sizeof(SweepStep), bytes = head + more_bytes;
         if (bytes > r_.seg_bytes) {
             throw std::logic_error("a program longer than its steps and windows");
         }
@@ -195,10 +200,16 @@ class ProgramBuffer {
         auto *to = static_cast<unsigned char *>(r_.dev) + at;
         if (r_.host) {
             auto *from = static_cast<unsigned char *>(r_.host) + at;
-            std::memcpy(from, steps.data(), bytes);
+            std::memcpy(from, steps.data(), head);
+            if (more_bytes > 0) {
+                std::memcpy(from + head, more, more_bytes);
+            }
             HIP_OK(hipMemcpyAsync(to, from, bytes, hipMemcpyHostToDevice, h_->stream));
         } else {
-            HIP_OK(hipMemcpyAsync(to, steps.data(), bytes, hipMemcpyHostToDevice, h_->stream));
+            HIP_OK(hipMemcpyAsync(to, steps.data(), head, hipMemcpyHostToDevice, h_->stream));
+            if (more_bytes > 0) {
+                HIP_OK(hipMemcpyAsync(to + head, more, more_bytes, hipMemcpyHostToDevice, h_->stream));
+            }
             HIP_OK(hipStreamSynchronize(h_->stream));
         }
         r_.used += bytes;
@@ -671,10 +682,8 @@ template <class T> struct Engine {
             // passes refuse a tape as a whole, except below the smallest tile.
             if (low < 0 && (std::is_same_v<T, double> || n() < kTileFloatQubits)) {
                 const int launches = apply_passes(sv, t, n() >= kTpMinBits);
-                if (launches >= 0) {
-                    HIP_OK(hipStreamSynchronize(h->stream));
-                    return launches;
-                }
+                HIP_OK(hipStreamSynchronize(h->stream));
+                return launches;
             }
             if (n() < kTpMinBits) {
                 int launches = 0;
@@ -793,8 +802,9 @@ template <class T> struct Engine {
     }
 
     // ---- forward passes on register tiles (kernels_pass.hpp) ------------------
-    // Applies a tape; returns the number of launches, or -1, with nothing done,
-    // where there is no memory for the passes' programs.  The operations
+    // Applies a tape; returns the number of launches.  A pass's steps are
+    // applied one by one where that costs less (SweepCost), or where there is
+    // no memory for programs.  The operations
     // before one that does not lower are applied before its error leaves, as
     // gate by gate, or none (whole).  The device is waited for only
     // where the program ring has gone round (ProgramBuffer).
@@ -838,7 +848,8 @@ template <class T> struct Engine {
                 }
                 parts.assign(1, op);
             }
-            for (const SweepOp &op : parts) {
+            for (SweepOp &op : parts) {
+                op.alone = sweep_forward_alone(op, n(), std::is_same_v<T, double>);
                 builder.add(op);
             }
         }
@@ -852,26 +863,40 @@ template <class T> struct Engine {
             SweepScheduler sched(n(), bits, low, steps);
             SweepPass ps;
             std::vector<SweepStep> prog;
-            ProgramBuffer pb(h, 2 * std::min(steps.size(), kSweepLookahead)); // a step and its window
-            if (!pb.ok()) {
-                return -1;
-            }
+            std::optional<ProgramBuffer> pb; // at the first pass that uploads one
             SweepGeom geo{};
             geo.bits = bits;
             geo.low = low;
             while (sched.next(ps)) {
-                launches++;
                 if (ps.big) {
-                    const int i = steps[ps.ops[0]].tape;
+                    launches++;
+                    const SweepOp &op = steps[ps.ops[0]];
+                    if (!op.big) {
+                        apply(sweep_group<T>(op), sv);
+                        continue;
+                    }
+                    const int i = op.tape;
                     gate(sv, t.ids[i], t.wires + woff[i], t.nwires[i], t.inverse[i] != 0, t.params + poff[i],
                          t.nparams[i]);
+                    continue;
+                }
+                const SweepCost cost = sweep_forward_us(steps, ps, n(), std::is_same_v<T, double>, !pb);
+                if (cost.together < cost.alone && !pb) {
+                    pb.emplace(h, sweep_longest(steps, true));
+                }
+                if (cost.alone <= cost.together || !pb->ok()) {
+                    for (int i : ps.ops) {
+                        apply(sweep_group<T>(steps[i]), sv);
+                    }
+                    launches += static_cast<int>(ps.ops.size());
                     continue;
                 }
                 prog.clear();
                 sweep_program(steps, ps, low, tb, RB, true, prog);
                 std::copy(ps.hb.begin(), ps.hb.end(), geo.hb);
-                HIP_OK(launch_pass<T>(1 << lw, sv, len() >> bits, geo, pb.put(prog), static_cast<int>(prog.size()),
+                HIP_OK(launch_pass<T>(1 << lw, sv, len() >> bits, geo, pb->put(prog), static_cast<int>(prog.size()),
                                       h->stream));
+                launches++;
             }
         }
         if (refused) {
@@ -1579,11 +1604,12 @@ void defer_gate(pl_sv_t h, int id, const int *wires, int nw, bool inverse, const
     }
 }
 
-// Tapes of at least this many operations run as passes on register tiles
-// (apply_passes); shorter ones gate by gate, a launch each and no program to
-// upload.  Three gates at 6 qubits: 34 us by either; five at 9 qubits 40 us
-// gate by gate, 38 us as a pass; 19 at 28 qubits 22.5 and 3.5 ms.
-constexpr int kPassMinOps = 4;
+// Tapes of at least this many operations are planned as passes on register
+// tiles (apply_passes); shorter ones go gate by gate.  On states below
+// kPassMinBytes a pass's program gains from about six launches on (four RX: 34 us
+// gate by gate and 38 as a pass at 14 qubits complex128, 51 and 41 at 20).
+constexpr int kPassMinOps = 4, kPassMinOpsSmall = 6;
+constexpr size_t kPassMinBytes = size_t{16} << 20;
 
 // Engine of the handle's precision, exceptions propagate
 template <class F> void dispatch_or_throw(pl_sv_t h, F &&f) {
@@ -1695,7 +1721,8 @@ void backward_sweep(Engine<T> &E, const SweepTape &t, v2<T> *lam, const std::vec
             continue;
         }
         if (sweep_expand_op(ud, train ? &g : nullptr, tr, parts)) {
-            for (const SweepOp &op : parts) {
+            for (SweepOp &op : parts) {
+                op.alone = sweep_backward_alone(op, E.n(), std::is_same_v<T, double>, static_cast<int>(hs.size()));
                 builder.add(op);
             }
             continue;
@@ -1741,13 +1768,7 @@ void backward_sweep(Engine<T> &E, const SweepTape &t, v2<T> *lam, const std::vec
     ScratchScope sc(h);
     V *other = two ? static_cast<V *>(sc.get()) : lam;
     V *mu = nullptr;
-    auto **dhs = static_cast<V **>(buf(h, kBufSweepStates, K * sizeof(V *)));
-    Drain drain{h->stream}; // hs
-    HIP_OK(hipMemcpyAsync(dhs, hs.data(), K * sizeof(V *), hipMemcpyHostToDevice, h->stream));
-    ProgramBuffer pb(h, 4 * std::min(steps.size(), kSweepLookahead)); // a step with two flips, and its window
-    if (!pb.ok()) {
-        throw DeviceError("no device memory for the sweep's programs");
-    }
+    std::optional<ProgramBuffer> pb; // at the first pass
     std::vector<SweepStep> prog;
     // slots in flight: partial sums of `cap` slots before a reduction
     size_t nslots_all = 0;
@@ -1762,7 +1783,8 @@ void backward_sweep(Engine<T> &E, const SweepTape &t, v2<T> *lam, const std::vec
     const size_t slot_bytes = size_t(NC) * pk * W * sizeof(double);
     const size_t cap = std::min<size_t>(std::max<size_t>(nslots_all, 1),
                                         std::max<size_t>(kSweepSlots, kSweepPartBytes / slot_bytes));
-    auto *part = static_cast<double *>(buf(h, kBufSweepPart, cap * slot_bytes));
+    const size_t alone_bytes = size_t(NC) * std::min(K, kStepObs) * W * sizeof(double); // a step by itself
+    auto *part = static_cast<double *>(buf(h, kBufSweepPart, std::max(cap * slot_bytes, alone_bytes)));
     auto *dsums = static_cast<double *>(buf(h, kBufSweepSums, std::max<size_t>(nslots_all, 1) * NC * K * sizeof(double)));
     struct Trim {
         pl_sv *h;
@@ -1784,15 +1806,56 @@ void backward_sweep(Engine<T> &E, const SweepTape &t, v2<T> *lam, const std::vec
     std::vector<SweepTrain> dot_train; // K dots each
     std::vector<int> slot_step; // step of every slot so far
     size_t reduced = 0;         // slots already added up
-    auto add_up = [&](size_t first, size_t m, int pk0) {
+    auto add_up = [&](size_t first, size_t m, int pk0, int pk) {
         HIP_OK(launch_sweep_sums(part, W, static_cast<unsigned>(m * NC), pk, pk0, K, dsums + first * NC * K, h->stream));
     };
     auto reduce = [&] {
         const size_t m = slot_step.size() - reduced;
         if (shared && m > 0) {
-            add_up(reduced, m, 0);
+            add_up(reduced, m, 0, K);
         }
         reduced = slot_step.size();
+    };
+
+    // step i on lambda and every h, by itself
+    auto step_alone = [&](int i) {
+        const SweepOp &s = steps[i];
+        const SweepLone l = sweep_lone(s);
+        const bool train = !s.train.empty();
+        SweepStepArgs<T> a{};
+        for (uint64_t b = l.pins; b; b &= b - 1) {
+            a.geo.pos[a.geo.nb++] = __builtin_ctzll(b);
+        }
+        a.geo.fixed = l.value;
+        a.lam = lam;
+        a.nwork = E.len() >> a.geo.nb;
+        a.flip = l.flip;
+        a.par = l.par;
+        for (int j = 0; j < 4; j++) {
+            a.u[j] = {s.u[j].real(), s.u[j].imag()};
+        }
+        if (train) {
+            if (slot_step.size() - reduced + 1 > cap) {
+                reduce();
+            }
+            a.partial = part;
+            a.slot = static_cast<int>(slot_step.size() - reduced);
+            slot_step.push_back(i);
+        }
+        for (int k0 = 0; k0 < K; k0 += kStepObs) {
+            a.nk = std::min(kStepObs, K - k0);
+            a.write_lam = k0 + a.nk == K;
+            std::copy(hs.begin() + k0, hs.begin() + k0 + a.nk, a.h);
+            a.pk = shared ? K : a.nk;
+            a.k0 = shared ? k0 : 0;
+            HIP_OK(launch_sweep_step<T>(W, FULL, a, h->stream));
+            if (train && !shared) {
+                add_up(reduced, 1, k0, a.nk);
+            }
+        }
+        if (!shared) {
+            reduced = slot_step.size();
+        }
     };
 
     SweepScheduler sched(E.n(), bits, low, steps);
@@ -1801,6 +1864,10 @@ void backward_sweep(Engine<T> &E, const SweepTape &t, v2<T> *lam, const std::vec
         if (ps.big) {
             // lambda and every h op by op: dots with mu = G lambda first
             const SweepOp &op = steps[ps.ops[0]];
+            if (!op.big) {
+                step_alone(ps.ops[0]);
+                continue;
+            }
             const int i = op.tape;
             const int *w = t.wires + woff[i];
             const GroupOp<T> ud = lower_gate_as<T>(E.n(), t.ids[i], w, t.nwires[i], t.inverse[i] == 0,
@@ -1823,6 +1890,16 @@ void backward_sweep(Engine<T> &E, const SweepTape &t, v2<T> *lam, const std::vec
             }
             continue;
         }
+        const SweepCost cost = sweep_backward_us(steps, ps, E.n(), std::is_same_v<T, double>, K, !pb);
+        if (cost.together < cost.alone && !pb) {
+            pb.emplace(h, sweep_longest(steps, false), K * sizeof(V *));
+        }
+        if (cost.alone <= cost.together || !pb->ok()) {
+            for (int i : ps.ops) {
+                step_alone(i);
+            }
+            continue;
+        }
         size_t mine = 0;
         for (int i : ps.ops) {
             mine += steps[i].train.empty() ? 0 : 1;
@@ -1839,7 +1916,9 @@ void backward_sweep(Engine<T> &E, const SweepTape &t, v2<T> *lam, const std::vec
         prog.clear();
         sweep_program(steps, ps, low, tb, RB, false, prog);
         const int ns = static_cast<int>(prog.size());
-        SweepArgs<T> a{lam, other, dhs, K, 0, 0, ngrp - 1, W, ntiles, {}, pb.put(prog), ns, static_cast<int>(mine),
+        const SweepStep *dprog = pb->put(prog, hs.data(), K * sizeof(V *));
+        auto *dhs = reinterpret_cast<V *const *>(dprog + ns); // the states' addresses
+        SweepArgs<T> a{lam, other, dhs, K, 0, 0, ngrp - 1, W, ntiles, {}, dprog, ns, static_cast<int>(mine),
                        static_cast<int>(slot0), part, pk, 0};
         a.geo.bits = bits;
         a.geo.low = low;
@@ -1850,7 +1929,7 @@ void backward_sweep(Engine<T> &E, const SweepTape &t, v2<T> *lam, const std::vec
             a.pk0 = shared ? 0 : g0 * KH;
             HIP_OK(launch_sweep<T>(waves, KH, FULL, a, h->stream));
             if (!shared && mine > 0) {
-                add_up(reduced, mine, a.pk0);
+                add_up(reduced, mine, a.pk0, pk);
             }
         }
         if (!shared) {
@@ -2203,8 +2282,8 @@ int pl_sv_apply_ops(pl_sv_t h, int nops, const int *ids, const int *nwires, cons
         });
     }
     return dispatch(h, [&](auto &E) {
-        if (nops >= kPassMinOps &&
-            E.apply_passes(E.psi(), TapeView{nops, ids, nwires, wires, inverse, nparams, params}) >= 0) {
+        if (nops >= (h->state_bytes() >= kPassMinBytes ? kPassMinOps : kPassMinOpsSmall)) {
+            E.apply_passes(E.psi(), TapeView{nops, ids, nwires, wires, inverse, nparams, params});
             return;
         }
         for (int i = 0, wo = 0, po = 0; i < nops; i++) {

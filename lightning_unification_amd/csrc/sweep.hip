@@ -30,6 +30,31 @@ template <class T> hipError_t launch_sweep(int waves, int kh, bool full, const S
     return waves == 4 ? go(I4{}, I1{}, I0{}) : waves == 2 ? go(I2{}, I1{}, I0{}) : go(I1{}, I1{}, I0{});
 }
 
+template <class T> hipError_t launch_sweep_step(int W, bool full, const SweepStepArgs<T> &a, hipStream_t s) {
+    auto go = [&](auto obs, auto f, auto dense, auto train) {
+        hipLaunchKernelGGL((k_sweep_step<T, decltype(obs)::value, decltype(f)::value, decltype(dense)::value,
+                                         decltype(train)::value>),
+                           dim3(W), dim3(kBlock), 0, s, a);
+        return hipGetLastError();
+    };
+    using Yes = std::true_type;
+    using No = std::false_type;
+    std::integral_constant<int, 1> one;
+    std::integral_constant<int, 4> four;
+    std::integral_constant<int, kStepObs> all;
+    const bool dense = a.flip != 0;
+    if (!a.partial) {
+        return dense ? go(all, No{}, Yes{}, No{}) : go(all, No{}, No{}, No{});
+    }
+    if (full) {
+        return dense ? go(one, Yes{}, Yes{}, Yes{}) : go(one, Yes{}, No{}, Yes{});
+    }
+    if (a.nk <= 4) {
+        return dense ? go(four, No{}, Yes{}, Yes{}) : go(four, No{}, No{}, Yes{});
+    }
+    return dense ? go(all, No{}, Yes{}, Yes{}) : go(all, No{}, No{}, Yes{});
+}
+
 template <class T>
 hipError_t launch_pass(int waves, v2<T> *sv, uint64_t ntiles, const SweepGeom &geo, const SweepStep *prog, int nsteps,
                        hipStream_t s) {
@@ -51,6 +76,7 @@ hipError_t launch_pass(int waves, v2<T> *sv, uint64_t ntiles, const SweepGeom &g
 #if PL_SWEEP_DOUBLE
 template hipError_t launch_pass<double>(int, v2<double> *, uint64_t, const SweepGeom &, const SweepStep *, int,
                                         hipStream_t);
+template hipError_t launch_sweep_step<double>(int, bool, const SweepStepArgs<double> &, hipStream_t);
 template hipError_t launch_sweep<double>(int, int, bool, const SweepArgs<double> &, hipStream_t);
 
 hipError_t launch_sweep_sums(const double *partial, int W, unsigned count, int pk, int pk0, int K, double *out,
@@ -61,6 +87,7 @@ hipError_t launch_sweep_sums(const double *partial, int W, unsigned count, int p
 #else
 template hipError_t launch_pass<float>(int, v2<float> *, uint64_t, const SweepGeom &, const SweepStep *, int,
                                        hipStream_t);
+template hipError_t launch_sweep_step<float>(int, bool, const SweepStepArgs<float> &, hipStream_t);
 template hipError_t launch_sweep<float>(int, int, bool, const SweepArgs<float> &, hipStream_t);
 #endif
 

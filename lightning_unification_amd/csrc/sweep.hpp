@@ -5,9 +5,9 @@
 // Step: a 2x2 on pairs that differ in one bit or two, or phases by the parity
 // of some bits, where other bits have given values.  Every gate of at most four
 // members is one or two such steps (IsingXX: one on pairs that differ in both
-// bits); members that differ in more bits (DoubleExcitation) are brought
-// together by CNOTs from one of those bits to the others, undone after.  A step merges into the last one that
-// touched any of its bits when that has the same geometry: nothing in between
+// bits).  Pairs that differ in more bits (DoubleExcitation) are brought
+// together in a pass by CNOTs from one of those bits to the others, undone
+// after.  A step merges into the last one that touched any of its bits when that has the same geometry: nothing in between
 // touches those bits, so it commutes back.  The merged step keeps the product
 // U^dagger = U_m^dagger .. U_1^dagger (U_1 the tape's last) and, for the j-th
 // operation's generator, W = A^dagger G A with A the product before it:
@@ -22,6 +22,7 @@
 #include <algorithm>
 #include <complex>
 #include <cstdint>
+#include <deque>
 #include <vector>
 
 #include "lower.hpp"
@@ -38,19 +39,21 @@ struct SweepTrain {
 
 struct SweepOp { // one step before it is placed on a tile
     bool big = false;  // applied state by state: operation `tape` of the tape
+    bool alone = false; // in no pass
     int tape = -1;
     uint64_t bit = 0;  // the bit a 2x2 mixes (the lower of two); 0: phases only
     uint64_t bit2 = 0; // a second bit its pairs differ in; tests are on the member with `bit` clear
+    uint64_t more = 0; // further ones, each tested
     uint64_t par = 0;  // phases: u[0] or u[3] by the parity of these bits
     uint64_t test = 0, value = 0; // bits tested, and their values
     std::complex<double> u[4] = {1, 0, 0, 1};
     std::vector<SweepTrain> train;
 
-    uint64_t touch() const { return bit | bit2 | par | test | extra; }
+    uint64_t touch() const { return bit | bit2 | more | par | test | extra; }
     uint64_t extra = 0; // big operations: all their bits
-    uint64_t need() const { return bit | bit2; }
+    uint64_t need() const { return bit | bit2 | more; }
     bool same_place(const SweepOp &o) const {
-        return !big && !o.big && bit == o.bit && bit2 == o.bit2 && par == o.par && test == o.test && value == o.value;
+        return !big && !o.big && bit == o.bit && bit2 == o.bit2 && more == o.more && par == o.par && test == o.test && value == o.value;
     }
     bool diagonal() const { return u[1] == 0.0 && u[2] == 0.0; }
     bool identity() const { return diagonal() && u[0] == 1.0 && u[3] == 1.0; }
@@ -143,26 +146,15 @@ inline bool sweep_expand_op(const GroupOp<double> &ud, const GroupOp<double> *g,
         out.push_back(proto);
         return true;
     }
-    // CNOTs from bit t to `bits`
-    auto frame = [&](uint64_t t, uint64_t bits) {
-        for (uint64_t b = bits; b; b &= b - 1) {
-            SweepOp c;
-            c.bit = b & (~b + 1);
-            c.test = c.value = t;
-            c.u[0] = c.u[3] = 0;
-            c.u[1] = c.u[2] = 1;
-            out.push_back(c);
-        }
-    };
-    // the 2x2 of members p and q, which differ in t, t2 and bits brought
-    // together by the frame of t (which leaves the member with t clear alone)
-    auto pair = [&](int p, int q, uint64_t t, uint64_t t2) {
+    // the 2x2 of members p and q, which differ in t, t2 and `more`
+    auto pair = [&](int p, int q, uint64_t t, uint64_t t2, uint64_t more) {
         if (mem[p] & t) {
             std::swap(p, q);
         }
         SweepOp s = proto;
         s.bit = t;
         s.bit2 = t2;
+        s.more = more;
         s.test = touch & ~t;
         s.value = mem[p] & s.test;
         s.u[0] = U(p, p);
@@ -180,13 +172,7 @@ inline bool sweep_expand_op(const GroupOp<double> &ud, const GroupOp<double> *g,
     };
     if (M == 2) {
         const uint64_t t = vary & (~vary + 1), up = vary & ~t, t2 = up & (~up + 1);
-        frame(t, up & ~t2);
-        const size_t nf = out.size();
-        out.push_back(pair(0, 1, t, t2));
-        for (size_t j = 0; j < nf; j++) {
-            const SweepOp c = out[j];
-            out.push_back(c);
-        }
+        out.push_back(pair(0, 1, t, t2, up & ~t2));
         return true;
     }
     if (__builtin_popcountll(vary) != 2) {
@@ -233,7 +219,7 @@ inline bool sweep_expand_op(const GroupOp<double> &ud, const GroupOp<double> *g,
     }
     const uint64_t t = mix & (~mix + 1), t2 = mix & ~t;
     const int a = at(0), b = at(mix), c = at(t == mix ? vary & ~mix : hi), d = at(t == mix ? vary : lo);
-    SweepOp s0 = pair(a, b, t, t2), s1 = pair(c, d, t, t2);
+    SweepOp s0 = pair(a, b, t, t2, 0), s1 = pair(c, d, t, t2, 0);
     auto same = [](const SweepOp &x, const SweepOp &y) {
         bool eq = std::equal(x.u, x.u + 4, y.u) && x.train.size() == y.train.size();
         for (size_t j = 0; eq && j < x.train.size(); j++) {
@@ -291,7 +277,7 @@ class SweepSteps {
             if (!s.big && s.identity() && s.train.empty()) {
                 continue;
             }
-            bool diag = !s.big && s.bit && s.diagonal() && !(s.test & s.bit2);
+            bool diag = !s.big && s.bit && s.diagonal() && !(s.test & (s.bit2 | s.more));
             for (const auto &t : s.train) {
                 diag = diag && t.w01 == 0.0;
             }
@@ -308,11 +294,167 @@ class SweepSteps {
     int last_[64];
 };
 
+// What a step by itself works on: members expand(g, pins) of the state, with
+// `value` set, and for pairs their partners across `flip`.
+struct SweepLone {
+    uint64_t pins = 0, value = 0, flip = 0, par = 0;
+};
+inline SweepLone sweep_lone(const SweepOp &s) {
+    SweepLone l;
+    l.pins = s.test | s.bit;
+    l.value = s.value;
+    if (s.bit) {
+        l.flip = s.need();
+        l.value &= ~s.bit;
+    } else {
+        l.par = s.par;
+        const bool one = s.train.empty() && __builtin_popcountll(s.par) == 1;
+        if (one && s.u[0] == 1.0) { // the other half of them stays
+            l.pins |= s.par;
+            l.value |= s.par;
+        } else if (one && s.u[3] == 1.0) {
+            l.pins |= s.par;
+        }
+    }
+    return l;
+}
+
+// The step as an operation of the per-gate kernels.
+template <class T> GroupOp<T> sweep_group(const SweepOp &s) {
+    const SweepLone l = sweep_lone(s);
+    auto cast = [](const std::complex<double> &z) {
+        return std::complex<T>(static_cast<T>(z.real()), static_cast<T>(z.imag()));
+    };
+    const std::complex<T> u[4] = {cast(s.u[0]), cast(s.u[1]), cast(s.u[2]), cast(s.u[3])}, none(0);
+    std::vector<int> pos;
+    auto pin = [&](uint64_t bits) {
+        for (uint64_t b = bits; b; b &= b - 1) {
+            pos.push_back(__builtin_ctzll(b));
+        }
+    };
+    if (!s.bit) {
+        const uint64_t par = s.par & ~l.pins;
+        if (l.pins == 0) {
+            GroupOp<T> g;
+            g.kind = GroupOp<T>::Parity;
+            g.parity_mask = par;
+            g.parity_phase[0] = u[0];
+            g.parity_phase[1] = u[3];
+            return g;
+        }
+        const int np = __builtin_popcountll(par);
+        pin(l.pins | par);
+        if (np == 0) {
+            return make_group<T>(pos, l.value, {0}, {(l.value & s.par) ? u[3] : u[0]}, true);
+        }
+        const uint64_t p0 = par & (~par + 1);
+        if (np == 1) {
+            return make_group<T>(pos, l.value, {0, p0}, {u[0], none, none, u[3]}, true);
+        }
+        if (np > 2) {
+            throw std::logic_error("tested phases by the parity of more than two bits");
+        }
+        return make_group<T>(pos, l.value, {0, p0, par & ~p0, par},
+                             {u[0], none, none, none, none, u[3], none, none, none, none, u[3], none, none, none, none,
+                              u[0]},
+                             true);
+    }
+    const uint64_t in = l.value & l.flip; // tested bits the pairs differ in
+    if (s.bit2 && !(s.test & s.bit2)) {   // (bit, bit2): 00 with 11, 01 with 10
+        pin(l.pins | s.bit2);
+        return make_group<T>(pos, l.value & ~l.flip, {0, s.bit, s.bit2, s.bit | s.bit2},
+                             {u[0], none, none, u[1], none, u[3], u[2], none, none, u[1], u[0], none, u[2], none, none,
+                              u[3]},
+                             s.diagonal());
+    }
+    pin(l.pins);
+    return make_group<T>(pos, l.value & ~l.flip, {in, in ^ l.flip}, {u[0], u[1], u[2], u[3]}, s.diagonal());
+}
+
 struct SweepPass {
-    bool big = false;
+    bool big = false;     // one step that no pass holds
     std::vector<int> ops; // step indices, in order
     std::vector<int> hb;  // tile bits above the low ones, ascending
 };
+
+// Microseconds a pass's steps take one by one (`alone`) and as a pass
+// (`together`), from which the cheaper is taken.  A pass reads and writes every
+// amplitude of its states and uploads a program, whatever its steps touch; a
+// step by itself is a launch and the traffic of its part of the state.  So a
+// few steps on a small state, and operations on an eighth of a large one, go
+// one by one.  `first`: no pass before it in the call, so nothing hides its
+// upload.
+struct SweepCost {
+    double alone = 0, together = 0;
+};
+
+// Fraction of the state's 128-byte lines that a step by itself touches.
+inline double sweep_lines(const SweepLone &l, bool c128) {
+    const uint64_t high = ~uint64_t{0} << (c128 ? 3 : 4);
+    return ((l.flip & l.pins & high) ? 2.0 : 1.0) /
+           static_cast<double>(uint64_t{1} << __builtin_popcountll(l.pins & high));
+}
+
+// Forward passes (kernels_pass.hpp against the per-gate kernels, both sides measured):
+//   14 qubits       4 RX 34 us one by one, 38 as a pass; 8 65, 43; 16 DoubleExcitation 83, 133
+//   28 qubits c128  4 RX 5480, 1550; 4 CZ 4500, 1510; 8 DoubleExcitation 7040, 5290
+//   28 qubits c64   8 RX 5510, 1660; 8 CSWAP 1970, 2880; 16 DoubleExcitation 6670, 10860
+// Of the whole state's time, half its lines take 0.55, a quarter 0.33, and an
+// eighth, scattered further, 0.45; a wire inside a line adds 0.3.
+inline SweepCost sweep_forward_us(const std::vector<SweepOp> &steps, const SweepPass &ps, int n, bool c128,
+                                  bool first) {
+    const double amps = std::ldexp(1.0, n), rw = 2 * amps * (c128 ? 16 : 8); // bytes
+    SweepCost c;
+    double units = 0; // steps, with the flips and windows of a frame
+    for (int i : ps.ops) {
+        const SweepLone l = sweep_lone(steps[i]);
+        const double f = sweep_lines(l, c128);
+        const bool in_line = ((l.pins | l.flip) & (c128 ? 7 : 15)) && l.pins != l.flip;
+        c.alone += 4 + rw * ((f >= 1 ? 1 : f >= 0.5 ? 0.55 : f >= 0.25 ? 0.33 : 0.45) + (in_line ? 0.3 : 0)) / 6.0e6;
+        units += 1 + 2.4 * __builtin_popcountll(steps[i].more);
+    }
+    c.together = std::max((first ? 19 : 8) + 1.1 * units,
+                          rw / (c128 ? 5.7e6 : 3.7e6) + units * amps * (c128 ? 6.3e-8 : 1.9e-7));
+    return c;
+}
+
+// Whether a step takes part in forward passes at all: the frames of a
+// DoubleExcitation, 6.5 us in a pass that its program bounds, take more than its
+// launch; where traffic bounds the pass they are hidden.
+inline bool sweep_forward_alone(const SweepOp &s, int n, bool c128) {
+    return s.more && 2 * std::ldexp(1.0, n) * (c128 ? 16 : 8) / (c128 ? 5.7e6 : 3.7e6) < 20;
+}
+
+// The backward sweep of lambda and K states (k_sweep against k_sweep_step), for
+// 1, 2 and 4 of a gate:
+//   6 qubits,       K = 1   CRX 53 54 79 us one by one, 59 64 63 as passes
+//   20 qubits c128, K = 4   RX 112 143 207, 118 125 130; CRX 104 118 170, 119 125 136
+//   24 qubits c64,  K = 4   RX 570 900 1490, 830 900 960; DoubleExcitation 400 460 990, 920 1070 1850
+//   26 qubits c128, K = 1   RX 1850 2720 4290, 1820 1810 1830; DoubleExcitation 1150 1260 2450, 1840 1940 2360
+// complex64 passes work in double: their arithmetic is not hidden behind half
+// the traffic.
+inline double sweep_whole_us(int n, bool c128, int K) { // a step by itself on every amplitude
+    return 2 * std::ldexp(1.0, n) * (c128 ? 16 : 8) * (1 + K) / 4.3e6;
+}
+// DoubleExcitations go alone: a pass's bits hold two of them (16 at 20 qubits c128,
+// K = 12: 980 us in passes, 530 alone).  With several launches each on a
+// state that passes hold whole, they stay in (6 us each in the pass).
+inline bool sweep_backward_alone(const SweepOp &s, int n, bool c128, int K) {
+    return s.more && (K <= kStepObs || sweep_whole_us(n, c128, K) > 10);
+}
+inline SweepCost sweep_backward_us(const std::vector<SweepOp> &steps, const SweepPass &ps, int n, bool c128, int K,
+                                   bool first) {
+    const double whole = sweep_whole_us(n, c128, K);
+    const int launches = (K + kStepObs - 1) / kStepObs;
+    SweepCost c;
+    double units = 0;
+    for (int i : ps.ops) {
+        c.alone += 5.0 * launches + whole * std::min(1.0, sweep_lines(sweep_lone(steps[i]), c128) + 0.05);
+        units += 1 + 1.7 * __builtin_popcountll(steps[i].more);
+    }
+    c.together = (first ? 14 : 7) + units * (1.2 + (c128 ? 0.03 : 0.2) * whole) + (c128 ? 1.2 : 1.6) * whole;
+    return c;
+}
 
 constexpr size_t kSweepLookahead = 1024; // steps scanned per pass
 constexpr int kSweepSearchQubits = 18;   // states whose passes outlast a search over single bits on the host
@@ -341,7 +483,7 @@ class SweepScheduler {
         for (size_t j = 0; j < pending_.size() && j < kSweepLookahead && blocked != all_; j++) {
             const SweepOp &s = steps_[pending_[j]];
             const uint64_t hi = s.need() & ~lowm_;
-            if (!s.big && !(s.touch() & blocked) && __builtin_popcountll(hmask | hi) <= budget_) {
+            if (!s.big && !s.alone && !(s.touch() & blocked) && __builtin_popcountll(hmask | hi) <= budget_) {
                 hmask |= hi;
             } else {
                 blocked |= s.touch();
@@ -391,7 +533,7 @@ class SweepScheduler {
         for (; j < pending_.size() && j < kSweepLookahead; j++) {
             const SweepOp &s = steps_[pending_[j]];
             const int more = s.train.empty() ? 0 : 1;
-            if (!s.big && !(s.touch() & blocked) && (s.need() & ~lowm_ & ~hmask) == 0 && slots + more <= kSweepSlots) {
+            if (!s.big && !s.alone && !(s.touch() & blocked) && (s.need() & ~lowm_ & ~hmask) == 0 && slots + more <= kSweepSlots) {
                 taken++;
                 slots += more;
                 if (ops) {
@@ -445,6 +587,17 @@ class SweepScheduler {
     std::vector<int> pending_;
 };
 
+// Steps of the longest program a pass of these can have: a step, its window,
+// its flips (two on bit2 unless the kernel takes pairs in two bits; a frame
+// of two per further bit, each with a window).
+inline size_t sweep_longest(const std::vector<SweepOp> &steps, bool two) {
+    size_t per = 0;
+    for (const SweepOp &s : steps) {
+        per = std::max(per, size_t{2} * (1 + 2 * __builtin_popcountll(s.more)) + (s.bit2 && !two ? 2 : 0));
+    }
+    return per * std::min(steps.size(), kSweepLookahead);
+}
+
 // A pass's program: windows of RB register bits claimed in step order, each
 // followed by the steps it can hold (those whose mixing bit is in the window
 // and which touch no bit of a step held back).  tb: thread bits of the tile;
@@ -487,15 +640,34 @@ inline void sweep_program(const std::vector<SweepOp> &steps, const SweepPass &ps
         return r;
     };
     struct Item {
-        int step, slot;
+        const SweepOp *op;
+        int slot;
+        uint64_t need; // window bits
     };
     std::vector<Item> pending, left;
+    std::deque<SweepOp> frames;
     int slots = 0;
     for (int i : ps.ops) {
-        pending.push_back({i, steps[i].train.empty() ? -1 : slots++});
+        const SweepOp &s = steps[i];
+        // CNOTs from the pairs' lowest bit bring `more` together; the member
+        // with that bit clear, which the tests are on, stays
+        const size_t f0 = frames.size();
+        for (uint64_t b = s.more; b; b &= b - 1) {
+            SweepOp c;
+            c.bit = b & (~b + 1);
+            c.test = c.value = s.bit;
+            c.u[0] = c.u[3] = 0;
+            c.u[1] = c.u[2] = 1;
+            frames.push_back(c);
+            pending.push_back({&frames.back(), -1, c.bit});
+        }
+        pending.push_back({&s, s.train.empty() ? -1 : slots++, s.bit | s.bit2});
+        for (size_t f = f0; f < frames.size(); f++) {
+            pending.push_back({&frames[f], -1, frames[f].bit});
+        }
     }
     auto put = [&](const Item &it) {
-        const SweepOp &s = steps[it.step];
+        const SweepOp &s = *it.op;
         SweepStep d{};
         d.slot = it.slot;
         d.omask = s.test & ~tile;
@@ -546,8 +718,8 @@ inline void sweep_program(const std::vector<SweepOp> &steps, const SweepPass &ps
             uint64_t blocked = 0;
             int taken = 0;
             for (const Item &it : pending) {
-                const SweepOp &s = steps[it.step];
-                const uint32_t nd = local(s.need());
+                const SweepOp &s = *it.op;
+                const uint32_t nd = local(it.need);
                 if (!(s.touch() & blocked) && ((nd & ~w) == 0 || (claim && __builtin_popcount(w | nd) <= RB))) {
                     w |= nd;
                     taken++;
@@ -557,8 +729,8 @@ inline void sweep_program(const std::vector<SweepOp> &steps, const SweepPass &ps
             }
             return taken;
         };
-        const SweepOp &first = steps[pending[0].step];
-        if (local(first.need()) & ~win) {
+        const uint32_t need0 = local(pending[0].need);
+        if (need0 & ~win) {
             // the better of the bits claimed in step order and the runs of
             // RB neighbours that hold the first step's bit
             uint32_t m = 0;
@@ -566,7 +738,7 @@ inline void sweep_program(const std::vector<SweepOp> &steps, const SweepPass &ps
             for (int b = bits - 1; b >= 0 && __builtin_popcount(m) < RB; b--) {
                 m |= 1U << b;
             }
-            const int at = __builtin_ctz(local(first.need()));
+            const int at = __builtin_ctz(need0);
             for (int b = std::max(0, at - RB + 1); b <= at && b + RB <= bits; b++) {
                 uint32_t run = ((1U << RB) - 1) << b;
                 const int c = fill(run, false);
@@ -589,8 +761,8 @@ inline void sweep_program(const std::vector<SweepOp> &steps, const SweepPass &ps
         left.clear();
         uint64_t blocked = 0;
         for (const Item &it : pending) {
-            const SweepOp &s = steps[it.step];
-            if ((s.touch() & blocked) || (local(s.need()) & ~win)) {
+            const SweepOp &s = *it.op;
+            if ((s.touch() & blocked) || (local(it.need) & ~win)) {
                 blocked |= s.touch();
                 left.push_back(it);
             } else {

@@ -72,9 +72,28 @@ template <class T> struct SweepArgs {
     int pk, pk0; // observables per slot of `partial`, the first one's number
 };
 
+// One step on lambda and up to kStepObs states, read and written in place
+// where it acts.  Pairs of a dense step: i = expand(g, geo) and i ^ flip (geo
+// pins the bit and the tested ones, so a bit2 no test is on stays free in g).  Phases (flip = 0): u[0] or u[3] by the parity of i & par.  partial, of a
+// trainable one: as SweepArgs, one walker a workgroup, the first state's
+// observable at k0 of pk.
+constexpr int kStepObs = 8;
+template <class T> struct SweepStepArgs {
+    v2<T> *lam;
+    v2<T> *h[kStepObs];
+    int nk, write_lam;
+    uint64_t nwork, flip, par;
+    Geom geo;
+    dcx<double> u[4];
+    double *partial; // nullptr: not trainable
+    int slot, pk, k0;
+};
+
 // One launch of args.ngrp observable groups (kh observables each) with `waves`
 // (1, 2 or 4) wavefronts per tile; full: the complex sums too.
 template <class T> hipError_t launch_sweep(int waves, int kh, bool full, const SweepArgs<T> &args, hipStream_t s);
+// W workgroups
+template <class T> hipError_t launch_sweep_step(int W, bool full, const SweepStepArgs<T> &args, hipStream_t s);
 // One forward pass (kernels_pass.hpp) of `waves` (1, 2, 4 or 8) wavefronts a tile.
 template <class T>
 hipError_t launch_pass(int waves, v2<T> *sv, uint64_t ntiles, const SweepGeom &geo, const SweepStep *prog, int nsteps,
