@@ -655,7 +655,7 @@ template <class T> struct Engine {
     // wins (fewer passes outweigh the lower occupancy)
     static constexpr int kTileDefaultBits = std::is_same_v<T, double> ? 11 : 12;
     static constexpr int kTileMaxBitsC128 = 11;
-    static constexpr int kTileFloatQubits = 23;
+    static constexpr int kTileFloatQubits = 23, kTileExciteQubits = 11;
     static constexpr int kTileDefaultLow = std::is_same_v<T, double> ? 3 : 4;
 
     // Applies a tape as tile passes (tile.hpp); returns the number of launches,
@@ -675,12 +675,17 @@ template <class T> struct Engine {
             // the default is the faster executor: passes on workgroup tiles
             // (apply_passes), except for complex64 states of
             // kTileFloatQubits or more, where this one's FP32 arithmetic and
-            // 2^12-amplitude wavefront tiles win (28 qubits, 185 gates: 11.8
-            // against 16.5 ms; 20 qubits, 133 gates: 0.45 against 0.26 ms;
-            // complex128 at 28 qubits: 24.2 against 16.4 ms).  A caller's
-            // low_bits is for the wavefront tiles.  Like their scheduler, the
+            // 2^12-amplitude wavefront tiles win, and for DoubleExcitations
+            // on a state of a few wavefronts, which it holds in registers
+            // (eight at 9 qubits: 45 us against 67).  Ten random layers,
+            // wavefront against workgroup tiles: complex64 22 qubits 548 and
+            // 388 us, 23 610 and 605, 24 1028 and 1047, 25 1650 and 2160, 28
+            // 11.8 and 16.7 ms; complex128 28 qubits 23.0 and 16.3 ms.  A
+            // caller's low_bits is for the wavefront tiles.  Like their scheduler, the
             // passes refuse a tape as a whole, except below the smallest tile.
-            if (low < 0 && (std::is_same_v<T, double> || n() < kTileFloatQubits)) {
+            const auto excitations = std::count(t.ids, t.ids + t.nops, static_cast<int>(DoubleExcitation));
+            const bool wavefront = n() >= kTpMinBits && n() <= kTileExciteQubits && 2 * excitations > t.nops;
+            if (low < 0 && !wavefront && (std::is_same_v<T, double> || n() < kTileFloatQubits)) {
                 const int launches = apply_passes(sv, t, n() >= kTpMinBits);
                 HIP_OK(hipStreamSynchronize(h->stream));
                 return launches;
@@ -802,6 +807,35 @@ template <class T> struct Engine {
     }
 
     // ---- forward passes on register tiles (kernels_pass.hpp) ------------------
+    // The arguments of a step by itself on lam (SweepStepArgs), but for the states.
+    SweepStepArgs<T> step_args(const SweepOp &s, V *lam) const {
+        const SweepLone l = sweep_lone(s);
+        SweepStepArgs<T> a{};
+        for (uint64_t b = l.pins; b; b &= b - 1) {
+            a.geo.pos[a.geo.nb++] = __builtin_ctzll(b);
+        }
+        a.geo.fixed = l.value;
+        a.lam = lam;
+        a.write_lam = 1;
+        a.nwork = len() >> a.geo.nb;
+        a.flip = l.flip;
+        a.par = l.par;
+        for (int j = 0; j < 4; j++) {
+            a.u[j] = {s.u[j].real(), s.u[j].imag()};
+        }
+        return a;
+    }
+    // DoubleExcitations through the sweep's kernel, whose grid strides over their
+    // groups: with a wire inside a line 237 us at 28 qubits complex64, 680 by
+    // a thread per group.
+    void apply_step(const SweepOp &s, V *sv) {
+        if (!s.more) {
+            return apply(sweep_group<T>(s), sv);
+        }
+        const SweepStepArgs<T> a = step_args(s, sv);
+        HIP_OK(launch_sweep_step<T>(grid_for(a.nwork, 1, 16), false, a, h->stream));
+    }
+
     // Applies a tape; returns the number of launches.  A pass's steps are
     // applied one by one where that costs less (SweepCost), or where there is
     // no memory for programs.  The operations
@@ -872,7 +906,7 @@ template <class T> struct Engine {
                     launches++;
                     const SweepOp &op = steps[ps.ops[0]];
                     if (!op.big) {
-                        apply(sweep_group<T>(op), sv);
+                        apply_step(op, sv);
                         continue;
                     }
                     const int i = op.tape;
@@ -886,7 +920,7 @@ template <class T> struct Engine {
                 }
                 if (cost.alone <= cost.together || !pb->ok()) {
                     for (int i : ps.ops) {
-                        apply(sweep_group<T>(steps[i]), sv);
+                        apply_step(steps[i], sv);
                     }
                     launches += static_cast<int>(ps.ops.size());
                     continue;
@@ -1607,9 +1641,9 @@ void defer_gate(pl_sv_t h, int id, const int *wires, int nw, bool inverse, const
 // Tapes of at least this many operations are planned as passes on register
 // tiles (apply_passes); shorter ones go gate by gate.  On states below
 // kPassMinBytes a pass's program gains from about six launches on (four RX: 34 us
-// gate by gate and 38 as a pass at 14 qubits complex128, 51 and 41 at 20).
+// gate by gate and 38 as a pass at 14 qubits, 43 and 39 at 20 complex64).
 constexpr int kPassMinOps = 4, kPassMinOpsSmall = 6;
-constexpr size_t kPassMinBytes = size_t{16} << 20;
+constexpr size_t kPassMinBytes = size_t{8} << 20;
 
 // Engine of the handle's precision, exceptions propagate
 template <class F> void dispatch_or_throw(pl_sv_t h, F &&f) {
@@ -1819,21 +1853,8 @@ void backward_sweep(Engine<T> &E, const SweepTape &t, v2<T> *lam, const std::vec
 
     // step i on lambda and every h, by itself
     auto step_alone = [&](int i) {
-        const SweepOp &s = steps[i];
-        const SweepLone l = sweep_lone(s);
-        const bool train = !s.train.empty();
-        SweepStepArgs<T> a{};
-        for (uint64_t b = l.pins; b; b &= b - 1) {
-            a.geo.pos[a.geo.nb++] = __builtin_ctzll(b);
-        }
-        a.geo.fixed = l.value;
-        a.lam = lam;
-        a.nwork = E.len() >> a.geo.nb;
-        a.flip = l.flip;
-        a.par = l.par;
-        for (int j = 0; j < 4; j++) {
-            a.u[j] = {s.u[j].real(), s.u[j].imag()};
-        }
+        const bool train = !steps[i].train.empty();
+        SweepStepArgs<T> a = E.step_args(steps[i], lam);
         if (train) {
             if (slot_step.size() - reduced + 1 > cap) {
                 reduce();

@@ -396,33 +396,39 @@ inline double sweep_lines(const SweepLone &l, bool c128) {
 }
 
 // Forward passes (kernels_pass.hpp against the per-gate kernels, both sides measured):
-//   14 qubits       4 RX 34 us one by one, 38 as a pass; 8 65, 43; 16 DoubleExcitation 83, 133
-//   28 qubits c128  4 RX 5480, 1550; 4 CZ 4500, 1510; 8 DoubleExcitation 7040, 5290
-//   28 qubits c64   8 RX 5510, 1660; 8 CSWAP 1970, 2880; 16 DoubleExcitation 6670, 10860
-// Of the whole state's time, half its lines take 0.55, a quarter 0.33, and an
-// eighth, scattered further, 0.45; a wire inside a line adds 0.3.
+//   14 qubits       4 RX 34 us one by one, 38 as a pass; 8 65, 43
+//   28 qubits c128  4 RX 5480, 1550; 4 CZ 4500, 1510
+//   28 qubits c64   8 RX 5510, 1660; 8 CSWAP 1970, 2880
+// Of the whole state's time, half its lines take 0.55, a quarter 0.33, and a
+// wire inside a line adds 0.3; a DoubleExcitation 1.15 times its lines'.
+//
+// A DoubleExcitation is kept out of passes where it is cheap by itself: a pass
+// holds two of them on wires outside the line, and its frame is 6.5 us
+// of a program that bounds the pass on a small state (16 at 18 qubits 172 us in
+// passes, 100 alone; 28 qubits complex64 10.8 and 2.75 ms).
+inline bool sweep_forward_alone(const SweepOp &s, int n, bool c128) {
+    const double rw = 2 * std::ldexp(1.0, n) * (c128 ? 16 : 8);
+    return s.more && (sweep_lines(sweep_lone(s), c128) <= 0.25 || rw / (c128 ? 5.7e6 : 3.7e6) < 20);
+}
 inline SweepCost sweep_forward_us(const std::vector<SweepOp> &steps, const SweepPass &ps, int n, bool c128,
                                   bool first) {
     const double amps = std::ldexp(1.0, n), rw = 2 * amps * (c128 ? 16 : 8); // bytes
-    SweepCost c;
     double units = 0; // steps, with the flips and windows of a frame
+    SweepCost c;
     for (int i : ps.ops) {
         const SweepLone l = sweep_lone(steps[i]);
         const double f = sweep_lines(l, c128);
-        const bool in_line = ((l.pins | l.flip) & (c128 ? 7 : 15)) && l.pins != l.flip;
-        c.alone += 4 + rw * ((f >= 1 ? 1 : f >= 0.5 ? 0.55 : f >= 0.25 ? 0.33 : 0.45) + (in_line ? 0.3 : 0)) / 6.0e6;
         units += 1 + 2.4 * __builtin_popcountll(steps[i].more);
+        if (steps[i].more) {
+            c.alone += 4 + 1.15 * rw * f / 6.0e6;
+            continue;
+        }
+        const bool in_line = ((l.pins | l.flip) & (c128 ? 7 : 15)) && l.pins != l.flip;
+        c.alone += 4 + rw * ((f >= 1 ? 1 : f >= 0.5 ? 0.55 : 0.33) + (in_line ? 0.3 : 0)) / 6.0e6;
     }
     c.together = std::max((first ? 19 : 8) + 1.1 * units,
                           rw / (c128 ? 5.7e6 : 3.7e6) + units * amps * (c128 ? 6.3e-8 : 1.9e-7));
     return c;
-}
-
-// Whether a step takes part in forward passes at all: the frames of a
-// DoubleExcitation, 6.5 us in a pass that its program bounds, take more than its
-// launch; where traffic bounds the pass they are hidden.
-inline bool sweep_forward_alone(const SweepOp &s, int n, bool c128) {
-    return s.more && 2 * std::ldexp(1.0, n) * (c128 ? 16 : 8) / (c128 ? 5.7e6 : 3.7e6) < 20;
 }
 
 // The backward sweep of lambda and K states (k_sweep against k_sweep_step), for

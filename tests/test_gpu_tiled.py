@@ -72,8 +72,8 @@ def test_tiled_errors():
 @pytest.mark.parametrize("dtype", [np.complex128, np.complex64])
 @pytest.mark.parametrize("n", [5, 8, 9, 12])
 def test_tiled_defaults(oracle, dtype, n):
-    """tile_bits = 0 / low_bits = -1: the precision's defaults, clamped to the
-    state; below 9 qubits the tape runs gate by gate."""
+    """tile_bits = 0 / low_bits = -1: the passes of pl_sv_apply_ops at these
+    sizes, on workgroup tiles."""
     from lightning_unification_amd import capi
     tape = zoo_tape(n, 300 + n)
     psi = random_state(n, 11 + n, dtype)
@@ -100,3 +100,23 @@ def test_tiled_long_tape_refills_program_buffers(oracle):
         got = sv.state()
     assert npass == len(capi.tile_plan(n, tape, 11, 3))
     assert rel_err(got, exp) < 1e-12
+
+
+@pytest.mark.parametrize("dtype", [np.complex128, np.complex64])
+@pytest.mark.parametrize("n", [8, 9, 11, 12])
+def test_tiled_default_of_excitations(oracle, dtype, n):
+    """Tapes of mostly DoubleExcitations take the wavefront tiles from 9 to 11
+    qubits."""
+    from lightning_unification_amd import capi
+    from lightning_unification_amd.circuits import Tape
+    rs = np.random.default_rng(n)
+    tape = Tape()
+    for i in range(9):
+        tape.add("DoubleExcitation", rs.choice(n, 4, replace=False).tolist(), [0.2 + i], bool(i & 1))
+        if i % 3 == 0:
+            tape.add("RX", [i % n], [0.5 * i])
+    psi = random_state(n, 5 + n, dtype)
+    exp = oracle.apply_tape(psi.astype(np.complex128), tape)
+    with capi.DeviceStateVector.from_array(psi) as sv:
+        sv.apply_tape_tiled(tape)
+        assert rel_err(sv.state(), exp) < TOL[dtype]
