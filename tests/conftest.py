@@ -35,6 +35,14 @@ def random_state(n, seed, dtype=np.complex128):
     return v.astype(dtype)
 
 
+def apply_each(sv, tape):
+    """The tape gate by gate, a call each: the single-gate kernels, where
+    apply_tape takes passes."""
+    for name, wires, inverse, params in tape.ops:
+        if name not in ("BasisState", "QubitStateVector"):  # skipped, as by apply_tape
+            sv.apply(name, wires, inverse, params)
+
+
 def rel_err(a, b, floor=1.0):
     """max |a-b| / max(|b|, floor): relative error with an absolute floor for
     entries near zero (the tolerance contract is 1e-12 relative, complex128)."""

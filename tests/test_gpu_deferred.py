@@ -1,12 +1,12 @@
 """Deferred gates (pl_sv_set_deferred): pl_sv_apply_gate / pl_sv_apply_ops
-queue their gates, which run as tile passes before anything else uses the
-state.  Every way of using the state must see what gate-by-gate application
-gives: the oracle at 1e-12 (complex128), and the eager path's own results for
-measurements.  Calls that overwrite the whole state drop the queue."""
+queue their gates, which run as passes before anything else uses the state.
+Every way of using the state must see what gate-by-gate application gives: the
+oracle at 1e-12 (complex128), and a state to which the gates were applied one
+call each for measurements.  Calls that overwrite the whole state drop the queue."""
 import numpy as np
 import pytest
 
-from conftest import random_state, rel_err
+from conftest import apply_each, random_state, rel_err
 from lightning_unification_amd.circuits import Obs, pauli_word, random_hamiltonian, random_layers
 from test_tile_plan import without_prep, zoo_tape
 
@@ -20,11 +20,11 @@ def _capi():
 
 def _pair(n, dtype, tape, seed=5):
     """An eager and a deferred state from the same start, the tape applied
-    to both (the deferred one only queued)."""
+    to both: gate by gate, and only queued."""
     capi = _capi()
     psi = random_state(n, seed, dtype)
     eager = capi.DeviceStateVector.from_array(psi)
-    eager.apply_tape(tape)
+    apply_each(eager, tape)
     lazy = capi.DeviceStateVector.from_array(psi)
     lazy.set_deferred(True)
     lazy.apply_tape(tape)
@@ -100,13 +100,13 @@ def test_adjoint_and_copy_and_distance_see_the_queue():
         jb = lazy.adjoint_jacobian(tape, obs, tp)
         assert rel_err(jb, ja) < 1e-12
         lazy.apply_tape(tape)
-        eager.apply_tape(tape)
+        apply_each(eager, tape)
         assert lazy.deferred_count() == len(tape.ops)
         dst.copy_from(lazy)
         assert lazy.deferred_count() == 0
         assert rel_err(dst.state(), eager.state()) < 1e-12
         lazy.apply_tape(tape)
-        eager.apply_tape(tape)
+        apply_each(eager, tape)
         assert eager.distance(lazy) < 1e-12
         assert lazy.deferred_count() == 0
 

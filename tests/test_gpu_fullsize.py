@@ -1,10 +1,10 @@
 """The large configurations at their full size.
 
 30 qubits, complex128 (16 GiB): the seeded 50-layer gate mix through the
-per-gate path, checked against scalars the reference's own Lightning-Qubit
-kernels produced at the same size (tests/golden/c2_n30.npz, written by
-tests/golden/make_golden.py from the reference compiled in place):
-amplitudes at 4096 seeded indices, each of the 100 Pauli terms' expectation
+single-gate kernels and through the passes of apply_tape, checked against
+scalars the reference's own Lightning-Qubit kernels produced at the same size
+(tests/golden/c2_n30.npz, written by tests/golden/make_golden.py from the
+reference compiled in place): amplitudes at 4096 seeded indices, each of the 100 Pauli terms' expectation
 and the Hamiltonian's, and the inverse-CDF indices of the first 10^4 of the
 benchmark's uniforms (bit-exact outside the tie band).
 
@@ -17,6 +17,7 @@ import os
 import numpy as np
 import pytest
 
+from conftest import apply_each
 from lightning_unification_amd.circuits import Obs, Tape, random_hamiltonian, random_layers
 
 pytestmark = pytest.mark.gpu
@@ -47,19 +48,25 @@ def _gather(sv, idx):
 
 
 @pytest.mark.skipif(not os.path.exists(GOLDEN), reason="c2_n30.npz not generated")
-def test_c2_30_qubits_against_the_reference():
+@pytest.mark.parametrize("how", ["gates", "passes"])
+def test_c2_30_qubits_against_the_reference(how):
     capi = _capi()
     g = np.load(GOLDEN)
     n = 30
     tape = random_layers(n, 50, seed=1002)
     ham = random_hamiltonian(n, 100, seed=1002)
-    print("c2 full size: forward, 990 gates on 30 qubits", flush=True)
+    print(f"c2 full size: forward, 990 gates on 30 qubits ({how})", flush=True)
     with capi.DeviceStateVector(n, np.complex128) as sv:
-        sv.apply_tape(tape)
+        if how == "gates":
+            apply_each(sv, tape)
+        else:
+            sv.apply_tape(tape)
         amps = _gather(sv, g["idx"])
         err = np.linalg.norm(amps - g["amps"]) / np.linalg.norm(g["amps"])
         assert err < 1e-12, err
         assert abs(np.sqrt(sv.norm2()) - g["norm"][0]) < 1e-12
+        if how == "gates":
+            return  # the state is the same: its measurements follow once
         print("c2 full size: 100 terms", flush=True)
         terms = np.array([sv.expval(t) for t in ham.terms])
         assert np.max(np.abs(terms - g["term_expvals"])) < 1e-12

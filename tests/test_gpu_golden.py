@@ -7,7 +7,7 @@ import os
 import numpy as np
 import pytest
 
-from conftest import rel_err
+from conftest import apply_each, rel_err
 from lightning_unification_amd.circuits import (Obs, Tape, plain_layers, random_hamiltonian,
                                                 random_layers, sample_uniforms)
 from lightning_unification_amd.gates import GATE_NAMES
@@ -49,12 +49,17 @@ def test_golden_plain_full_size():
     assert rel_err(jac, z["jac"]) < 1e-12
 
 
-def test_golden_random_circuit_n16():
+@pytest.mark.parametrize("how", ["gates", "passes"])
+def test_golden_random_circuit_n16(how):
     from lightning_unification_amd import capi
     z = load("random_n16.npz")
     n = 16
     with capi.DeviceStateVector(n) as sv:
-        sv.apply_tape(random_layers(n, 50, seed=1002))
+        tape = random_layers(n, 50, seed=1002)
+        if how == "gates":
+            apply_each(sv, tape)
+        else:
+            sv.apply_tape(tape)
         st = sv.state()
         assert rel_err(st[z["idx"]], z["amps"]) < 1e-12
         e = sv.expval(random_hamiltonian(n, 100, seed=1002))

@@ -7,7 +7,7 @@ complex128; complex64 accumulates rounding over ~200 gates, 1e-4."""
 import numpy as np
 import pytest
 
-from conftest import random_state, rel_err
+from conftest import apply_each, random_state, rel_err
 from lightning_unification_amd.circuits import random_layers
 from test_tile_plan import without_prep, zoo_tape
 
@@ -48,7 +48,7 @@ def test_tiled_matches_per_gate_path_20q(dtype, k, low):
     if dtype == np.complex128 and k > 11:
         pytest.skip("complex128 tiles hold at most 2^11 amplitudes (covered by the oracle test)")
     with capi.DeviceStateVector(n, dtype) as a, capi.DeviceStateVector(n, dtype) as b:
-        a.apply_tape(tape)
+        apply_each(a, tape)
         npass = b.apply_tape_tiled(tape, k, low)
         assert npass < len(tape.ops) // 5
         d = a.distance(b)
