@@ -234,10 +234,9 @@ def bench_c1():
     of RX, RY, RZ per wire + CNOT ladder, <Z_w> for every wire and the full
     20 x 600 adjoint Jacobian (complex128).  Reports the GPU time of forward +
     expvals + Jacobian, the unfused-minimum algorithmic bytes of the Jacobian
-    (sum over ops of (K+1) 2 f S + per trainable op (K+1) S, plus K S) and the
-    bytes this engine's fused adjoint moves ((K+G) 2 f S per op for G groups
-    of observables, K + G state preparations), and the compiled reference (all host cores, OpenMP over
-    observables as in the reference) beside the GPU on a one-layer prefix."""
+    (sum over ops of (K+1) 2 f S + per trainable op (K+1) S, plus K S), and the
+    compiled reference (all host cores, OpenMP over observables as in the
+    reference) beside the GPU on a one-layer prefix."""
     from lightning_unification_amd import capi
     from lightning_unification_amd.circuits import plain_layers
     n, K = 20, 20
@@ -256,18 +255,9 @@ def bench_c1():
     _, jac = run(tape, tp)
     t_gpu = time.perf_counter() - t0
     alg = sum((K + 1) * 2 * touched_fraction(op[0]) * S for op in tape.ops) + len(tp) * (K + 1) * S + K * S
-    # the engine runs the sweep over groups of observables that fit its 192 MiB
-    # cache budget, each group with its own lambda (two groups of 10 here)
-    budget = 192 << 20
-    groups = 1
-    if S * (K + 1) > budget and 2 * S <= budget:
-        fit = max(1, budget // S - 1)
-        groups = -(-K // fit)
-    moved = sum((K + groups) * 2 * touched_fraction(op[0]) * S for op in tape.ops) + (K + groups) * 2 * S
     out = {"qubits": n, "ops": len(tape), "params": len(tp), "observables": K,
            "gpu_forward_expval_jacobian_ms": round(t_gpu * 1e3, 1),
            "jacobian_algorithmic_GB": round(alg / 1e9, 1),
-           "jacobian_moved_GB": round(moved / 1e9, 1),
            "algorithmic_GBs": round(alg / t_gpu / 1e9, 1)}
     # one-layer prefix on both sides
     pre, _, _ = plain_layers(n, 1, seed=1001)

@@ -37,7 +37,10 @@
  *      from `mats`); is_ham = 1 takes one coefficient per term, in order,
  *      from `coeffs`.
  *  - Calls on one handle are ordered on that handle's HIP stream; calls that
- *    return host data synchronise.  Handles are not thread-safe.
+ *    return host data synchronise, and so do pl_sv_apply_ops_tiled and the
+ *    application of deferred gates.  Others may return with their work queued:
+ *    before it reads or writes the memory of pl_sv_device_ptr itself, a caller
+ *    calls pl_sv_synchronize.  Handles are not thread-safe.
  */
 #ifndef PL_AMD_H
 #define PL_AMD_H
@@ -115,8 +118,8 @@ int pl_sv_apply_ops(pl_sv_t sv, int nops, const int *ids, const int *nwires,
  * returns with the gate applied; here the result is the same by the time
  * anything can observe it).  With on != 0, pl_sv_apply_gate and
  * pl_sv_apply_ops check each gate as they otherwise would (same errors, at
- * the call) and queue it; the queue is applied as tile passes, with the
- * precision's default tiles, before any other call on sv reads or changes
+ * the call) and queue it; the queue is applied as pl_sv_apply_ops_tiled
+ * applies a tape by default, before any other call on sv reads or changes
  * the state (measurements, adjoint, copies, downloads, pl_sv_device_ptr,
  * pl_sv_synchronize, timing events), and whenever it holds 4096 gates.  A
  * call that overwrites the whole state (pl_sv_upload, pl_sv_set_basis_state,
@@ -293,7 +296,8 @@ int pl_sv_apply_ops_tiled(pl_sv_t sv, int nops, const int *ids, const int *nwire
                           const int *wires, const uint8_t *inverse,
                           const int *nparams, const double *params, int tile_bits,
                           int low_bits, int flags, int *npasses);
-/* The pass plan of pl_sv_apply_ops_tiled, computed on the host only: for
+/* The pass plan of pl_sv_apply_ops_tiled for given tile_bits and low_bits (the
+ * default's workgroup tiles are planned otherwise), computed on the host only: for
  * pass p, pass_nops[p] operations, pass_tiled[p] (0 = one operation applied
  * by the per-gate kernels), pass_bits[16 p ..] the higher tile bit positions
  * (ascending, -1 padded); order[] lists the tape indices of all operations

@@ -14,7 +14,7 @@
 // goes through LDS, one state at a time through one buffer.  A step per trip
 // through LDS instead (amplitudes kept there) was bound by LDS latency and
 // address arithmetic: 5 us a step for six resident wavefronts.
-// 20 qubits, 600 parameters, 20 observables: 8 passes of 0.67 ms, 5.4 ms for
+// 20 qubits, 600 parameters, 20 observables: 8 passes of 0.64 ms, 5.1 ms for
 // the Jacobian against 84 ms; bound by FP64 issue (about 2.5 ms of multiply-adds
 // at full rate, window changes, wavefront reductions) and by the states'
 // traffic (0.16 ms a pass).

@@ -650,9 +650,11 @@ template <class T> struct Engine {
     }
 
     // ---- tile passes: many gates per read and write of the state --------------
-    // defaults measured on the 50-layer random circuit (30 qubits complex128,
-    // 33 qubits complex64): the largest tile each precision's registers hold
-    // wins (fewer passes outweigh the lower occupancy)
+    // the wavefront tiles taken where only low_bits is given, for complex64
+    // states of kTileFloatQubits on, and for DoubleExcitations: the largest
+    // each precision's registers hold, as measured on the 50-layer random
+    // circuit (30 qubits complex128, 33 qubits complex64; fewer passes
+    // outweigh the lower occupancy)
     static constexpr int kTileDefaultBits = std::is_same_v<T, double> ? 11 : 12;
     static constexpr int kTileMaxBitsC128 = 11;
     static constexpr int kTileFloatQubits = 23, kTileExciteQubits = 11;
@@ -661,8 +663,7 @@ template <class T> struct Engine {
     // Applies a tape as tile passes (tile.hpp); returns the number of launches,
     // with the state final: the deferred gates' flush behind pl_sv_device_ptr
     // and the callers of pl_sv_apply_ops_tiled hand the memory to other streams.
-    // k = 0 / low < 0 pick the measured defaults of the precision; with k = 0
-    // a state narrower than the smallest tile runs gate by gate.  Each pass is
+    // k = 0 / low < 0 pick the measured defaults of the precision.  Each pass is
     // planned, compiled and launched before the next is planned, so the host's
     // planning overlaps the device's passes.
     int apply_tiled(V *sv, const TapeView &t, int k, int low) {
@@ -1584,7 +1585,7 @@ template <class T> struct Engine {
 // ---- deferred gates --------------------------------------------------------
 // While deferral is on, pl_sv_apply_gate / pl_sv_apply_ops check each gate as
 // the per-gate path would (same errors, at the call) and queue it; the queue
-// is applied as tile passes (the precision's default tiles) by the first call
+// is applied as passes (the tiled executor's defaults) by the first call
 // that reads or changes the state otherwise, or once it holds
 // kDeferMaxOps gates.
 constexpr size_t kDeferMaxOps = 4096;

@@ -5,8 +5,8 @@
 // change of window goes through an LDS buffer of real parts and imaginary
 // parts (an element of both would tie the two registers of an amplitude into
 // one tuple, which in-place updates would have to copy out of and back into).
-// Used by the backward sweep (kernels_adjoint.hpp) and the batched circuits
-// (kernels_batch.hpp).
+// Used by the backward sweep (kernels_adjoint.hpp), forward passes
+// (kernels_pass.hpp) and the batched circuits (kernels_batch.hpp).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -64,7 +64,10 @@ __device__ __forceinline__ int rt_row(int r) { return ((r & 1) << 1) | (r >> 1);
 // map folds bits 4..8 into the low five so that for windows of three and four
 // neighbouring bits the first four lane bits give 16 places that differ mod 16
 // and the first five 32 mod 32 (all but one case): no two lanes of an access
-// share a bank.  Found by trying every such map.
+// share a bank.  Found by trying every such map.  Measured, conflicts take up to 2 % of
+// the LDS cycles in the sweep and the batched stages, but 21 % there on tiles
+// of 2^10 amplitudes, and 25 % in a forward pass at 28 qubits, whose windows
+// hold any four bits.
 __device__ __forceinline__ uint32_t rt_place(uint32_t e) {
     return e ^ ((e >> 4) & 1U) ^ ((e >> 3) & 4U) ^ (((e >> 6) & 1U) * 10U) ^ (((e >> 7) & 1U) * 28U) ^ ((e >> 4) & 16U);
 }
