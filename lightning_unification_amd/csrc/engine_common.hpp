@@ -214,7 +214,7 @@ template <class F> int guarded(F &&f) {
 // segments of pinned memory, each copied to the same place of a device buffer.
 struct ProgramRing {
     static constexpr int kSegs = 4;
-    static constexpr size_t kSegBytes = size_t{32} << 10; // at first: about 240 steps
+    static constexpr size_t kSegBytes = size_t{128} << 10; // at first: about 960 steps
     void *host = nullptr, *dev = nullptr; // host: nullptr where it cannot be pinned
     size_t seg_bytes = 0, used = 0;       // used: bytes of the current segment
     int seg = 0;
@@ -232,7 +232,7 @@ struct HandleKit {
     void *io = nullptr;
 };
 struct HandleKits {
-    static constexpr size_t kKits = 4; // 192 KiB pinned and 128 KiB of device memory each
+    static constexpr size_t kKits = 4; // 576 KiB pinned and 512 KiB of device memory each
     std::mutex mu;
     std::vector<HandleKit> kept;
     int live = 0; // handles

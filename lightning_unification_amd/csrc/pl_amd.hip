@@ -169,9 +169,9 @@ template <class T> constexpr int kSweepLow = std::is_same_v<T, double> ? 3 : 4; 
 // The passes' programs on their way to the device: appended to the current
 // segment of the handle's pinned ring and copied from there without waiting.
 // A full segment is left with an event behind its copies (and the passes
-// between them) and taken again once that event has come, so calls run ahead of the device by
-// up to three segments; the device side of a segment is safe by the stream's
-// order.  A call whose longest program may not fit a segment grows the ring,
+// between them) and taken again once that event has come, so calls run ahead
+// of the device by up to three segments; the device side of a segment is safe
+// by the stream's order.  A call whose longest program may not fit a segment grows the ring,
 // after a wait.  Where the ring cannot be pinned, each copy is waited for.
 // With one buffer for a whole call, taken again when the call's last pass had
 // ended, a tape right behind another waited for it.
@@ -682,8 +682,9 @@ template <class T> struct Engine {
             // wavefront against workgroup tiles: complex64 22 qubits 548 and
             // 388 us, 23 610 and 605, 24 1028 and 1047, 25 1650 and 2160, 28
             // 11.8 and 16.7 ms; complex128 28 qubits 23.0 and 16.3 ms.  A
-            // caller's low_bits is for the wavefront tiles.  Like their scheduler, the
-            // passes refuse a tape as a whole, except below the smallest tile.
+            // caller's low_bits is for the wavefront tiles.  Like their
+            // scheduler, the passes refuse a tape as a whole, except below the
+            // smallest tile.
             const auto excitations = std::count(t.ids, t.ids + t.nops, static_cast<int>(DoubleExcitation));
             const bool wavefront = n() >= kTpMinBits && n() <= kTileExciteQubits && 2 * excitations > t.nops;
             if (low < 0 && !wavefront && (std::is_same_v<T, double> || n() < kTileFloatQubits)) {
@@ -839,10 +840,10 @@ template <class T> struct Engine {
 
     // Applies a tape; returns the number of launches.  A pass's steps are
     // applied one by one where that costs less (SweepCost), or where there is
-    // no memory for programs.  The operations
-    // before one that does not lower are applied before its error leaves, as
-    // gate by gate, or none (whole).  The device is waited for only
-    // where the program ring has gone round (ProgramBuffer).
+    // no memory for programs.  The operations before one that does not lower
+    // are applied before its error leaves, as gate by gate, or none (whole).
+    // The device is waited for only where the program ring has gone round
+    // (ProgramBuffer).
     int apply_passes(V *sv, const TapeView &t, bool whole = false) {
         SweepSteps builder;
         std::vector<SweepOp> parts;

@@ -599,6 +599,9 @@ class SweepScheduler {
 inline size_t sweep_longest(const std::vector<SweepOp> &steps, bool two) {
     size_t per = 0;
     for (const SweepOp &s : steps) {
+        if (s.big || s.alone) {
+            continue;
+        }
         per = std::max(per, size_t{2} * (1 + 2 * __builtin_popcountll(s.more)) + (s.bit2 && !two ? 2 : 0));
     }
     return per * std::min(steps.size(), kSweepLookahead);
