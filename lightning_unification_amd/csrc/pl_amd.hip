@@ -164,6 +164,8 @@ static void download_host(pl_sv_t h, void *dst, const void *src, size_t bytes) {
     drain(nchunks - 1);
 }
 
+constexpr size_t kPassMinBytes = size_t{8} << 20; // a state whose gates are more than launches
+
 template <class T> constexpr int kSweepLow = std::is_same_v<T, double> ? 3 : 4; // one 128-byte line
 
 // The passes' programs on their way to the device: appended to the current
@@ -827,11 +829,12 @@ template <class T> struct Engine {
         }
         return a;
     }
-    // DoubleExcitations through the sweep's kernel, whose grid strides over their
-    // groups: with a wire inside a line 237 us at 28 qubits complex64, 680 by
-    // a thread per group.
+    // DoubleExcitations of states that are more than a launch go through the
+    // sweep's kernel, whose grid strides over their groups: with a wire inside a
+    // line 237 us at 28 qubits complex64, 680 by a thread per group (14 qubits
+    // 6.0 us and 5.3).
     void apply_step(const SweepOp &s, V *sv) {
-        if (!s.more) {
+        if (!s.more || h->state_bytes() < kPassMinBytes) {
             return apply(sweep_group<T>(s), sv);
         }
         const SweepStepArgs<T> a = step_args(s, sv);
@@ -884,8 +887,7 @@ template <class T> struct Engine {
                 }
                 parts.assign(1, op);
             }
-            for (SweepOp &op : parts) {
-                op.alone = sweep_forward_alone(op, n(), std::is_same_v<T, double>);
+            for (const SweepOp &op : parts) {
                 builder.add(op);
             }
         }
@@ -906,12 +908,7 @@ template <class T> struct Engine {
             while (sched.next(ps)) {
                 if (ps.big) {
                     launches++;
-                    const SweepOp &op = steps[ps.ops[0]];
-                    if (!op.big) {
-                        apply_step(op, sv);
-                        continue;
-                    }
-                    const int i = op.tape;
+                    const int i = steps[ps.ops[0]].tape;
                     gate(sv, t.ids[i], t.wires + woff[i], t.nwires[i], t.inverse[i] != 0, t.params + poff[i],
                          t.nparams[i]);
                     continue;
@@ -1645,7 +1642,6 @@ void defer_gate(pl_sv_t h, int id, const int *wires, int nw, bool inverse, const
 // kPassMinBytes a pass's program gains from about six launches on (four RX: 34 us
 // gate by gate and 38 as a pass at 14 qubits, 43 and 39 at 20 complex64).
 constexpr int kPassMinOps = 4, kPassMinOpsSmall = 6;
-constexpr size_t kPassMinBytes = size_t{8} << 20;
 
 // Engine of the handle's precision, exceptions propagate
 template <class F> void dispatch_or_throw(pl_sv_t h, F &&f) {

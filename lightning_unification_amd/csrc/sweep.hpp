@@ -400,16 +400,10 @@ inline double sweep_lines(const SweepLone &l, bool c128) {
 //   28 qubits c128  4 RX 5480, 1550; 4 CZ 4500, 1510
 //   28 qubits c64   8 RX 5510, 1660; 8 CSWAP 1970, 2880
 // Of the whole state's time, half its lines take 0.55, a quarter 0.33, and a
-// wire inside a line adds 0.3; a DoubleExcitation 1.15 times its lines'.
-//
-// A DoubleExcitation is kept out of passes where it is cheap by itself: a pass
-// holds two of them on wires outside the line, and its frame is 6.5 us
-// of a program that bounds the pass on a small state (16 at 18 qubits 172 us in
-// passes, 100 alone; 28 qubits complex64 10.8 and 2.75 ms).
-inline bool sweep_forward_alone(const SweepOp &s, int n, bool c128) {
-    const double rw = 2 * std::ldexp(1.0, n) * (c128 ? 16 : 8);
-    return s.more && (sweep_lines(sweep_lone(s), c128) <= 0.25 || rw / (c128 ? 5.7e6 : 3.7e6) < 20);
-}
+// wire inside a line adds 0.3; the phases of a parity take 1.3 times the whole, a
+// DoubleExcitation its lines' share times 1.3, or 0.9 in the last-level cache.
+// In a pass a DoubleExcitation is a frame of some six steps (16 at 18 qubits 172
+// us in passes, 100 one by one; 28 qubits complex64 10.8 and 2.75 ms).
 inline SweepCost sweep_forward_us(const std::vector<SweepOp> &steps, const SweepPass &ps, int n, bool c128,
                                   bool first) {
     const double amps = std::ldexp(1.0, n), rw = 2 * amps * (c128 ? 16 : 8); // bytes
@@ -420,11 +414,12 @@ inline SweepCost sweep_forward_us(const std::vector<SweepOp> &steps, const Sweep
         const double f = sweep_lines(l, c128);
         units += 1 + 2.4 * __builtin_popcountll(steps[i].more);
         if (steps[i].more) {
-            c.alone += 4 + 1.15 * rw * f / 6.0e6;
+            c.alone += 4 + (rw > 5.4e8 ? 1.3 : 0.9) * rw * f / 6.0e6;
             continue;
         }
         const bool in_line = ((l.pins | l.flip) & (c128 ? 7 : 15)) && l.pins != l.flip;
-        c.alone += 4 + rw * ((f >= 1 ? 1 : f >= 0.5 ? 0.55 : 0.33) + (in_line ? 0.3 : 0)) / 6.0e6;
+        const double all = l.flip ? 1 : 1.3;
+        c.alone += 4 + rw * ((f >= 1 ? all : f >= 0.5 ? 0.55 : 0.33) + (in_line ? 0.3 : 0)) / 6.0e6;
     }
     c.together = std::max((first ? 19 : 8) + 1.1 * units,
                           rw / (c128 ? 5.7e6 : 3.7e6) + units * amps * (c128 ? 6.3e-8 : 1.9e-7));
