@@ -402,8 +402,8 @@ inline double sweep_lines(const SweepLone &l, bool c128) {
 // Of the whole state's time, half its lines take 0.55, a quarter 0.33, and a
 // wire inside a line adds 0.3; the phases of a parity take 1.3 times the whole, a
 // DoubleExcitation its lines' share times 1.3, or 0.9 in the last-level cache.
-// In a pass a DoubleExcitation is a frame of some six steps (16 at 18 qubits 172
-// us in passes, 100 one by one; 28 qubits complex64 10.8 and 2.75 ms).
+// In a pass a DoubleExcitation is a frame of some six steps (16 at 18 qubits 190
+// us in passes, 120 one by one; 28 qubits complex64 11.2 and 3.0 ms).
 inline SweepCost sweep_forward_us(const std::vector<SweepOp> &steps, const SweepPass &ps, int n, bool c128,
                                   bool first) {
     const double amps = std::ldexp(1.0, n), rw = 2 * amps * (c128 ? 16 : 8); // bytes

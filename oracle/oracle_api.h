@@ -1,5 +1,5 @@
 /*
- * Checker-side C interface shared by the two CPU oracles:
+ * C interface shared by the two CPU oracles:
  *   - liblq_oracle.so   : this repository's restatement of Lightning-Qubit
  *                         (oracle/lq_oracle.cpp), and
  *   - _ref/libref_lq.so : a thin driver (oracle/ref_driver.cpp) over the
